@@ -34,6 +34,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <climits>
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -461,17 +462,53 @@ constexpr int kLdsMaxNodes = kLdsPerThread * kLdsBlock;
 #define TAPGPU_LDS_QUEUE_MAX 4096
 #endif
 constexpr int kLdsQueueMax = TAPGPU_LDS_QUEUE_MAX;   // frontier queue entries per round
-#ifndef TAPGPU_LDS_GROUP
-#define TAPGPU_LDS_GROUP 6
-#endif
-constexpr int kGroup = TAPGPU_LDS_GROUP;             // lanes per expanded node (one link each)
-constexpr unsigned short kNoPred = 0xFFFF;
+constexpr int kGroup = 4;                            // lanes per expanded node (one link each)
+constexpr int kGroupsPerWave = kWave / kGroup;
+constexpr unsigned kNoPred = 0xFFFF;
+
+// Mirrors of the graph and of each variant's costs that the LDS kernel
+// reads, written wherever a cost is (store_cost).  Neither holds self-loops
+// (they never lower a label and are never a tree link).
+//  * Out-link records, 64 bytes per node: kRecLinks costs, then as many
+//    16-bit heads; only links to through nodes (a zone's label is needed by
+//    no other node, so it is taken from its in-links at the end).  A slot
+//    without a link has the node itself as its head and an infinite cost.
+//    kRecMore marks every head of a node with more than kGroup links,
+//    kRecCsr those of one with more than kRecLinks, whose links are then
+//    read from the CSR.
+//  * In-links in slices of 64 nodes, slot-major (SELL): row s of a slice
+//    holds the s-th in-link of its 64 nodes, a word of link id and tail and
+//    the cost.  Only links between through nodes: those of zones are looked
+//    at by themselves.  An entry without a link has the node itself as its
+//    tail and an infinite cost.
+//    At most kSellWidth rows a slice; a node with more in-links is redone
+//    from the CSR.
+constexpr int kRecDoubles = 8, kRecLinks = 6;
+constexpr unsigned kRecNode = 0x3FFF, kRecMore = 0x4000, kRecCsr = 0x8000;
+static_assert(kRecLinks * 10 <= 64 && kRecLinks <= 2 * kGroup, "an out-link record is 64 bytes");
+static_assert(kLdsMaxNodes <= (int)kRecNode + 1, "heads are 14-bit");
+constexpr int kSellWidth = 16;
+constexpr int kSellFetch = 4;        // rows of a slice loaded ahead
+constexpr unsigned kSellNone = 0xFFFF0000u;
+
+// LDS atomicAdd by one lane.  The address is made to look divergent: for a
+// uniform one the compiler adds a wave-wide reduction around the atomic.
+__device__ __forceinline__ int lds_add(int* p, int n) {
+  int z = 0;
+  asm("" : "+v"(z));
+  return atomicAdd(p + z, n);
+}
 
 struct OriginArgs {
   int N, E, ft0, Z;
   const int *fw_off, *fw_dst, *rv_off, *rv_src, *rv_eid, *tail;
   const double* fww;                 // [V * E] forward costs (INF: absent)
   const double* rvw;                 // [V * E] reverse-order costs
+  const double* rec;                 // [V][N] out-link records (LDS kernel)
+  const double* sellw;               // [V][sell_n] sliced in-link costs
+  const unsigned* sell_id;           // [sell_n] link id << 16 | tail
+  const int* sell_ptr;               // [ceil(N/64) + 1] first entry of each slice
+  long long sell_n;
   const long long* od_start;         // [Z + 1]
   const int* od_dest;                // 0-based zone
   const double* od_val;
@@ -520,12 +557,12 @@ __device__ __forceinline__ int wave_max_i32(int x) {
 }
 __device__ __forceinline__ unsigned long long as_b(double d) { return (unsigned long long)__double_as_longlong(d); }
 
-// LDS layout (bytes): labels 8N (flows while loading) | three bitmaps
-// 3*8W | offs/pred 2A | ptail 2A | two frontier queues 2*2Q, with
-// W = ceil(N/64), A = N+1 rounded up to 4, Q = queue entries.
+// LDS layout (bytes): labels 8N (flows while loading) | two bitmaps 2*8W |
+// pred 2A | ptail 2A | two frontier queues 2*2(Q+2), with W = ceil(N/64),
+// A = N+1 rounded up to 4, Q = queue entries (entry Q takes what overflows).
 size_t origin_lds_bytes(int N, int qcap) {
   const size_t W = (size_t)(N + 63) / 64, A = (size_t)((N + 1 + 3) & ~3);
-  return 8ull * N + 24ull * W + 4ull * A + 4ull * (size_t)qcap;
+  return 8ull * N + 16ull * W + 4ull * A + 4ull * ((size_t)qcap + 2);
 }
 
 // Second step of the predecessor rule: the nodes flagged in `pending` have
@@ -577,19 +614,18 @@ __device__ bool attach_level_ties(const OriginArgs& A, const double* __restrict_
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
   extern __shared__ unsigned long long sm[];
+  constexpr int kWaves = BLOCK / kWave;
   const int N = A.N;
   const int W = (N + 63) >> 6;
   const int Al = (N + 1 + 3) & ~3;
-  unsigned long long* dist = sm;                                   // [N] (flow later)
-  unsigned long long* bmA = dist + N;                              // 3 x [W]
-  unsigned long long* bmB = bmA + W;
+  unsigned long long* key = sm;                                    // [N] label << 1 | listed
+  double* flow = (double*)sm;                                      //     (flows while loading)
+  unsigned long long* bmB = key + N;                               // 2 x [W] (attach_level_ties)
   unsigned long long* bmC = bmB + W;
-  unsigned short* offs = (unsigned short*)(bmC + W);               // [N+1], then pred [N]
-  unsigned short* pred = offs;
-  unsigned short* ptail = offs + Al;                               // [N]
-  unsigned short* queue0 = ptail + Al;                             // 2 x [qcap]
-  unsigned short* queue1 = queue0 + A.qcap;
-  auto qw_of = [&](int rr) { return (rr & 1) ? queue1 : queue0; };   // queue written in round rr
+  unsigned short* pred = (unsigned short*)(bmC + W);               // [N]
+  unsigned short* ptail = pred + Al;                               // [N]
+  unsigned short* queue0 = ptail + Al;                             // 2 x [qcap + 2]
+  unsigned short* queue1 = queue0 + A.qcap + 2;
   __shared__ int s_qn[3];
   __shared__ unsigned long long s_cnt[8];
 
@@ -597,195 +633,329 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
   if (A.var_on && !A.var_on[var]) return;
   const int src = A.src_list ? A.src_list[blockIdx.x] : (int)blockIdx.x;
   const int tid = threadIdx.x;
+  const int wave = uniform(tid / kWave);
+  const int lane = tid & (kWave - 1);
   const double* __restrict__ fw = A.fww + (size_t)var * A.E;
   const double* __restrict__ rw = A.rvw + (size_t)var * A.E;
+  const double* __restrict__ rec = A.rec + (size_t)var * N * kRecDoubles;
+  const double* __restrict__ sellw = A.sellw + (size_t)var * A.sell_n;
   const unsigned long long kMax = as_b(DBL_MAX);
 
-  for (int v = tid; v < N; v += BLOCK) dist[v] = kMax;
-  for (int v = tid; v <= N; v += BLOCK) offs[v] = (unsigned short)A.fw_off[v];
-  for (int w = tid; w < 3 * W; w += BLOCK) bmA[w] = 0;
+  for (int v = tid; v < N; v += BLOCK) key[v] = kMax << 1;
+  for (int w = tid; w < 2 * W; w += BLOCK) bmB[w] = 0;
   if (tid < 3) s_qn[tid] = tid == 0 ? 1 : 0;
   if (tid < 8) s_cnt[tid] = 0;
   __syncthreads();
   if (tid == 0) {
-    dist[src] = 0ull;                     // +0.0
-    bmA[src >> 6] = 1ull << (src & 63);
-    if (A.qcap > 0) queue0[0] = (unsigned short)src;
+    key[src] = 1ull;                      // +0.0, listed
+    queue0[0] = (unsigned short)src;
   }
   __syncthreads();
 
-  unsigned long long n_exp = 0, n_scan = 0, n_upd = 0;
+  unsigned n_exp = 0, n_scan = 0, n_upd = 0;
   const long long clk0 = wall_clock64();
   // ---- label-correcting rounds, one barrier each.  Round r expands the
   //      nodes lowered in round r-1.  Normally they are listed in a queue
-  //      (count s_qn[(r-1)%3], buffer (r-1)&1) and each gets a group of
-  //      kGroup lanes, one out-link per lane: the group's loads are
-  //      consecutive, and a round costs one link's chain of latencies.
-  //      When more nodes were lowered than the queue holds, the round scans
-  //      their bitmap `cur` in 16-bit slots instead, a lane expanding each
-  //      set bit's node (and chaining up to A.chase further expansions of
-  //      nodes it lowers itself).  A node lowered in round r is listed
-  //      once: the lane whose atomicOr sets its bit in `nxt` appends it to
-  //      queue r&1, one LDS atomicAdd per wave for all of the wave's
-  //      appends.  Three rotating bitmaps: the third one is cleared while
-  //      the first is read.  Labels are the same least fixed point for any
-  //      such order. ----
-  unsigned long long *cur = bmA, *nxt = bmB, *clr = bmC;
-  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-  int r = 1;
-  // relaxes u -> v at cost w and, if this lane lowered v and `want`, lists
-  // it unless listed already; returns whether this lane lowered v
-  auto relax = [&](double du, int v, double w, bool want) {
-    const unsigned long long cb = as_b(du + w);
-    // no pre-read of dist[v]: one LDS round trip, and measured faster
-    const bool low = cb < atomicMin(&dist[v], cb);
-    bool first = false;
-    if (low) {
-      ++n_upd;
-      if (want && v >= A.ft0) {
-        const unsigned long long bit = 1ull << (v & 63);
-        first = !(atomicOr(&nxt[v >> 6], bit) & bit);
-      }
-    }
-    const unsigned long long bal = __ballot(first);
-    if (bal) {
-      const int leader = __ffsll((long long)bal) - 1;
+  //      (count s_qn[cnt]) and each gets a group of kGroup lanes of one
+  //      wavefront, one out-link per lane, whose costs and heads are one
+  //      64-byte record.  When more nodes were lowered than the queue holds,
+  //      the round looks for their flags among the labels instead, a lane
+  //      expanding each (and chaining up to A.chase further expansions of
+  //      nodes it lowers itself).
+  //      A label is kept as (bits << 1) | listed: labels are non-negative,
+  //      so the sign bit is free and the keys order like the labels.  An
+  //      expansion reads the label and clears the flag in one atomic, and a
+  //      lane that lowers a label sets it in the same atomic min: the old
+  //      key it gets back tells whether the node waits in a queue already.
+  //      So one LDS atomic lowers and deduplicates, and a node lowered again
+  //      before its expansion is not listed twice.  Labels are the same
+  //      least fixed point for any such order.
+  //      A round is a chain of five latencies (queue entry, record, label
+  //      atomic, append, barrier) and of the instructions between them, and
+  //      4 wavefronts share a SIMD's issue slots, so what bounds it is the
+  //      instructions of the few wavefronts with nodes to expand (~73 nodes
+  //      a round on metro: 5 of 16).  Hence links to zones are left out
+  //      (they would need a 5th and 6th lane for one node in five), empty
+  //      record slots relax like links instead of being masked, control flow
+  //      is wave-uniform, and the lane that lists a node starts a load of
+  //      its record, which has the line in the CU's L1 before the next
+  //      round asks for it.  Taken branches cost as much as an LDS read, so
+  //      the common round is laid out straight.  Measured on metro (1,000
+  //      origins, 146 rounds; us per workgroup): 69, and 143 with 6 lanes
+  //      per node, CSR reads, a bitmap atomic beside the label's and
+  //      divergent loop control. ----
+  const int qcap = A.qcap, ft0 = A.ft0;
+  int c_now = 0, c_next = 1, c_free = 2;   // s_qn slots, in turn: written, cleared, idle
+  const int qstride = qcap + 2;
+  int qoff = 0;                            // the queue written last
+  int pf_node = -1;                        // listed by this lane in the last round
+  unsigned pf_sink = 0;
+  // relaxes a link to the through node v at label bits cb and, if this lane
+  // lowered v and `want`, lists it unless listed already; returns whether
+  // this lane lowered v (without `want` the lane then expands v itself,
+  // which clears the flag set here)
+  auto relax = [&](unsigned long long cb, int v, bool want) {
+    // no pre-read of key[v]: one LDS round trip, and measured faster
+    const unsigned long long kb = (cb << 1) | 1ull;
+    const unsigned long long old = atomicMin(&key[v], kb);
+    const bool low = kb < old;
+    n_upd += low;
+    if (low && want && !(old & 1ull)) {
+      // one LDS atomic for the wavefront's appends
+      const unsigned long long m = __builtin_amdgcn_read_exec();
+      const int rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
       int b0 = 0;
-      if (lane == leader) b0 = atomicAdd(&s_qn[r % 3], __popcll(bal));
-      b0 = __builtin_amdgcn_readlane(b0, leader);
-      if (first) {
-        const int pos = b0 + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
-                                                            __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
-        if (pos < A.qcap) qw_of(r)[pos] = (unsigned short)v;
-      }
+      if (rank == 0) b0 = lds_add(&s_qn[c_now], __popcll(m));
+      queue0[qoff + min(uniform(b0) + rank, qcap)] = (unsigned short)v;
+      pf_node = v;
     }
     return low;
   };
-  for (;; ++r) {
-    const unsigned short* qr = (r & 1) ? queue0 : queue1;
-    const int j0 = tid / kGroup;
-    const int u0 = j0 < A.qcap ? qr[j0] : 0;      // read beside the count
-    const int qn = s_qn[(r - 1) % 3];
-    if (qn <= A.qcap) {
-      for (int idx = tid; idx / kGroup < qn; idx += BLOCK) {
-        const int u = idx == tid ? u0 : qr[idx / kGroup];
-        const int g = idx % kGroup;
-        const double du = as_d(dist[u]);
-        const int eb = offs[u], ee = offs[u + 1];
-        if (g == 0) { ++n_exp; n_scan += (unsigned long long)(ee - eb); }
-        for (int e = eb + g; e < ee; e += kGroup) relax(du, A.fw_dst[e], fw[e], true);
+  // the label of a node about to be expanded; clears its flag
+  auto take = [&](int u) { return as_d(atomicAnd(&key[u], ~1ull) >> 1); };
+  const char* recb = (const char*)rec;
+  const unsigned g = lane % kGroup;
+  // expands a listed node with the kGroup lanes of a group
+  auto expand = [&](int u) {
+    const unsigned at = (unsigned)u * 64u;
+    const double w = *(const double*)(recb + (at + g * 8u));
+    const unsigned h = *(const unsigned short*)(recb + (at + 8u * kRecLinks + g * 2u));
+    const double du = take(u);
+    relax(as_b(du + w), (int)(h & kRecNode), true);
+    n_scan += (int)(h & kRecNode) != u;
+    if (__builtin_expect(h & kRecMore, 0)) {          // more out-links than lanes
+      if (h & kRecCsr) {                              // ... than the record holds
+        const int ee = A.fw_off[u + 1];
+        for (int e = A.fw_off[u] + (int)g; e < ee; e += kGroup) {
+          const int v = A.fw_dst[e];
+          if (v < ft0) continue;
+          ++n_scan;
+          relax(as_b(du + fw[e]), v, true);
+        }
+      } else if (g < kRecLinks - kGroup) {
+        const double w2 = *(const double*)(recb + (at + (g + kGroup) * 8u));
+        const unsigned h2 = *(const unsigned short*)(recb + (at + 8u * kRecLinks + (g + kGroup) * 2u));
+        n_scan += (int)(h2 & kRecNode) != u;
+        relax(as_b(du + w2), (int)(h2 & kRecNode), true);
       }
+    }
+  };
+  constexpr int kPass = kWaves * kGroupsPerWave;       // nodes expanded at once
+  const int j0 = wave * kGroupsPerWave + lane / kGroup;
+  const int jq = min(j0, qcap);
+  const int pass = min(kPass, qcap);
+  int r = 0, qn;
+  unsigned n_listed = 0;                   // (wave-uniform)
+  for (;;) {
+    unsigned pf = 0;
+    if (pf_node >= 0)
+      pf = __hip_atomic_load((const unsigned*)(recb + (unsigned)pf_node * 64u), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WAVEFRONT);
+    pf_node = -1;
+    __syncthreads();
+    int u0 = queue0[qoff + jq], n0 = s_qn[c_now];
+    asm volatile("" : "+v"(u0), "+v"(n0));              // (both read before either is used)
+    qn = uniform(n0);
+    if (qn == 0 || r > N + 8) break;
+    ++r;
+    qoff = qstride - qoff;
+    // (this slot was read before the barrier and is written after the next)
+    s_qn[c_free] = 0;
+    { const int t = c_now; c_now = c_next; c_next = c_free; c_free = t; }
+    if (__builtin_expect(qn <= pass, 1)) {
+      if (j0 < qn) expand(u0);
+      n_listed += (unsigned)qn;
+    } else if (qn <= qcap) {
+      const unsigned short* qr = queue0 + (qstride - qoff);
+      for (int j = j0; j < qn; j += kPass) expand(qr[j]);
+      n_listed += (unsigned)qn;
     } else {
-      for (int slot = tid; slot < 4 * W; slot += BLOCK) {
-        const int w = slot >> 2, q = slot & 3;
-        unsigned bits = (unsigned)((cur[w] >> (16 * q)) & 0xFFFFull);
-        while (bits) {
-          const int b = __ffs(bits) - 1;
-          bits &= bits - 1;
-          int u = (w << 6) + 16 * q + b;
-          for (int hops = 0;; ++hops) {
-            const double du = as_d(dist[u]);
-            const int eb = offs[u], ee = offs[u + 1];
-            ++n_exp;
-            n_scan += (unsigned long long)(ee - eb);
-            int next = -1;
-            for (int e = eb; e < ee; ++e) {
-              const int v = A.fw_dst[e];
-              // the first node this lane lowers is chained, not listed
-              const bool chain = next < 0 && hops < A.chase;
-              if (relax(du, v, fw[e], !chain) && chain && v >= A.ft0) next = v;
-            }
-            if (next < 0) break;
-            u = next;
+      for (int v0 = tid; v0 < N; v0 += BLOCK) {
+        if (!(__hip_atomic_load(&key[v0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & 1ull)) continue;
+        int x = v0;
+        for (int hops = 0;; ++hops) {
+          const double du = take(x);
+          const int eb = A.fw_off[x], ee = A.fw_off[x + 1];
+          ++n_exp;
+          int next = -1;
+          for (int e = eb; e < ee; ++e) {
+            const int v = A.fw_dst[e];
+            if (v < ft0) continue;
+            ++n_scan;
+            // the first node this lane lowers is chained, not listed
+            const bool chain = next < 0 && hops < A.chase;
+            if (relax(as_b(du + fw[e]), v, !chain) && chain) next = v;
           }
+          if (next < 0) break;
+          x = next;
         }
       }
     }
-    for (int w = tid; w < W; w += BLOCK) clr[w] = 0;
-    if (tid == 0) s_qn[(r + 1) % 3] = 0;
-    __syncthreads();
-    if (!s_qn[r % 3]) break;
-    if (r > N + 8) {            // only possible with negative costs
-      if (tid == 0 && atomicCAS(&A.err[0], 0, 2) == 0) { A.err[1] = src; A.err[2] = 0; }
-      return;
-    }
-    unsigned long long* t = cur; cur = nxt; nxt = clr; clr = t;
+    pf_sink ^= pf;
   }
+  if (tid == 0) n_exp += n_listed;
+  if (qn) {                     // only possible with negative costs
+    if (tid == 0 && atomicCAS(&A.err[0], 0, 2) == 0) { A.err[1] = src; A.err[2] = 0; }
+    return;
+  }
+  if (N < 0) s_cnt[7] = pf_sink;            // (never: keeps the loads)
   const int relax_rounds = r;
   const long long clk1 = wall_clock64();
   if (A.work && tid == 0 && blockIdx.y == 0) A.work[src] = relax_rounds;
 
-  // ---- predecessor links (label, then tail id; see above).  The in-link
-  //      offsets are staged in LDS (the out-link offsets are dead); each
-  //      node's tails, costs and link ids are loaded together, so a node
-  //      costs one L2 round trip.  Results stay in registers until every
-  //      thread is done reading offsets (pred shares their space). ----
+  // ---- predecessor links (label, then tail id; see above), every flag
+  //      being clear now.  Through nodes first.  A wavefront takes slices of
+  //      64 consecutive nodes; row s of a slice (the s-th in-links) is
+  //      contiguous in the sliced copy, so every line is read once, and the
+  //      first kSellFetch rows of the next slice are on their way while a
+  //      slice is processed.  Zones other than the origin still have no
+  //      label, so no test keeps them from being tails, and the links of an
+  //      origin that is a zone (which are in no slice) are looked at before
+  //      the slices: its label 0 is the smallest there is, and its id too,
+  //      so such a link wins where it is tight.  Then the zones, whose
+  //      labels are the minimum over their in-links.  Bound by instruction
+  //      issue (about 15 a row; 156 slices of 4 rows on metro): 13.7 us per
+  //      workgroup, 25.6 with a thread reading its node's in-links from the
+  //      CSR. ----
   __shared__ int s_level_ties;
-  for (int v = tid; v <= N; v += BLOCK) offs[v] = (unsigned short)A.rv_off[v];
-  for (int w = tid; w < W; w += BLOCK) bmB[w] = 0;     // nodes left for attach_level_ties
   if (tid == 0) s_level_ties = 0;
+  // this thread's first destination, on its way while the links are chosen
+  long long od0 = 0, od1 = 0;
+  int d0 = 0;
+  double f0 = 0.0;
+  if (load) {
+    od0 = A.od_start[src];
+    od1 = A.od_start[src + 1];
+    if (od0 + tid < od1) { d0 = A.od_dest[od0 + tid]; f0 = A.od_val[od0 + tid]; }
+  }
+  if (src < ft0)
+    for (int e = A.fw_off[src] + tid; e < A.fw_off[src + 1]; e += BLOCK) {
+      const int v = A.fw_dst[e];
+      const unsigned long long wb = as_b(0.0 + fw[e]);
+      if (v < ft0 || wb == 0ull || key[v] >> 1 != wb || wb >= kMax) continue;
+      bool first = true;                     // of equal parallel links
+      for (int k = A.fw_off[src]; k < e; ++k) first = first && !(A.fw_dst[k] == v && fw[k] == fw[e]);
+      if (!first) continue;
+      pred[v] = (unsigned short)e;
+      ptail[v] = (unsigned short)src;
+      atomicOr(&bmC[v >> 6], 1ull << (v & 63));        // chosen
+    }
   __syncthreads();
-  unsigned short my_tail[kLdsPerThread], my_pred[kLdsPerThread];
+  // records v's choice `id` (link and tail; kSellNone's link: none)
+  auto choose = [&](int v, unsigned id, unsigned long long dk) {
+    const bool none = id >= kSellNone, reached = v != src && dk != kMax << 1;
+    pred[v] = (unsigned short)(id >> 16);
+    ptail[v] = (unsigned short)id;
+    // reached, not the origin, and no tight tail with a smaller label:
+    // every tight tail has this label
+    const bool level_tie = none && reached;
+    if (level_tie) {
+      atomicOr(&bmB[v >> 6], 1ull << (v & 63));
+      s_level_ties = 1;
+    }
+    if (A.out_dist) {
+      const size_t o = (size_t)v * A.ld + blockIdx.x;
+      A.out_dist[o] = as_d(dk >> 1);
+      if (!level_tie) A.out_pred[o] = none ? -1 : (int)(id >> 16);
+    }
+  };
   {
-    int j = 0;
-    for (int v = tid; v < N; v += BLOCK, ++j) {
-      unsigned short p = kNoPred, pt = 0;
-      const unsigned long long dv = dist[v];
-      if (v != src && dv != kMax) {
-        // starting from (dv, 0) only tails with a smaller label can win
-        unsigned best = 0;
-        unsigned long long best_du = dv;
-        const int kb = offs[v], ke = offs[v + 1];
-        for (int k0 = kb; k0 < ke; k0 += 8) {
-          int hu[8], he[8];
-          double hw[8];
+    constexpr int kSlices = kLdsPerThread;             // slices per wavefront, at most
+    const int sl0 = ft0 / kWave + wave;                // its first
+    int first = 0, last = 0;                           // lane k: entries of the k-th slice
+    if (lane < kSlices && sl0 + lane * kWaves < W) {
+      first = A.sell_ptr[sl0 + lane * kWaves];
+      last = A.sell_ptr[sl0 + lane * kWaves + 1];
+    }
+    struct Rows { unsigned id[kSellFetch]; double w[kSellFetch]; };
+    auto rows_of = [&](int k) {
+      return (__builtin_amdgcn_readlane(last, k) - __builtin_amdgcn_readlane(first, k)) / kWave;
+    };
+    auto fetch = [&](int k, Rows& R) {
+      const unsigned at = (unsigned)(__builtin_amdgcn_readlane(first, k) + lane);
+      const int rows = rows_of(k);
 #pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if (k0 + i < ke) { hu[i] = A.rv_src[k0 + i]; hw[i] = rw[k0 + i]; he[i] = A.rv_eid[k0 + i]; }
+      for (int i = 0; i < kSellFetch; ++i)
+        if (i < rows) { R.id[i] = A.sell_id[at + i * kWave]; R.w[i] = sellw[at + i * kWave]; }
+    };
+    auto select = [&](int k, const Rows& R) {
+      const int sl = sl0 + k * kWaves, v = sl * kWave + lane, rows = rows_of(k);
+      const unsigned long long dk = v < N ? key[v] : kMax << 1, dv = dk >> 1;
+      // starting from (dv, tail 0) only tails with a smaller label can win
+      unsigned best = kSellNone;
+      unsigned long long best_du = dk;
+      auto offer = [&](unsigned id, double w) {
+        const unsigned u = id & 0xFFFFu;
+        const unsigned long long du = key[u];
+        const bool tight = as_b(as_d(du >> 1) + w) == dv;
+        if (__ballot(tight && du == best_du) && tight && du == best_du && u < (best & 0xFFFFu)) best = id;
+        if (tight && du < best_du) { best = id; best_du = du; }
+      };
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            if (k0 + i >= ke) break;
-            const int u = hu[i];
-            if (u == v || (u < A.ft0 && u != src)) continue;
-            const unsigned long long du = dist[u];
-            if (du == kMax) continue;
-            if (as_b(as_d(du) + hw[i]) != dv) continue;
-            const unsigned key = (unsigned)u;
-            if (du < best_du || (du == best_du && key < best)) {
-              best = key;
-              best_du = du;
-              p = (unsigned short)he[i];
-              pt = (unsigned short)u;
-            }
-          }
-        }
+      for (int i = 0; i < kSellFetch; ++i)
+        if (i < rows) offer(R.id[i], R.w[i]);
+      if (rows > kSellFetch) {
+        const unsigned at = (unsigned)(__builtin_amdgcn_readlane(first, k) + lane);
+        for (int i = kSellFetch; i < rows; ++i) offer(A.sell_id[at + i * kWave], sellw[at + i * kWave]);
+        if (rows == kSellWidth && v < N && v >= ft0)
+          for (int e = A.rv_off[v]; e < A.rv_off[v + 1]; ++e)
+            if (A.rv_src[e] >= ft0 && A.rv_src[e] != v)
+              offer((unsigned)A.rv_src[e] | (unsigned)A.rv_eid[e] << 16, rw[e]);
       }
-      my_tail[j] = pt;
-      my_pred[j] = p;
-      // reached, not the origin, and no tight tail with a smaller label:
-      // every tight tail has this label
-      const bool level_tie = p == kNoPred && v != src && dv != kMax;
-      if (level_tie) {
-        atomicOr(&bmB[v >> 6], 1ull << (v & 63));
-        s_level_ties = 1;
+      const bool chosen = (bmC[min(sl, W - 1)] >> lane) & 1ull;
+      if (v < N && v >= ft0) {
+        if (dk == kMax << 1 || v == src) best = kSellNone | 0xFFFFu;
+        if (!chosen)
+          choose(v, best, dk);
+        else if (A.out_dist)
+          choose(v, (unsigned)pred[v] << 16 | (unsigned)src, dk);
       }
-      if (A.out_dist) {
-        const size_t o = (size_t)v * A.ld + blockIdx.x;
-        A.out_dist[o] = as_d(dv);
-        if (!level_tie) A.out_pred[o] = (p == kNoPred) ? -1 : (int)p;
-      }
+    };
+    const int n = sl0 < W ? (W - sl0 + kWaves - 1) / kWaves : 0;
+    Rows Ra, Rb;
+    if (n > 0) fetch(0, Ra);
+    for (int k = 0; k < n; k += 2) {
+      if (k + 1 < n) fetch(k + 1, Rb);
+      select(k, Ra);
+      if (k + 2 < n) fetch(k + 2, Ra);
+      if (k + 1 < n) select(k + 1, Rb);
     }
   }
-  __syncthreads();        // every offs[] read is done
-  const long long clk2 = wall_clock64();
-  {
-    int j = 0;
-    for (int v = tid; v < N; v += BLOCK, ++j) { pred[v] = my_pred[j]; ptail[v] = my_tail[j]; }
+  if (ft0 > 0) {
+    __syncthreads();                        // the through nodes' selections read no zone label
+    for (int v = tid; v < ft0 && v < N; v += BLOCK) {
+      unsigned id = kSellNone | 0xFFFFu;
+      unsigned long long dk = key[v];
+      if (v != src) {
+        auto tails = [&](auto&& f) {        // f(tail, link, label bits through it)
+          for (int e = A.rv_off[v]; e < A.rv_off[v + 1]; ++e) {
+            const int u = A.rv_src[e];
+            if (u == v || (u < ft0 && u != src)) continue;
+            const unsigned long long du = key[u];
+            if (du != kMax << 1) f(u, A.rv_eid[e], du, as_b(as_d(du >> 1) + rw[e]) << 1);
+          }
+        };
+        tails([&](int, int, unsigned long long, unsigned long long c) { dk = min(dk, c); });
+        unsigned long long best_du = dk;
+        tails([&](int u, int e, unsigned long long du, unsigned long long c) {
+          if (c == dk && (du < best_du || (du == best_du && (unsigned)u < (id & 0xFFFFu) && id < kSellNone))) {
+            best_du = du;
+            id = (unsigned)u | (unsigned)e << 16;
+          }
+        });
+        if (dk == kMax << 1) id = kSellNone | 0xFFFFu;
+        key[v] = dk;
+      }
+      choose(v, id, dk);
+    }
   }
+  __syncthreads();
+  const long long clk2 = wall_clock64();
   if (s_level_ties) {
     __shared__ int s_left, s_added;
     const bool ok = attach_level_ties<BLOCK>(
-        A, rw, src, bmB, bmC, &s_left, &s_added, [&](int v) { return dist[v]; },
+        A, rw, src, bmB, bmC, &s_left, &s_added, [&](int v) { return key[v] >> 1; },
         [&](int v, int e, int u) {
           pred[v] = (unsigned short)e;
           ptail[v] = (unsigned short)u;
@@ -793,12 +963,13 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
         });
     if (!ok && tid == 0 && atomicCAS(&A.err[0], 0, 3) == 0) { A.err[1] = src; A.err[2] = 0; }
   }
+  auto flush_counts = [&]() {
+    const unsigned long long a = wave_sum_u64(n_exp), b = wave_sum_u64(n_scan), c = wave_sum_u64(n_upd);
+    if (lane == 0) { atomicAdd(&s_cnt[0], a); atomicAdd(&s_cnt[1], b); atomicAdd(&s_cnt[2], c); }
+  };
   if (!load) {
     if (A.counters) {
-      n_exp = wave_sum_u64(n_exp); n_scan = wave_sum_u64(n_scan); n_upd = wave_sum_u64(n_upd);
-      if (lane == 0) {
-        atomicAdd(&s_cnt[0], n_exp); atomicAdd(&s_cnt[1], n_scan); atomicAdd(&s_cnt[2], n_upd);
-      }
+      flush_counts();
       __syncthreads();
       if (tid == 0) {
         atomicAdd(&A.counters[0], s_cnt[0]); atomicAdd(&A.counters[1], s_cnt[1]);
@@ -813,32 +984,42 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
   //      (the flow on the node's tree in-link); no rounds, no barriers.
   //      Integer demands make every partial sum exact, so the order of the
   //      LDS atomics does not matter. ----
-  double* flow = (double*)dist;
+  __syncthreads();                 // every label read is done
   for (int v = tid; v < N; v += BLOCK) flow[v] = 0.0;
   __shared__ unsigned long long s_steps;
   __shared__ int s_maxlen, s_loaded;
-  if (tid == 0) { s_steps = 0; s_maxlen = 0; s_loaded = 0; }
+  if (tid == 0) { s_steps = 0; s_maxlen = 0; s_loaded = 0; ptail[src] = (unsigned short)src; }
   __syncthreads();
   unsigned long long steps = 0;
   int maxlen = 0;
-  for (long long i = A.od_start[src] + tid; i < A.od_start[src + 1]; i += BLOCK) {
-    const int d = A.od_dest[i];
-    const double f = A.od_val[i];
+  for (long long i = od0 + tid; i < od1; i += BLOCK) {
+    const int d = i == od0 + tid ? d0 : A.od_dest[i];
+    const double f = i == od0 + tid ? f0 : A.od_val[i];
     if (d == src || !(f > 0.0)) continue;
     if (pred[d] == kNoPred) {
       if (atomicCAS(&A.err[0], 0, 1) == 0) { A.err[1] = src; A.err[2] = d; }
       continue;
     }
+    // The longest walk (one LDS read a step) sets the time, so four steps
+    // go without a branch: a walk that has arrived stays at the origin, its
+    // own tail here, and adds zero to a node of its lane's own (metro: 15 us
+    // per workgroup for the loading, 22.9 with a branch a step).
     int v = d, len = 0;
-    while (v != src) {
+    const int idle = min(lane, N - 1);
+    do {
       if (len > N) {        // a predecessor cycle
         if (atomicCAS(&A.err[0], 0, 3) == 0) { A.err[1] = src; A.err[2] = 0; }
         break;
       }
-      atomicAdd(&flow[v], f);
-      v = ptail[v];
-      ++len;
-    }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int next = ptail[v];
+        const bool on = v != src;
+        atomicAdd(&flow[on ? v : idle], on ? f : 0.0);
+        len += on;
+        v = next;
+      }
+    } while (v != src);
     steps += (unsigned long long)len;
     maxlen = max(maxlen, len);
   }
@@ -853,12 +1034,11 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
     }
   }
   if (A.counters) {
-    n_exp = wave_sum_u64(n_exp); n_scan = wave_sum_u64(n_scan); n_upd = wave_sum_u64(n_upd);
+    flush_counts();
     steps = wave_sum_u64(steps);
     maxlen = wave_max_i32(maxlen);
     const unsigned long long ld = wave_sum_u64((unsigned long long)loaded);
     if (lane == 0) {
-      atomicAdd(&s_cnt[0], n_exp); atomicAdd(&s_cnt[1], n_scan); atomicAdd(&s_cnt[2], n_upd);
       atomicAdd(&s_steps, steps);
       atomicMax(&s_maxlen, maxlen);
       atomicAdd(&s_loaded, (int)ld);
@@ -1268,7 +1448,70 @@ struct Links {
   double *x, *y, *c;                 // [V * E]
   double* rvw;                       // [V * E]  costs, reverse-CSR order, INF: absent
   double* fww;                       // [V * E]  costs, link order, INF: absent
+  // mirrors of the LDS kernel (null: it does not apply to this network)
+  double *rec, *sellw;
+  const int *recpos, *sellpos;       // [E] position of link k in a variant's mirror, -1: none
+  long long rec_n, sell_n;           // their sizes per variant
 };
+
+// The cost of link k of variant var, in every order a search reads it.
+__device__ __forceinline__ void store_cost(const Links& K, int var, int k, double c) {
+  const size_t off = (size_t)var * K.E;
+  const double wv = K.present[off + k] ? c : INFINITY;
+  K.rvw[off + K.rvpos[k]] = wv;
+  K.fww[off + k] = wv;
+  if (K.rec) {
+    const int a = K.recpos[k], b = K.sellpos[k];
+    if (a >= 0) K.rec[(size_t)var * K.rec_n + a] = wv;
+    if (b >= 0) K.sellw[(size_t)var * K.sell_n + b] = wv;
+  }
+}
+
+// The fixed parts of the LDS kernel's mirrors (heads, tails, link ids and
+// every link's positions) and infinite costs where a slot holds no link; a
+// thread per node, and per padding lane of the last slice.
+__global__ __launch_bounds__(kBlock) void k_mirrors(Graph G, Links K, const int* sell_ptr,
+                                                    unsigned* sell_id, int* recpos, int* sellpos) {
+  const int v = blockIdx.x * kBlock + threadIdx.x;
+  const int sl = v / kWave;
+  if (sl >= (G.N + kWave - 1) / kWave) return;
+  const int base = sell_ptr[sl] + v % kWave, end = sell_ptr[sl + 1];
+  int at = base;
+  if (v < G.N) {
+    unsigned short head[8] = {};
+    int n = 0;
+    for (int g = 0; g < kRecLinks; ++g) head[g] = (unsigned short)v;
+    for (int k = G.fw_off[v]; k < G.fw_off[v + 1]; ++k) {
+      const int d = G.fw_dst[k];
+      recpos[k] = -1;
+      if (d < G.ft0 || d == v) continue;
+      if (n < kRecLinks) {
+        head[n] = (unsigned short)d;
+        recpos[k] = v * kRecDoubles + n;
+      }
+      ++n;
+    }
+    const unsigned mark = (n > kGroup ? kRecMore : 0u) | (n > kRecLinks ? kRecCsr : 0u);
+    for (int g = 0; g < kRecLinks; ++g) head[g] |= (unsigned short)mark;
+    for (int var = 0; var < K.V; ++var) {
+      double* r = K.rec + (size_t)var * K.rec_n + (size_t)v * kRecDoubles;
+      for (int g = 0; g < kRecLinks; ++g) r[g] = INFINITY;
+      __builtin_memcpy(r + kRecLinks, head, 16);
+    }
+    for (int k = G.rv_off[v]; k < G.rv_off[v + 1]; ++k) {
+      const int u = G.rv_src[k], e = G.rv_eid[k];
+      sellpos[e] = -1;
+      if (v < G.ft0 || u < G.ft0 || u == v || at >= end) continue;
+      sell_id[at] = (unsigned)u | (unsigned)e << 16;
+      sellpos[e] = at;
+      at += kWave;
+    }
+  }
+  for (; at < end; at += kWave) {
+    sell_id[at] = kSellNone | (unsigned)min(v, G.N - 1);
+    for (int var = 0; var < K.V; ++var) K.sellw[(size_t)var * K.sell_n + at] = INFINITY;
+  }
+}
 
 struct VarState {
   double best_lb, relgap, lambda, objective, total_demand, vht;
@@ -1302,9 +1545,7 @@ __global__ __launch_bounds__(kBlock) void k_costs(Links K, int mode, const unsig
     else if (mode == 1) c = tap_bpr(K.t0[j], K.cap[j], K.B[j], K.pw[j], K.x[j]);
     else c = K.c[j];
     K.c[j] = c;
-    const double wv = K.present[j] ? c : INFINITY;
-    K.rvw[(size_t)var * K.E + K.rvpos[k]] = wv;
-    K.fww[j] = wv;
+    store_cost(K, var, k, c);
   }
 }
 
@@ -1500,9 +1741,7 @@ __global__ __launch_bounds__(kBlock) void k_link_step(Links K, VarState* st) {
     K.x[i] = x;
     const double c = tap_bpr(K.t0[i], K.cap[i], K.B[i], K.pw[i], x);
     K.c[i] = c;
-    const double wv = K.present[i] ? c : INFINITY;
-    K.rvw[off + K.rvpos[k]] = wv;
-    K.fww[i] = wv;
+    store_cost(K, var, k, c);
   }
 }
 
@@ -1563,9 +1802,7 @@ __global__ __launch_bounds__(kBlock) void k_link_small(Links K, VarState* st, un
     K.x[i] = x;
     const double c = tap_bpr(K.t0[i], K.cap[i], K.B[i], K.pw[i], x);
     K.c[i] = c;
-    const double wv = K.present[i] ? c : INFINITY;
-    K.rvw[off + K.rvpos[k]] = wv;
-    K.fww[i] = wv;
+    store_cost(K, var, k, c);
   }
   if (threadIdx.x == 0) {
     s.stepping = 0;
@@ -1658,6 +1895,11 @@ struct tapgpu_ctx {
   double *t0 = nullptr, *cap = nullptr, *B = nullptr, *pw = nullptr;
   unsigned char* present = nullptr;
   double *x = nullptr, *y = nullptr, *c = nullptr, *rvw = nullptr, *fww = nullptr;
+  // the LDS kernel's mirrors of the graph and the costs
+  double *rec = nullptr, *sellw = nullptr;
+  int *recpos = nullptr, *sellpos = nullptr, *sell_ptr = nullptr;
+  unsigned* sell_id = nullptr;
+  long long sell_n = 0;
   // origin-major demand (per-origin workgroups)
   long long* od_start = nullptr;
   int* od_dest = nullptr;
@@ -1839,7 +2081,8 @@ Labels make_labels(tapgpu_ctx* c, const int* col_src, const int* grp_var,
 
 Links make_links(tapgpu_ctx* c) {
   return Links{c->E, c->V, c->t0, c->cap, c->B, c->pw, c->present, c->rvpos,
-               c->x, c->y, c->c, c->rvw, c->fww};
+               c->x, c->y, c->c, c->rvw, c->fww, c->rec, c->sellw, c->recpos, c->sellpos,
+               (long long)c->N * kRecDoubles, c->sell_n};
 }
 
 // Round loop shared by the sweeps and the loading levels: launch
@@ -2020,6 +2263,8 @@ OriginArgs make_origin_args(tapgpu_ctx* c, const unsigned char* var_on) {
   A.N = c->N; A.E = c->E; A.ft0 = c->ft0; A.Z = c->Z;
   A.fw_off = c->fw_off; A.fw_dst = c->fw_dst; A.rv_off = c->rv_off; A.rv_src = c->rv_src;
   A.rv_eid = c->rv_eid; A.tail = c->tail; A.fww = c->fww; A.rvw = c->rvw;
+  A.rec = c->rec; A.sellw = c->sellw; A.sell_id = c->sell_id; A.sell_ptr = c->sell_ptr;
+  A.sell_n = c->sell_n;
   A.od_start = c->od_start; A.od_dest = c->od_dest; A.od_val = c->od_val;
   A.var_on = var_on; A.y = c->y; A.err = c->err_dev; A.counters = c->counters;
   A.chase = c->chase >= 0 ? c->chase : kDefaultChase;
@@ -2030,6 +2275,16 @@ OriginArgs make_origin_args(tapgpu_ctx* c, const unsigned char* var_on) {
   A.z0 = 0;
   A.zn = c->Z;
   return A;
+}
+
+// The cost arrays of A moved to variant v (the kernels' variant 0).
+void advance_variant(tapgpu_ctx* c, OriginArgs& A, int64_t v) {
+  A.fww += (size_t)v * c->E;
+  A.rvw += (size_t)v * c->E;
+  if (c->rec) {
+    A.rec += (size_t)v * c->N * kRecDoubles;
+    A.sellw += (size_t)v * c->sell_n;
+  }
 }
 
 // Workgroup size the LDS kernel runs with (before tuning: kLdsBlock).
@@ -2078,7 +2333,7 @@ int launch_origin(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, fl
     HIPCHK(c, hipMemsetAsync(c->y + (size_t)v0 * c->E, 0, sizeof(double) * (size_t)Vn * c->E, c->stream));
   if (c->Z > 0) {
     OriginArgs A = make_origin_args(c, var_on);
-    A.fww += (size_t)v0 * c->E; A.rvw += (size_t)v0 * c->E; A.y += (size_t)v0 * c->E;
+    advance_variant(c, A, v0); A.y += (size_t)v0 * c->E;
     if (var_on) A.var_on = var_on + v0;
     const int zh = (c->hbm_ok && c->split > 0) ? std::min(c->split, c->Z - 1) : 0;
     const int zl = c->Z - zh;
@@ -2370,7 +2625,7 @@ int launch_hbm(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, int i
     HIPCHK(c, hipMemsetAsync(c->y + (size_t)v0 * c->E, 0, sizeof(double) * (size_t)Vn * c->E, c->stream));
   if (c->Z == 0) return TAPGPU_OK;
   OriginArgs A = make_origin_args(c, var_on);
-  A.fww += (size_t)v0 * c->E; A.rvw += (size_t)v0 * c->E; A.y += (size_t)v0 * c->E;
+  advance_variant(c, A, v0); A.y += (size_t)v0 * c->E;
   if (var_on) A.var_on = var_on + v0;
   const int items = std::min(c->Z * Vn, items_cap);
   const int G = std::min(c->hbm_grid, items);
@@ -2671,13 +2926,14 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
       lds_max = 0;
-    c->lds_bytes = origin_lds_bytes(c->N, 0);
+    // (8W bytes more than the layout: room for a queue on the largest networks)
+    c->lds_bytes = origin_lds_bytes(c->N, 0) + 8ull * ((N + 63) / 64);
     if (hipDeviceGetAttribute(&c->clock_khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess)
       c->clock_khz = 0;
     c->lds_ok = c->lds_bytes + 128 <= (size_t)lds_max && E < 65535 && N <= kLdsMaxNodes;
     if (c->lds_ok) {
       // the rest of the LDS, up to kLdsQueueMax entries, holds the frontier queues
-      const size_t spare = (size_t)lds_max - 128 - c->lds_bytes;
+      const size_t spare = (size_t)lds_max - 128 - origin_lds_bytes(c->N, 0);
       c->qcap_max = (int)std::min<size_t>(kLdsQueueMax, spare / 4) & ~63;
       c->qcap = c->qcap_max;
       c->lds_bytes = origin_lds_bytes(c->N, c->qcap_max);
@@ -2807,6 +3063,26 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
 
   ALLOC(part, (size_t)V * kLinkBlocks * kQ);
   ALLOC(prm, 1);
+  // the LDS kernel's mirrors (k_mirrors fills them in, store_cost their costs)
+  const int W = (int)((N + 63) / 64);
+  std::vector<int> sell_ptr;
+  if (c->lds_ok) {
+    sell_ptr.assign(W + 1, 0);
+    for (int64_t v = c->ft0; v < N; ++v) {
+      int n = 0;
+      for (int k = rv_off[v]; k < rv_off[v + 1]; ++k) n += rv_src[k] != v && rv_src[k] >= c->ft0;
+      int& rows = sell_ptr[v / kWave + 1];
+      rows = std::max(rows, std::min(kSellWidth, n));
+    }
+    for (int i = 0; i < W; ++i) sell_ptr[i + 1] = sell_ptr[i] + sell_ptr[i + 1] * kWave;
+    c->sell_n = sell_ptr[W];
+    ALLOC(rec, (size_t)V * (N * kRecDoubles + c->sell_n));
+    ALLOC(recpos, 2 * (size_t)E + W + 1 + c->sell_n);
+    c->sellw = c->rec + (size_t)V * N * kRecDoubles;
+    c->sellpos = c->recpos + E;
+    c->sell_ptr = c->sellpos + E;
+    c->sell_id = (unsigned*)(c->sell_ptr + W + 1);
+  }
 #undef ALLOC
   if ((rc = upload(c, c->fw_off, fw_off.data(), N + 1))) return rc;
   if ((rc = upload(c, c->fw_dst, fw_dst.data(), E))) return rc;
@@ -2822,6 +3098,12 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
   if ((rc = upload(c, c->present, hpres.data(), VE))) return rc;
   if ((rc = upload(c, c->col_src, col_src.data(), c->P))) return rc;
   if ((rc = upload(c, c->grp_var, grp_var.data(), c->Galloc))) return rc;
+  if (c->lds_ok) {
+    if ((rc = upload(c, c->sell_ptr, sell_ptr.data(), sell_ptr.size()))) return rc;
+    hipLaunchKernelGGL(k_mirrors, dim3((W * kWave + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream,
+                       make_graph(c), make_links(c), c->sell_ptr, c->sell_id, c->recpos, c->sellpos);
+    HIPCHK(c, hipGetLastError());
+  }
   c->h_odc = std::move(odc);
   if ((rc = dalloc(c, &c->od_start, Z + 1))) return rc;
   if ((rc = dalloc(c, &c->od_dest, h_od_dest.size()))) return rc;
@@ -2973,7 +3255,7 @@ int tapgpu_sssp(tapgpu_ctx* c, int64_t variant, const int64_t* start_nodes, int6
         break;
       }
       OriginArgs A = make_origin_args(c, nullptr);
-      A.fww += (size_t)variant * c->E; A.rvw += (size_t)variant * c->E;
+      advance_variant(c, A, variant);
       A.src_list = d_src; A.out_dist = d_dist; A.out_pred = d_pred; A.ld = chunk;
       if (hbm)
         hipLaunchKernelGGL(k_origin_hbm, dim3((unsigned)std::min<int64_t>(ns, c->hbm_grid)),
@@ -3163,8 +3445,7 @@ int tapgpu_sssp_noalloc(tapgpu_ctx* c, int64_t variant, const int64_t* d_start_n
   unsigned char* p = (unsigned char*)base;
   int* d_src = (int*)p;
   OriginArgs A = make_origin_args(c, nullptr);
-  A.fww += (size_t)variant * c->E;
-  A.rvw += (size_t)variant * c->E;
+  advance_variant(c, A, variant);
   A.src_list = d_src;
   A.out_dist = d_dist;
   A.out_pred = d_pred;
