@@ -56,7 +56,6 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kJ = 16;                      // step sizes 2^-j evaluated per link pass
 constexpr int kQ = 3 + kJ;                  // g0, objective, vht, g(2^-j)...
 constexpr int kMaxHalvings = 1001;          // lambda = 2^-1 ... 2^-1001
-constexpr int kLinkBlocks = 120;            // partial-sum blocks per variant
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
 
@@ -1530,6 +1529,19 @@ struct FwParams {
   int jwin;                 // step sizes a line-search window decides on (<= kJ)
 };
 
+// The LDS kernel's mirrors of the current costs (after passes that did not
+// keep them).
+__global__ __launch_bounds__(kBlock) void k_mirror_costs(Links K) {
+  const long long n = (long long)K.E * K.V;
+  for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n;
+       i += (long long)gridDim.x * kBlock) {
+    const int var = (int)(i / K.E), k = (int)(i - (long long)var * K.E);
+    const int a = K.recpos[k], b = K.sellpos[k];
+    if (a >= 0) K.rec[(size_t)var * K.rec_n + a] = K.fww[i];
+    if (b >= 0) K.sellw[(size_t)var * K.sell_n + b] = K.fww[i];
+  }
+}
+
 // mode 0: c = t0 (free-flow, initial Wa); mode 1: c = BPR(x); mode 2: c given
 __global__ __launch_bounds__(kBlock) void k_costs(Links K, int mode, const unsigned char* var_on,
                                                   int v0, int Vn) {
@@ -1549,40 +1561,62 @@ __global__ __launch_bounds__(kBlock) void k_costs(Links K, int mode, const unsig
   }
 }
 
-// All kQ compensated sums of a block at once, in a fixed order: a butterfly
-// inside each wavefront (lane 0's result is kept), then thread 0 merges the
-// wavefronts in order.  One barrier; the result is in thread 0's v[].
-__device__ void block_reduce_acc(tap_acc* v, tap_acc* sh /* [kBlock / kWave][kQ] */) {
-  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+// All kQ compensated sums of a block at once, in a fixed order.  Inside a
+// wavefront by recursive halving: at each step a lane hands half of the sums
+// it still carries to its partner and merges the partner's share of the
+// other half (10 + 5 + 3 + 2 + 1 + 1 merges, where a butterfly of all 19
+// sums takes 114), then one thread per sum merges the wavefronts.  The
+// result is in out[] for every thread after the call's last barrier; sh
+// holds a row per wavefront.
+template <int kOff, int kHave>
+__device__ __forceinline__ void halve_acc(tap_acc* v, int lane) {
+  constexpr int kKeep = (kHave + 1) / 2;
+  const bool up = lane & kOff;
 #pragma unroll
-  for (int q = 0; q < kQ; ++q) {
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-      tap_acc o;
-      o.s = __shfl_xor(v[q].s, off);
-      o.c = __shfl_xor(v[q].c, off);
-      tap_acc_merge(&v[q], o);
-    }
-  }
-  if (lane == 0) {
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) sh[w * kQ + q] = v[q];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) {
-      tap_acc a = sh[q];
-      for (int j = 1; j < kBlock / kWave; ++j) tap_acc_merge(&a, sh[j * kQ + q]);
-      v[q] = a;
-    }
+  for (int i = 0; i < kKeep; ++i) {
+    const tap_acc lo = v[i];
+    tap_acc hi{0.0, 0.0};
+    if (kKeep + i < kHave) hi = v[kKeep + i];
+    const tap_acc give = up ? lo : hi;
+    tap_acc keep = up ? hi : lo, got;
+    got.s = __shfl_xor(give.s, kOff);
+    got.c = __shfl_xor(give.c, kOff);
+    tap_acc_merge(&keep, got);
+    v[i] = keep;
   }
 }
 
-// Partial sums per (variant, block): g0 = sum c*d, objective, vht and
-// g(2^-j) for j in [jbase, jbase + kJ) (j = 0 is lambda = 1).  A block is
-// one wavefront (kLinkThreads): each lane sums several links, then one
-// shuffle reduction per accumulator, with no LDS stage.
-constexpr int kLinkThreads = kWave;
+template <int kWaves>
+__device__ void block_reduce_acc(tap_acc* v, tap_acc* sh /* [kWaves][kQ] */, tap_acc* out /* [kQ] */) {
+  static_assert(kQ == 19, "the halving below is written for 19 sums");
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  halve_acc<32, 19>(v, lane);      // 10 and 9
+  halve_acc<16, 10>(v, lane);      // 5 and 5
+  halve_acc<8, 5>(v, lane);        // 3 and 2
+  halve_acc<4, 3>(v, lane);        // 2 and 1
+  halve_acc<2, 2>(v, lane);        // 1 and 1
+  {
+    tap_acc got;
+    got.s = __shfl_xor(v[0].s, 1);
+    got.c = __shfl_xor(v[0].c, 1);
+    // (the lower lane's share first in both lanes)
+    tap_acc a = (lane & 1) ? got : v[0];
+    tap_acc_merge(&a, (lane & 1) ? v[0] : got);
+    v[0] = a;
+  }
+  const int b5 = lane >> 5 & 1, b4 = lane >> 4 & 1, b3 = lane >> 3 & 1, b2 = lane >> 2 & 1, b1 = lane >> 1 & 1;
+  const int in5 = 3 * b3 + 2 * b2 + b1;                       // of the 5 sums of this 8-lane group
+  const int q = 10 * b5 + 5 * b4 + in5;
+  const bool holds = (b3 ? !b2 : !(b2 && b1)) && q < kQ && !(lane & 1);
+  if (holds) sh[w * kQ + q] = v[0];
+  __syncthreads();
+  if (threadIdx.x < kQ) {
+    tap_acc a = sh[threadIdx.x];
+    for (int j = 1; j < kWaves; ++j) tap_acc_merge(&a, sh[j * kQ + threadIdx.x]);
+    out[threadIdx.x] = a;
+  }
+  __syncthreads();
+}
 
 // acc[3 + j] += BPR(x + 2^-(jbase+j) d) * d for the kJ step sizes of a
 // window (lam0 = 2^-jbase).  Halving is exact for every step size used
@@ -1599,50 +1633,24 @@ __device__ __forceinline__ void step_sums(tap_acc* acc, double lam0, double x, d
   }
 }
 
-__global__ __launch_bounds__(kLinkThreads) void k_link_partials(Links K, const VarState* st,
-                                                                tap_acc* part, int only_g) {
-  const int var = blockIdx.y;
-  const VarState s = st[var];
-  if (!s.stepping || (only_g && !s.need_more)) return;
-  const int jbase = only_g ? s.jnext : 0;
-  tap_acc acc[kQ];
-#pragma unroll
-  for (int q = 0; q < kQ; ++q) acc[q] = tap_acc{0.0, 0.0};
-  const double lam0 = ldexp(1.0, -jbase);
-  const size_t off = (size_t)var * K.E;
-  for (int k = blockIdx.x * kLinkThreads + threadIdx.x; k < K.E; k += gridDim.x * kLinkThreads) {
-    const size_t i = off + k;
-    if (!K.present[i]) continue;
-    const double x = K.x[i];
-    const double d = K.y[i] - x;
-    const double t0 = K.t0[i], cap = K.cap[i], B = K.B[i], pw = K.pw[i];
-    if (!only_g) {
-      const double c = K.c[i];
-      tap_acc_add(&acc[0], c * d);
-      tap_acc_add(&acc[1], tap_integral(t0, cap, B, pw, x));
-      tap_acc_add(&acc[2], x * c);
-    }
-    step_sums(acc, lam0, x, d, t0, cap, B, pw);
+// acc += a link's terms of a window; the first window also sums g(0) = c d,
+// the objective and VHT.
+__device__ __forceinline__ void link_sums(tap_acc* acc, const Links& K, size_t i, double lam0, bool first) {
+  const double x = K.x[i];
+  const double d = K.y[i] - x;
+  const double t0 = K.t0[i], cap = K.cap[i], B = K.B[i], pw = K.pw[i];
+  if (first) {
+    const double c = K.c[i];
+    tap_acc_add(&acc[0], c * d);
+    tap_acc_add(&acc[1], tap_integral(t0, cap, B, pw, x));
+    tap_acc_add(&acc[2], x * c);
   }
-#pragma unroll
-  for (int q = 0; q < kQ; ++q) {
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-      tap_acc t;
-      t.s = __shfl_xor(acc[q].s, o);
-      t.c = __shfl_xor(acc[q].c, o);
-      tap_acc_merge(&acc[q], t);
-    }
-  }
-  if (threadIdx.x == 0) {
-    tap_acc* out = part + ((size_t)var * gridDim.x + blockIdx.x) * kQ;
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) out[q] = acc[q];
-  }
+  step_sums(acc, lam0, x, d, t0, cap, B, pw);
 }
 
-// Per variant: combine partials, pick lambda (first 2^-j with g <= 0, the
-// reference's rule), then gap, objective, lower bound, relative gap, average
-// excess cost, trace record, stop test.
+// Per variant: lambda (first 2^-j with g <= 0, the reference's rule), then
+// gap, objective, lower bound, relative gap, average excess cost, trace
+// record, stop test.
 // The decision of one window for one variant from its merged sums acc[kQ]
 // (thread 0 of the caller): on the first window the iteration's scalars
 // and trace record, then lambda = the first 2^-j with g <= 0, or a request
@@ -1707,165 +1715,173 @@ __device__ __forceinline__ void decide_window(VarState& s, const tap_acc* acc, i
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_link_decide(VarState* st, const tap_acc* part,
-                                                        int nparts, int only_g,
-                                                        const FwParams* prm) {
-  const int var = blockIdx.x;
-  VarState s = st[var];
-  if (!s.stepping || (only_g && !s.need_more)) return;
-  tap_acc acc[kQ];
-#pragma unroll
-  for (int q = 0; q < kQ; ++q) acc[q] = tap_acc{0.0, 0.0};
-  for (int b = threadIdx.x; b < nparts; b += kBlock) {
-    const tap_acc* in = part + ((size_t)var * nparts + b) * kQ;
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) tap_acc_merge(&acc[q], in[q]);
-  }
-  __shared__ tap_acc sh[kBlock / kWave * kQ];
-  block_reduce_acc(acc, sh);
-  if (threadIdx.x != 0) return;
-  decide_window(s, acc, only_g, prm, var);
-  st[var] = s;
+// x += lambda * (y - x), c = BPR(x) and its mirrors; clears y for the next
+// loading.
+__device__ __forceinline__ void step_link(const Links& K, int var, int k, double lambda) {
+  const size_t i = (size_t)var * K.E + k;
+  const double x = K.x[i] + lambda * (K.y[i] - K.x[i]);
+  K.x[i] = x;
+  K.y[i] = 0.0;
+  const double c = tap_bpr(K.t0[i], K.cap[i], K.B[i], K.pw[i], x);
+  K.c[i] = c;
+  store_cost(K, var, k, c);
 }
 
-// x += lambda * (y - x); c = BPR(x); reverse-order costs for the next sweep.
-__global__ __launch_bounds__(kBlock) void k_link_step(Links K, VarState* st) {
-  const int var = blockIdx.y;
-  if (!st[var].stepping || st[var].need_more) return;     // no step until lambda is known
-  const double lambda = st[var].lambda;
-  const size_t off = (size_t)var * K.E;
-  for (int k = blockIdx.x * kBlock + threadIdx.x; k < K.E; k += gridDim.x * kBlock) {
-    const size_t i = off + k;
-    const double d = K.y[i] - K.x[i];
-    const double x = K.x[i] + lambda * d;
-    K.x[i] = x;
-    const double c = tap_bpr(K.t0[i], K.cap[i], K.B[i], K.pw[i], x);
-    K.c[i] = c;
-    store_cost(K, var, k, c);
+// Hands this block's sums[kQ] over and, in the last of the gridDim.x blocks
+// to do so, leaves the merged sums (in a fixed order) in sums[] and returns
+// true.  part: [gridDim.x][kQ]; done: a counter, 0 before and after; sh:
+// [kMergeGroups][kQ].  The sums go through the XCDs' caches as device-scope
+// stores and loads, and the stores have arrived before the count: no fence,
+// which would write back a whole L2 for every block (512 variants of metro:
+// 13 ms a step).
+constexpr int kMergeGroups = kBlock / kQ;
+__device__ bool merge_blocks(tap_acc* sums, tap_acc* sh, tap_acc* part, unsigned* done) {
+  __shared__ int s_last;
+  const int tid = threadIdx.x, nb = gridDim.x;
+  if (tid < kQ) {
+    tap_acc* mine = part + (size_t)blockIdx.x * kQ + tid;
+    __hip_atomic_store(&mine->s, sums[tid].s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&mine->c, sums[tid].c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  __syncthreads();
+  if (tid == 0)
+    s_last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)nb - 1;
+  __syncthreads();
+  if (!s_last) return false;
+  if (tid < kMergeGroups * kQ) {
+    const int q = tid % kQ, g = tid / kQ;
+    tap_acc a{0.0, 0.0};
+    for (int b = g; b < nb; b += kMergeGroups) {
+      tap_acc t;
+      t.s = __hip_atomic_load(&part[(size_t)b * kQ + q].s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      t.c = __hip_atomic_load(&part[(size_t)b * kQ + q].c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      tap_acc_merge(&a, t);
+    }
+    sh[g * kQ + q] = a;
+  }
+  if (tid == 0) *done = 0;
+  __syncthreads();
+  if (tid < kQ) {
+    tap_acc a = sh[tid];
+    for (int g = 1; g < kMergeGroups; ++g) tap_acc_merge(&a, sh[g * kQ + tid]);
+    sums[tid] = a;
+  }
+  __syncthreads();
+  return true;
 }
 
-// All link passes of an iteration for a small network, one workgroup per
-// variant and one launch: the window sums (block reduction), the decision,
-// further windows while the step is undecided, the step (x, costs, both
-// cost mirrors) and the flags.  A workgroup owns its variant's links, so
-// nothing waits on other workgroups.  Used where links <= kSmallLinks;
-// the sums are the same compensated sums as the multi-block passes.
-constexpr int kSmallLinks = 4096;
+// The line search of an iteration in one launch: `blocks` blocks a variant
+// sum the first window, and the last one to finish merges their sums and
+// decides; a step below the first window (2^-15: rare) makes it sum further
+// windows over all links by itself.  A variant that is off, and every
+// variant after a loading that reported an error (a level tie in the lanes
+// kernel, redone by the host), takes no step: its state stays as it was.
+// With one block a variant (small networks) the block also takes the step,
+// so an iteration's link work is one launch; else k_link_step follows.
+//
+// A link costs 16 cost evaluations (~1,000 instructions) and a block's
+// reduction ~450, so a thread takes one link while that leaves the chip
+// unfilled, and up to kLinkPer where a batch or a large network fills it
+// anyway.  Measured: metro (43,600 links) search and step 22 us an
+// iteration, and ~58 as eight launches (two windows of 120 single-wavefront
+// blocks with a butterfly reduction, two decisions, step, flags, clears);
+// 512 variants of metro 1.0 ms with 8 links a thread, 2.0 ms with one;
+// town (3,840 links) 15 us, and ~40 for one block doing all of it (rocprof).
+constexpr int kLinkPer = 8;
+constexpr long long kLinkFill = 1 << 20;   // links a launch has per link of a thread
+constexpr int kSmallLinks = 512;     // links up to which one block a variant is faster
 
-__global__ __launch_bounds__(kBlock) void k_link_small(Links K, VarState* st, unsigned char* var_on,
-                                                       const FwParams* prm) {
-  const int var = blockIdx.x;
-  VarState s = st[var];
-  if (!s.stepping) return;
-  __shared__ tap_acc sh[kBlock / kWave * kQ];
+int link_blocks(long long E, long long V, bool alone) {
+  const long long per = std::min<long long>(kLinkPer, 1 + E * V / kLinkFill + E / 65536);
+  return alone ? 1 : (int)std::max<long long>(1, (E + kBlock * per - 1) / (kBlock * per));
+}
+
+__global__ __launch_bounds__(kBlock) void k_link_search(Links K, VarState* st, unsigned char* var_on,
+                                                        tap_acc* part, unsigned* done, const int* err,
+                                                        const FwParams* prm, int alone) {
+  constexpr int kWaves = kBlock / kWave;
+  const int var = blockIdx.y, tid = threadIdx.x;
+  if (!var_on[var] || err[0] != 0) {
+    if (blockIdx.x == 0 && tid == 0) st[var].stepping = 0;
+    return;
+  }
+  __shared__ tap_acc sh[kMergeGroups * kQ], sums[kQ];
   __shared__ int s_more, s_jnext;
   __shared__ double s_lambda;
   const size_t off = (size_t)var * K.E;
-  int jbase = 0;                     // first window, then the ones thread 0's decisions ask for
-  for (int only_g = 0;; only_g = 1) {
+  const int nb = gridDim.x;
+  auto window = [&](int jbase, bool first, int k0, int stride) {
     tap_acc acc[kQ];
 #pragma unroll
     for (int q = 0; q < kQ; ++q) acc[q] = tap_acc{0.0, 0.0};
     const double lam0 = ldexp(1.0, -jbase);
-    for (int k = threadIdx.x; k < K.E; k += kBlock) {
-      const size_t i = off + k;
-      if (!K.present[i]) continue;
-      const double x = K.x[i];
-      const double d = K.y[i] - x;
-      const double t0 = K.t0[i], cap = K.cap[i], B = K.B[i], pw = K.pw[i];
-      if (!only_g) {
-        const double c = K.c[i];
-        tap_acc_add(&acc[0], c * d);
-        tap_acc_add(&acc[1], tap_integral(t0, cap, B, pw, x));
-        tap_acc_add(&acc[2], x * c);
-      }
-      step_sums(acc, lam0, x, d, t0, cap, B, pw);
-    }
-    block_reduce_acc(acc, sh);
-    if (threadIdx.x == 0) {
-      decide_window(s, acc, only_g, prm, var);
+    for (int k = k0; k < K.E; k += stride)
+      if (K.present[off + k]) link_sums(acc, K, off + k, lam0, first);
+    block_reduce_acc<kWaves>(acc, sh, sums);
+  };
+  window(0, true, blockIdx.x * kBlock + tid, nb * kBlock);
+  if (nb > 1 && !merge_blocks(sums, sh, part + (size_t)var * nb * kQ, &done[var])) return;
+  VarState s;                                                // (thread 0's)
+  if (tid == 0) s = st[var];
+  for (int only_g = 0;; only_g = 1) {
+    if (tid == 0) {
+      decide_window(s, sums, only_g, prm, var);
       s_more = s.need_more;
       s_jnext = s.jnext;
       s_lambda = s.lambda;
     }
     __syncthreads();
     if (!s_more) break;
-    jbase = s_jnext;
-    __syncthreads();                   // (s_more and s_jnext are rewritten next window)
+    window(s_jnext, false, tid, kBlock);
   }
-  const double lambda = s_lambda;
-  for (int k = threadIdx.x; k < K.E; k += kBlock) {
-    const size_t i = off + k;
-    const double d = K.y[i] - K.x[i];
-    const double x = K.x[i] + lambda * d;
-    K.x[i] = x;
-    const double c = tap_bpr(K.t0[i], K.cap[i], K.B[i], K.pw[i], x);
-    K.c[i] = c;
-    store_cost(K, var, k, c);
-  }
-  if (threadIdx.x == 0) {
-    s.stepping = 0;
+  if (alone)
+    for (int k = tid; k < K.E; k += kBlock) step_link(K, var, k, s_lambda);
+  if (tid == 0) {
+    s.stepping = !alone;
     st[var] = s;
     var_on[var] = (unsigned char)s.active;
   }
 }
 
+__global__ __launch_bounds__(kBlock) void k_link_step(Links K, const VarState* st) {
+  const int var = blockIdx.y;
+  if (!st[var].stepping) return;
+  const double lambda = st[var].lambda;
+  for (int k = blockIdx.x * kBlock + threadIdx.x; k < K.E; k += gridDim.x * kBlock) step_link(K, var, k, lambda);
+}
+
 // Per variant at the current volumes: out[2v] = VHT = sum x * c, out[2v+1]
 // = the Beckmann objective (sum of the link cost integrals), compensated
 // sums in a fixed order.
-__global__ __launch_bounds__(kBlock) void k_totals(Links K, double* out) {
-  const int var = blockIdx.x;
+__global__ __launch_bounds__(kBlock) void k_totals(Links K, tap_acc* part, unsigned* done, double* out) {
+  const int var = blockIdx.y, nb = gridDim.x;
   tap_acc acc[kQ];
+#pragma unroll
   for (int q = 0; q < kQ; ++q) acc[q] = tap_acc{0.0, 0.0};
   const size_t off = (size_t)var * K.E;
-  for (int k = threadIdx.x; k < K.E; k += kBlock) {
+  for (int k = blockIdx.x * kBlock + threadIdx.x; k < K.E; k += nb * kBlock) {
     const size_t i = off + k;
     if (!K.present[i]) continue;
     tap_acc_add(&acc[0], K.x[i] * K.c[i]);
     tap_acc_add(&acc[1], tap_integral(K.t0[i], K.cap[i], K.B[i], K.pw[i], K.x[i]));
   }
-  __shared__ tap_acc sh[kBlock / kWave * kQ];
-  block_reduce_acc(acc, sh);
-  if (threadIdx.x == 0) {
-    out[2 * var] = tap_acc_value(acc[0]);
-    out[2 * var + 1] = tap_acc_value(acc[1]);
-  }
+  __shared__ tap_acc sh[kMergeGroups * kQ], sums[kQ];
+  block_reduce_acc<kBlock / kWave>(acc, sh, sums);
+  if (nb > 1 && !merge_blocks(sums, sh, part + (size_t)var * nb * kQ, &done[var])) return;
+  if (threadIdx.x < 2) out[2 * var + threadIdx.x] = tap_acc_value(sums[threadIdx.x]);
 }
 
-__global__ void k_finish_step(VarState* st, int V, unsigned char* var_on) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= V) return;
-  if (st[v].stepping && st[v].need_more) return;          // still searching lambda
-  st[v].stepping = 0;
-  var_on[v] = (unsigned char)st[v].active;
-}
-
-// Opens an FW iteration in one launch: the step flags, and the loading's
-// volumes cleared; the error flag and counters too unless `keep` (later
-// iterations of a multi-iteration graph, which report the first error and
-// the sum of the counters).
-__global__ __launch_bounds__(kBlock) void k_iter_begin(VarState* st, int V, const unsigned char* var_on,
-                                                       int* err, unsigned long long* counters,
-                                                       double* y, long long ny, int keep) {
+// Opens an FW iteration (or a replay of several) in one launch: the error
+// flag and the counters, and the loading's volumes (the step clears them
+// for the iteration after it).
+__global__ __launch_bounds__(kBlock) void k_iter_begin(int* err, unsigned long long* counters, double* y,
+                                                       long long ny) {
   const long long i0 = (long long)blockIdx.x * kBlock + threadIdx.x;
   const long long stride = (long long)gridDim.x * kBlock;
-  for (long long v = i0; v < V; v += stride) {
-    st[v].stepping = var_on[v] ? 1 : 0;
-    st[v].need_more = 0;
-  }
-  if (!keep) {
-    if (i0 < 4) err[i0] = 0;
-    if (i0 < 16) counters[i0] = 0ull;
-  }
+  if (i0 < 4) err[i0] = 0;
+  if (i0 < 16) counters[i0] = 0ull;
   for (long long i = i0; i < ny; i += stride) y[i] = 0.0;
-}
-
-__global__ void k_begin_step(VarState* st, int V, const unsigned char* var_on) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= V) return;
-  st[v].stepping = var_on[v] ? 1 : 0;
-  st[v].need_more = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1900,6 +1916,7 @@ struct tapgpu_ctx {
   int *recpos = nullptr, *sellpos = nullptr, *sell_ptr = nullptr;
   unsigned* sell_id = nullptr;
   long long sell_n = 0;
+  bool mirrors_stale = false;         // not kept since the last lanes loading
   // origin-major demand (per-origin workgroups)
   long long* od_start = nullptr;
   int* od_dest = nullptr;
@@ -1955,7 +1972,8 @@ struct tapgpu_ctx {
   // FW state
   unsigned char* var_on = nullptr;
   VarState* st = nullptr;
-  tap_acc* part = nullptr;
+  tap_acc* part = nullptr;            // [V][link_blocks][kQ] sums of the line search's blocks
+  unsigned* done = nullptr;           // [V] its blocks that have finished
   double* vht = nullptr;              // [2V] VHT, objective at the current volumes
   FwParams* prm = nullptr;            // the fw_run call's limits and trace
   // captured iteration graphs (replayed while profiling is off):
@@ -2079,7 +2097,16 @@ Labels make_labels(tapgpu_ctx* c, const int* col_src, const int* grp_var,
   return Labels{c->dist, c->pred, c->pend, c->P, c->Galloc, col_src, grp_var, var_on, c->rvw};
 }
 
-Links make_links(tapgpu_ctx* c) {
+// Without `mirrors` the passes do not keep the LDS kernel's copies of the
+// costs (batches on the lanes kernel, where they would double the writes of
+// a step); launch_lds brings them up to date when it needs them.
+Links make_links(tapgpu_ctx* c, bool mirrors = true) {
+  if (!mirrors) {
+    c->mirrors_stale = c->mirrors_stale || c->rec;
+    Links K = make_links(c);
+    K.rec = nullptr;
+    return K;
+  }
   return Links{c->E, c->V, c->t0, c->cap, c->B, c->pw, c->present, c->rvpos,
                c->x, c->y, c->c, c->rvw, c->fww, c->rec, c->sellw, c->recpos, c->sellpos,
                (long long)c->N * kRecDoubles, c->sell_n};
@@ -2287,6 +2314,14 @@ void advance_variant(tapgpu_ctx* c, OriginArgs& A, int64_t v) {
   }
 }
 
+// (before any capture too: a replay takes the mirrors as the passes keep them)
+void refresh_mirrors(tapgpu_ctx* c) {
+  if (!c->mirrors_stale || c->capturing) return;
+  hipLaunchKernelGGL(k_mirror_costs, dim3(grid_for((long long)c->E * c->V / kWave + 1)), dim3(kBlock), 0,
+                     c->stream, make_links(c));
+  c->mirrors_stale = false;
+}
+
 // Workgroup size the LDS kernel runs with (before tuning: kLdsBlock).
 int lds_threads(const tapgpu_ctx* c) { return c->lds_block > 0 ? c->lds_block : kLdsBlock; }
 
@@ -2294,6 +2329,7 @@ int lds_threads(const tapgpu_ctx* c) { return c->lds_block > 0 ? c->lds_block : 
 // LDS its queue size needs (a smaller queue leaves room for more
 // workgroups per CU).
 void launch_lds(tapgpu_ctx* c, dim3 grid, hipStream_t st, const OriginArgs& A, int load) {
+  refresh_mirrors(c);
   const size_t sh = origin_lds_bytes(c->N, A.qcap);
   switch (lds_threads(c)) {
     case 256: hipLaunchKernelGGL(k_origin_lds<256>, grid, dim3(256), sh, st, A, load); break;
@@ -2752,7 +2788,7 @@ int load_variants(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on,
 
 int launch_costs(tapgpu_ctx* c, int mode, const unsigned char* var_on, int v0, int Vn) {
   hipLaunchKernelGGL(k_costs, dim3(grid_for((long long)c->E * Vn / kWave + 1)), dim3(kBlock), 0,
-                     c->stream, make_links(c), mode, var_on, v0, Vn);
+                     c->stream, make_links(c, !use_lanes(c, v0, Vn, nullptr)), mode, var_on, v0, Vn);
   HIPCHK(c, hipGetLastError());
   return TAPGPU_OK;
 }
@@ -3061,7 +3097,8 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
   }
 
 
-  ALLOC(part, (size_t)V * kLinkBlocks * kQ);
+  ALLOC(part, (size_t)V * link_blocks(c->E, V, false) * kQ);
+  ALLOC(done, V);
   ALLOC(prm, 1);
   // the LDS kernel's mirrors (k_mirrors fills them in, store_cost their costs)
   const int W = (int)((N + 63) / 64);
@@ -3129,6 +3166,7 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
   HIPCHK(c, hipMemsetAsync(c->x, 0, sizeof(double) * VE, c->stream));
   HIPCHK(c, hipMemsetAsync(c->y, 0, sizeof(double) * VE, c->stream));
   HIPCHK(c, hipMemsetAsync(c->var_on, 1, V, c->stream));
+  HIPCHK(c, hipMemsetAsync(c->done, 0, sizeof(unsigned) * V, c->stream));
   // Wa = free-flow time (trunk/tap/tap_functions.c:331)
   if ((rc = launch_costs(c, 0, nullptr, 0, c->V))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -3566,35 +3604,26 @@ static int upload_params(tapgpu_ctx* c, int max_iters, double target) {
   return TAPGPU_OK;
 }
 
-// The link passes of an iteration: two line-search windows (the second does
-// nothing for variants the first decided), the step, the flags, and the
-// copy of the iteration block (error flag, counters, states, flags) to
-// pinned host memory.
-static int issue_link_passes(tapgpu_ctx* c, const Links& K, dim3 lgrid, bool readback = true) {
-  const bool small = c->link_mode == 1 || (c->link_mode == 0 && c->E <= kSmallLinks);
-  if (small) {                        // one launch, one workgroup per variant
-    hipLaunchKernelGGL(k_link_small, dim3(c->V), dim3(kBlock), 0, c->stream, K, c->st, c->var_on,
-                       c->prm);
-    HIPCHK(c, hipGetLastError());
-    if (readback)
-      HIPCHK(c, hipMemcpyAsync(c->pin_block, c->iter_dev, c->iter_bytes, hipMemcpyDeviceToHost,
-                               c->stream));
-    return TAPGPU_OK;
-  }
-  hipLaunchKernelGGL(k_link_partials, lgrid, dim3(kLinkThreads), 0, c->stream, K, c->st, c->part, 0);
-  hipLaunchKernelGGL(k_link_decide, dim3(c->V), dim3(kBlock), 0, c->stream, c->st, c->part,
-                     kLinkBlocks, 0, c->prm);
-  hipLaunchKernelGGL(k_link_partials, lgrid, dim3(kLinkThreads), 0, c->stream, K, c->st, c->part, 1);
-  hipLaunchKernelGGL(k_link_decide, dim3(c->V), dim3(kBlock), 0, c->stream, c->st, c->part,
-                     kLinkBlocks, 1, c->prm);
-  hipLaunchKernelGGL(k_link_step, lgrid, dim3(kBlock), 0, c->stream, K, c->st);
-  hipLaunchKernelGGL(k_finish_step, dim3((c->V + 255) / 256), dim3(256), 0, c->stream, c->st,
-                     c->V, c->var_on);
+// The link passes of an iteration: the line search (with the flags) and the
+// step, and the copy of the iteration block (error flag, counters, states,
+// flags) to pinned host memory.
+static int issue_link_passes(tapgpu_ctx* c, const Links& K, bool readback = true) {
+  const bool alone = c->link_mode == 1 || (c->link_mode == 0 && c->E <= kSmallLinks);
+  const int nb = link_blocks(c->E, c->V, alone);
+  hipLaunchKernelGGL(k_link_search, dim3(nb, c->V), dim3(kBlock), 0, c->stream, K, c->st, c->var_on,
+                     c->part, c->done, c->err_dev, c->prm, alone ? 1 : 0);
+  if (!alone)
+    hipLaunchKernelGGL(k_link_step, dim3(nb, c->V), dim3(kBlock), 0, c->stream, K, c->st);
   HIPCHK(c, hipGetLastError());
   if (readback)
     HIPCHK(c, hipMemcpyAsync(c->pin_block, c->iter_dev, c->iter_bytes, hipMemcpyDeviceToHost,
                              c->stream));
   return TAPGPU_OK;
+}
+
+static void launch_totals(tapgpu_ctx* c) {
+  hipLaunchKernelGGL(k_totals, dim3(link_blocks(c->E, c->V, false), c->V), dim3(kBlock), 0, c->stream,
+                     make_links(c), c->part, c->done, c->vht);
 }
 
 // Records what `issue` puts on the context's stream into an executable
@@ -3632,12 +3661,10 @@ static int capture(tapgpu_ctx* c, hipGraphExec_t* exec, F&& issue) {
 // captured again when the schedule that its launches bake in changes.
 // With m > 1 the graph holds m iterations back to back and one readback: a
 // variant that stops (or converges) in one of them is skipped by the rest
-// (its flag is off), and a step that needs a third line-search window is
-// retried unchanged by the following iterations and finished by the host
-// after the replay, so the results are those of m single replays.  Used
+// (its flag is off), so the results are those of m single replays.  Used
 // where an iteration is short enough for the launch and synchronisation
 // to matter.
-static int iter_graph(tapgpu_ctx* c, const Links& K, dim3 lgrid, int m) {
+static int iter_graph(tapgpu_ctx* c, const Links& K, int m) {
   const bool lds = use_lds(c);
   if (!lds) {
     int rc = ensure_hbm(c);
@@ -3649,10 +3676,10 @@ static int iter_graph(tapgpu_ctx* c, const Links& K, dim3 lgrid, int m) {
                             c->chase, c->qcap, c->hqcap, dbits, lds_threads(c)};
   if (c->g_iter && std::equal(key, key + 6, c->g_iter_key)) return TAPGPU_OK;
   int rc = capture(c, &c->g_iter, [&]() -> int {
+    const long long ny = (long long)c->V * c->E;
+    hipLaunchKernelGGL(k_iter_begin, dim3(grid_for(ny / kWave + 1)), dim3(kBlock), 0, c->stream,
+                       c->err_dev, c->counters, c->y, ny);
     for (int it = 0; it < m; ++it) {
-      const long long ny = (long long)c->V * c->E;
-      hipLaunchKernelGGL(k_iter_begin, dim3(grid_for(ny / kWave + 1)), dim3(kBlock), 0, c->stream,
-                         c->st, c->V, c->var_on, c->err_dev, c->counters, c->y, ny, it > 0 ? 1 : 0);
       c->defer_origin = true;
       c->pre_cleared = true;
       int r = lds ? aon_lds(c, 0, c->V, c->var_on) : aon_hbm(c, 0, c->V, c->var_on);
@@ -3660,7 +3687,7 @@ static int iter_graph(tapgpu_ctx* c, const Links& K, dim3 lgrid, int m) {
       c->pre_cleared = false;
       c->origin_pending = false;
       if (r) return r;
-      if ((r = issue_link_passes(c, K, lgrid, it == m - 1))) return r;
+      if ((r = issue_link_passes(c, K, it == m - 1))) return r;
     }
     return TAPGPU_OK;
   });
@@ -3670,33 +3697,32 @@ static int iter_graph(tapgpu_ctx* c, const Links& K, dim3 lgrid, int m) {
 }
 
 // The whole iteration of a batch on the lanes kernel as one graph:
-// k_iter_begin (flags, error flag, counters), pack, the lanes kernel, unpack,
-// the gate, the link passes and the readback.  The lane map and the memo
+// k_iter_begin (error flag, counters), pack, the lanes kernel, unpack, the
+// link passes and the readback.  The lane map and the memo
 // stamps are device data, set before each replay; the graph is captured
 // again when the number of groups or the kernel's schedule changes.
-static int lanes_graph(tapgpu_ctx* c, const Links& K, dim3 lgrid, int G) {
+static int lanes_graph(tapgpu_ctx* c, const Links& K, int G) {
   long long dbits;
   std::memcpy(&dbits, &c->lanes_delta_mult, sizeof dbits);
   const long long key[6] = {3 + (c->origin_order_ready ? 64 : 0) + 128 * c->link_mode, G, c->lanes_qcap,
                             dbits, (long long)c->lanes_lds, c->lanes_grid};
   if (c->g_iter && std::equal(key, key + 6, c->g_iter_key)) return TAPGPU_OK;
   int rc = capture(c, &c->g_iter, [&]() {
-    hipLaunchKernelGGL(k_iter_begin, dim3(1), dim3(kBlock), 0, c->stream, c->st, c->V, c->var_on,
-                       c->err_dev, c->counters, c->y, 0ll, 0);
+    hipLaunchKernelGGL(k_iter_begin, dim3(1), dim3(kBlock), 0, c->stream, c->err_dev, c->counters,
+                       c->y, 0ll);
     int r = launch_lanes(c, G, (long long)c->Z * G, nullptr);
     if (r) return r;
-    hipLaunchKernelGGL(k_lanes_gate, dim3(1), dim3(kBlock), 0, c->stream, c->err_dev, c->st, c->V);
-    return issue_link_passes(c, K, lgrid);
+    return issue_link_passes(c, K);
   });
   if (rc) return rc;
   std::copy(key, key + 6, c->g_iter_key);
   return TAPGPU_OK;
 }
 
-static int link_graph(tapgpu_ctx* c, const Links& K, dim3 lgrid) {
+static int link_graph(tapgpu_ctx* c, const Links& K) {
   if (c->g_link && c->g_link_mode == c->link_mode) return TAPGPU_OK;
   c->g_link_mode = c->link_mode;
-  return capture(c, &c->g_link, [&]() { return issue_link_passes(c, K, lgrid); });
+  return capture(c, &c->g_link, [&]() { return issue_link_passes(c, K); });
 }
 
 int tapgpu_set_link_passes(tapgpu_ctx* c, int mode, int window) {
@@ -3727,7 +3753,6 @@ int tapgpu_fw_run(tapgpu_ctx* c, int max_iters, double target_relgap, tapgpu_res
   c->stats = tapgpu_stats{};
   auto t_start = std::chrono::steady_clock::now();
   Links K = make_links(c);
-  const dim3 lgrid(kLinkBlocks, c->V);
   std::vector<unsigned char> hon(c->V);
   std::vector<VarState> hs(c->V);
   // variants already past the stop rule do not run (the loop test comes first)
@@ -3741,11 +3766,7 @@ int tapgpu_fw_run(tapgpu_ctx* c, int max_iters, double target_relgap, tapgpu_res
   if ((rc = upload(c, c->var_on, hon.data(), c->V))) return rc;
   // One synchronisation per iteration (or per replay of several): the
   // loading's error flag and counters, the variants' states and flags are
-  // read back together at the end.  On networks above kSmallLinks links a
-  // second line-search window pass is always queued and does nothing for
-  // variants whose lambda the first window decided; a variant that needs
-  // more windows skips the step and is finished by the host loop below
-  // (rare: lambda below 2^-31).  k_link_small runs every window itself.
+  // read back together at the end.
   if (!c->ev[2])
     for (auto& e : c->ev) HIPCHK(c, hipEventCreate(&e));
   if ((rc = upload_params(c, max_iters, target_relgap))) return rc;
@@ -3790,7 +3811,8 @@ int tapgpu_fw_run(tapgpu_ctx* c, int max_iters, double target_relgap, tapgpu_res
       m = c->graph_iters > 0 ? c->graph_iters
           : (c->last_iter_ms > 0 && c->last_iter_ms < 2.0) ? kMaxGraphIters : 1;
       // the loading's error flag and counters come back in the iteration block
-      if ((rc = iter_graph(c, K, lgrid, m))) return rc;
+      refresh_mirrors(c);
+      if ((rc = iter_graph(c, K, m))) return rc;
       HIPCHK(c, hipGraphLaunch(c->g_iter, c->stream));
       c->graph_launches += 1;
       c->origin_pending = true;
@@ -3801,7 +3823,7 @@ int tapgpu_fw_run(tapgpu_ctx* c, int max_iters, double target_relgap, tapgpu_res
     } else if (mode == 2) {
       const long long tasks = (long long)c->Z * G;
       if ((rc = lanes_reserve(c, tasks))) return rc;
-      if ((rc = lanes_graph(c, K, lgrid, G))) return rc;
+      if ((rc = lanes_graph(c, make_links(c, false), G))) return rc;
       HIPCHK(c, hipGraphLaunch(c->g_iter, c->stream));
       c->graph_launches += 1;
       HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -3810,21 +3832,16 @@ int tapgpu_fw_run(tapgpu_ctx* c, int max_iters, double target_relgap, tapgpu_res
                              &fallback)))
         return rc;
       if (fallback) {
-        // the gate kept every variant from stepping: open the step again,
-        // load with a per-origin kernel and run the link passes
-        hipLaunchKernelGGL(k_begin_step, dim3((c->V + 255) / 256), dim3(256), 0, c->stream, c->st,
-                           c->V, c->var_on);
+        // the error flag kept every variant from stepping: load with a
+        // per-origin kernel and run the link passes
         if ((rc = redo_per_origin(c, 0, c->V, c->var_on))) return rc;
-        if ((rc = issue_link_passes(c, K, lgrid))) return rc;
+        if ((rc = issue_link_passes(c, K))) return rc;
       }
     } else {
       if (tuned) {
         const long long ny = (long long)c->V * c->E;
         hipLaunchKernelGGL(k_iter_begin, dim3(grid_for(ny / kWave + 1)), dim3(kBlock), 0, c->stream,
-                           c->st, c->V, c->var_on, c->err_dev, c->counters, c->y, ny, 0);
-      } else {
-        hipLaunchKernelGGL(k_begin_step, dim3((c->V + 255) / 256), dim3(256), 0, c->stream, c->st,
-                           c->V, c->var_on);
+                           c->err_dev, c->counters, c->y, ny);
       }
       HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
       c->defer_origin = true;
@@ -3835,38 +3852,16 @@ int tapgpu_fw_run(tapgpu_ctx* c, int max_iters, double target_relgap, tapgpu_res
       if (rc) return rc;
       HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
       if (graphs) {
-        if ((rc = link_graph(c, K, lgrid))) return rc;
+        if ((rc = link_graph(c, K))) return rc;
         HIPCHK(c, hipGraphLaunch(c->g_link, c->stream));
         c->graph_launches += 1;
-      } else if ((rc = issue_link_passes(c, K, lgrid))) {
+      } else if ((rc = issue_link_passes(c, lanes_now ? make_links(c, false) : K))) {
         return rc;
       }
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if ((rc = absorb_pending(c))) return rc;
     c->stats.link_passes += 1;
-    auto need_more = [&]() {
-      bool more = false;
-      for (int v = 0; v < c->V; ++v) more = more || (c->pin_st[v].stepping && c->pin_st[v].need_more);
-      return more;
-    };
-    bool more = need_more();
-    if (more) c->stats.link_passes += 1;              // the queued second window was used
-    while (more) {
-      hipLaunchKernelGGL(k_link_partials, lgrid, dim3(kLinkThreads), 0, c->stream, K, c->st, c->part, 1);
-      hipLaunchKernelGGL(k_link_decide, dim3(c->V), dim3(kBlock), 0, c->stream, c->st, c->part,
-                         kLinkBlocks, 1, c->prm);
-      hipLaunchKernelGGL(k_link_step, lgrid, dim3(kBlock), 0, c->stream, K, c->st);
-      hipLaunchKernelGGL(k_finish_step, dim3((c->V + 255) / 256), dim3(256), 0, c->stream, c->st,
-                         c->V, c->var_on);
-      HIPCHK(c, hipGetLastError());
-      HIPCHK(c, hipMemcpyAsync(c->pin_st, c->st, sizeof(VarState) * c->V, hipMemcpyDeviceToHost,
-                               c->stream));
-      HIPCHK(c, hipMemcpyAsync(c->pin_on, c->var_on, c->V, hipMemcpyDeviceToHost, c->stream));
-      HIPCHK(c, hipStreamSynchronize(c->stream));
-      c->stats.link_passes += 1;
-      more = need_more();
-    }
     std::copy(c->pin_st, c->pin_st + c->V, hs.begin());
     std::copy(c->pin_on, c->pin_on + c->V, hon.begin());
     const double it_ms =
@@ -3887,7 +3882,7 @@ int tapgpu_fw_run(tapgpu_ctx* c, int max_iters, double target_relgap, tapgpu_res
       int rc2 = dalloc(c, &c->vht, 2 * (size_t)c->V);
       if (rc2) return rc2;
     }
-    hipLaunchKernelGGL(k_totals, dim3(c->V), dim3(kBlock), 0, c->stream, K, c->vht);
+    launch_totals(c);
     HIPCHK(c, hipGetLastError());
     std::vector<double> tot(2 * (size_t)c->V);
     HIPCHK(c, hipMemcpyAsync(hs.data(), c->st, sizeof(VarState) * c->V, hipMemcpyDeviceToHost,
@@ -3926,7 +3921,7 @@ int tapgpu_get_totals(tapgpu_ctx* c, int64_t variant, double* objective, double*
   if (rc) return rc;
   if (!c->initialised) return c->fail(TAPGPU_E_STATE, "tapgpu_fw_init was not called");
   if (!c->vht && (rc = dalloc(c, &c->vht, 2 * (size_t)c->V))) return rc;
-  hipLaunchKernelGGL(k_totals, dim3(c->V), dim3(kBlock), 0, c->stream, make_links(c), c->vht);
+  launch_totals(c);
   HIPCHK(c, hipGetLastError());
   double t[2];
   HIPCHK(c, hipMemcpyAsync(t, c->vht + 2 * variant, sizeof t, hipMemcpyDeviceToHost, c->stream));
