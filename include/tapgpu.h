@@ -335,16 +335,18 @@ double tapgpu_get_lanes_delta(const tapgpu_ctx *ctx);
 
 /* Launch form of tapgpu_fw_run's iterations (no counterpart in the
    reference, whose steps are host loops).  mode = 1 (the default): once the
-   loading's schedule is tuned, each iteration (opening kernel, loading,
-   both line-search windows, step, readback) is a replay of a captured HIP
-   graph -- on the per-origin LDS and HBM paths and on the lanes kernel;
-   elsewhere the link passes are.  On the per-origin paths iterations
-   shorter than 2 ms go 8 to a replay, so the launch and the
-   synchronisation are paid once for several.  mode = 2..8: that many
-   iterations per replay on those paths.  mode = 0: the same launches issued
-   one by one.  Profiling (tapgpu_set_profiling) issues them one by one too,
-   so the events around the loading are recorded.  Results do not depend on
-   it. */
+   loading's schedule is tuned, each iteration (loading, line search, step,
+   readback) is a replay of a captured HIP graph -- on the per-origin LDS and
+   HBM paths and on the lanes kernel; elsewhere the link passes are.  On the
+   per-origin paths iterations shorter than 2 ms go 8 to a replay, so the
+   launch and the synchronisation are paid once for several.  mode = 2..8:
+   that many iterations per replay on those paths.  Networks of up to 192
+   nodes, 1,024 links and 64 zones whose powers are all 4 run up to 256
+   iterations (and tapgpu_fw_init's loading) inside one kernel instead, with
+   the LDS strategy and the default link passes, unless the lanes kernel was
+   asked for (tapgpu_set_lanes).  mode = 0: the same launches issued one by
+   one.  Profiling (tapgpu_set_profiling) issues them one by one too, so the
+   events around the loading are recorded.  Results do not depend on it. */
 int tapgpu_set_graphs(tapgpu_ctx *ctx, int mode);
 int tapgpu_get_graphs(tapgpu_ctx *ctx, int *mode);
 

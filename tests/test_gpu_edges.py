@@ -1,0 +1,170 @@
+"""Sizes at which a kernel's tiling or dispatch changes: node counts around
+the slices of 64 and the one-workgroup kernel's limits, nodes with more links
+than an out-link record (4 lanes, 6 slots) or an in-link slice (16 rows)
+holds, link counts around a workgroup of the line search.  Labels equal the
+oracle's bit for bit; volumes, costs and step sizes of two paths are equal
+bit for bit (integer demand, so every partial sum is exact)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import pred_reaches_origin, pred_tie_check, random_demand
+
+pytestmark = pytest.mark.gpu
+
+
+def small_network(seed, N, Z, ft, extra, kind, hub=0):
+    """A two-way ring of the through nodes, every zone joined to one of them,
+    `extra` random links (self-loops and parallel links among them) and
+    `hub` links out of and into one through node."""
+    from traffic_assignment_amd import synth
+    rng = np.random.default_rng(seed)
+    thru = np.arange(ft, N + 1)
+    z = np.arange(1, ft)
+    t = rng.integers(ft, N + 1, z.size)
+    a = [thru, np.roll(thru, -1), z, t, rng.integers(1, N + 1, extra)]
+    b = [np.roll(thru, -1), thru, t, z, rng.integers(1, N + 1, extra)]
+    if hub:
+        h = rng.integers(ft, N + 1, hub)
+        c = np.full(hub, ft + (N - ft) // 2)
+        a += [c, h]
+        b += [h, c]
+    init, term = np.concatenate(a), np.concatenate(b)
+    order = np.lexsort((term, init))
+    init, term = init[order].astype(np.int64), term[order].astype(np.int64)
+    E = init.size
+    if kind == "ints":
+        cost = rng.integers(0, 4, E).astype(np.float64)
+    else:
+        cost = rng.uniform(0.01, 5.0, E)
+    net = synth.Network(num_zones=Z, num_nodes=N, first_thru_node=ft, init=init, term=term,
+                        capacity=rng.uniform(20.0, 200.0, E), length=np.ones(E), fftime=cost,
+                        B=np.full(E, 0.15), power=np.full(E, 4.0), speed=np.zeros(E),
+                        toll=np.zeros(E), ltype=np.ones(E, np.int16))
+    return net, rng
+
+
+@pytest.mark.parametrize("N,ft,hub", [(63, 1, 0), (64, 20, 5), (65, 1, 6), (128, 65, 7), (129, 64, 16),
+                                      (300, 1, 17), (1000, 90, 60), (4097, 300, 700)])
+@pytest.mark.parametrize("kind", ["cont", "ints"])
+def test_lds_kernel_records_and_slices(engine_mod, oracle_lib, N, ft, hub, kind):
+    import oracle
+    print(f"case lds edges N={N} ft={ft} hub={hub} {kind}", flush=True)
+    Z = min(max(ft - 1, 12), 40)
+    net, rng = small_network(N + hub, N, Z, ft, N, kind, hub)
+    dem = random_demand(net, rng)
+    origins = np.arange(1, Z + 1)
+    od, op = oracle.sssp_all(net, net.fftime)
+    with engine_mod.TapEngine(net, dem) as eng:
+        eng.set_strategy("lds")
+        d, p = eng.sssp(origins)
+        assert np.array_equal(d[1:].view(np.int64), od[1:].view(np.int64))
+        bad, _ = pred_tie_check(net, net.fftime, d, p, op, origins)
+        assert bad == 0
+        pred_reaches_origin(net, d, p, origins)
+        ys = []
+        for q in (-1, 0, 1, 16):                       # queue sizes: scan rounds and mixed rounds
+            eng.set_origin_queue(q)
+            ys.append(eng.aon())
+        eng.set_strategy("hbm")
+        ys.append(eng.aon())
+    for y in ys[1:]:
+        assert np.array_equal(y, ys[0])
+
+
+def _run(engine_mod, net, dem, graphs, chunks, window=0, **kw):
+    with engine_mod.TapEngine(net, dem, **kw) as eng:
+        eng.set_graphs(graphs)
+        eng.set_link_passes(0, window)
+        eng.fw_init()
+        out = [eng.flows(v) for v in range(eng.V)]
+        for n in chunks:
+            eng.fw_run(max_iters=n)
+            out += [eng.flows(v) for v in range(eng.V)]
+        return out, [eng.trace(v) for v in range(eng.V)]
+
+
+def _same(a, b):
+    for (xa, ca), (xb, cb) in zip(a[0], b[0]):
+        assert np.array_equal(xa, xb) and np.array_equal(ca, cb)
+    for ta, tb in zip(a[1], b[1]):
+        assert np.array_equal(ta["lambda_"], tb["lambda_"])
+        # compensated sums in another order: a few units in the last place
+        for k in ("objective", "vht"):
+            assert np.allclose(ta[k], tb[k], rtol=1e-14, atol=0.0)
+
+
+@pytest.mark.parametrize("N,Z,ft", [(2, 2, 1), (24, 24, 1), (31, 8, 9), (32, 32, 1), (33, 10, 11), (64, 16, 1),
+                                    (65, 30, 31), (128, 17, 1), (129, 40, 41), (192, 64, 65), (193, 20, 1)])
+@pytest.mark.parametrize("kind", ["cont", "ints"])
+def test_one_workgroup_iterations(engine_mod, N, Z, ft, kind):
+    """Iterations inside one kernel (up to 192 nodes, 64 zones) against the
+    same iterations launch by launch: the wavefront's and half wavefront's
+    origins, two and three nodes a lane, nodes with more in-links than its
+    registers hold, zero-cost links and their level ties."""
+    print(f"case one-workgroup N={N} Z={Z} ft={ft} {kind}", flush=True)
+    net, rng = small_network(N, N, Z, ft, 2 * N, kind, hub=min(9, N // 4))
+    dem = random_demand(net, rng)
+    _same(_run(engine_mod, net, dem, 1, (5, 12)), _run(engine_mod, net, dem, 0, (5, 12)))
+
+
+def test_one_workgroup_batch_and_windows(engine_mod):
+    """Three variants with their own capacities, presence and stopping
+    iteration; line-search windows of two step sizes; a launch's 256
+    iterations passed; deep steps on a converged network."""
+    print("case one-workgroup batch", flush=True)
+    net, rng = small_network(7, 40, 12, 1, 60, "cont")
+    dem = random_demand(net, rng)
+    E = net.num_links
+    ring = np.isin(np.arange(E), rng.choice(E, E // 3, replace=False))
+    thru = np.abs(net.init - net.term) % (net.num_nodes - 2) <= 1        # the ring's own links stay
+    present = np.stack([np.ones(E, bool), ~ring | thru, np.ones(E, bool)]).astype(np.uint8)
+    cap = np.stack([net.capacity, net.capacity, 0.7 * net.capacity])
+    kw = dict(num_variants=3, present=present, capacity=cap)
+    for window in (0, 2):
+        _same(_run(engine_mod, net, dem, 1, (3, 300), window, **kw),
+              _run(engine_mod, net, dem, 0, (3, 300), window, **kw))
+    with engine_mod.TapEngine(net, dem) as a, engine_mod.TapEngine(net, dem) as b:
+        b.set_graphs(0)
+        for eng in (a, b):
+            eng.fw_init()
+        ra, rb = a.fw_run(3000, 1e-3)[0], b.fw_run(3000, 1e-3)[0]
+        assert ra["iterations"] == rb["iterations"] and ra["converged"] == rb["converged"]
+        assert np.array_equal(a.flows()[0], b.flows()[0])
+
+
+def test_one_workgroup_no_path(engine_mod):
+    """Demand between disconnected zones is an error in the one-workgroup
+    kernel too, and the engine works on afterwards."""
+    from traffic_assignment_amd import synth
+    net, rng = small_network(3, 20, 6, 7, 10, "cont")
+    keep = net.term != 4                                # nothing reaches zone 4
+    import dataclasses
+    f = {k: getattr(net, k)[keep] for k in ("init", "term", "capacity", "length", "fftime", "B", "power",
+                                            "speed", "toll", "ltype")}
+    cut = dataclasses.replace(net, **f)
+    dem = synth.Demand(6, np.array([0, 1, 1, 1, 1, 1, 1]), np.array([4]), np.array([5.0]))
+    with engine_mod.TapEngine(cut, dem) as eng:
+        with pytest.raises(engine_mod.NoPathError):
+            eng.fw_init()
+        d, _ = eng.sssp([1])
+        assert d[4, 0] > 1.7e308
+
+
+@pytest.mark.parametrize("E", [255, 256, 257, 511, 512, 513, 1025])
+def test_line_search_blocks(engine_mod, E):
+    """Link counts around a workgroup of the line search: one workgroup per
+    variant against many."""
+    print(f"case line search E={E}", flush=True)
+    net, rng = small_network(E, 80, 10, 1, E - 160, "cont")
+    assert net.num_links == E
+    dem = random_demand(net, rng)
+    res = []
+    for mode in (1, 2):
+        with engine_mod.TapEngine(net, dem) as eng:
+            eng.set_link_passes(mode)
+            eng.fw_init()
+            eng.fw_run(max_iters=20)
+            res.append(([eng.flows()], [eng.trace()]))
+    _same(*res)

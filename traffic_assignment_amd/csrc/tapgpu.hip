@@ -1568,22 +1568,75 @@ __global__ __launch_bounds__(kBlock) void k_costs(Links K, int mode, const unsig
 // sums takes 114), then one thread per sum merges the wavefronts.  The
 // result is in out[] for every thread after the call's last barrier; sh
 // holds a row per wavefront.
+//
+// The exchanges are register moves, not LDS permutes: between the halves of
+// 32 and of 16 lanes the swap instructions, which hand over and keep in
+// one, inside a row of 16 the data-parallel moves.  (kOff 4 is i ^ 7: it
+// also turns the lanes of a quad round, whose shares are all different yet.)
+template <int kOff>
+__device__ __forceinline__ unsigned xchg_u32(unsigned x) {
+  constexpr int ctrl = kOff == 8 ? 0x128 /* row_ror:8 */ : kOff == 4 ? 0x141 /* row_half_mirror */
+                       : kOff == 2 ? 0x4E /* quad_perm 2,3,0,1 */ : 0xB1 /* quad_perm 1,0,3,2 */;
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, ctrl, 0xf, 0xf, false);
+}
+template <int kOff>
+__device__ __forceinline__ double xchg(double x) {
+  const unsigned long long b = as_b(x);
+  const unsigned lo = xchg_u32<kOff>((unsigned)b), hi = xchg_u32<kOff>((unsigned)(b >> 32));
+  return as_d((unsigned long long)hi << 32 | lo);
+}
+// lower half: {own a, partner's a}; upper half: {partner's b, own b}
+template <int kOff>
+__device__ __forceinline__ void swap_halves(double& a, double& b) {
+  const unsigned long long x = as_b(a), y = as_b(b);
+  unsigned r0[2], r1[2];
+  if constexpr (kOff == 32) {
+    auto p = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    auto q = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    r0[0] = p[0]; r0[1] = p[1]; r1[0] = q[0]; r1[1] = q[1];
+  } else {
+    auto p = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    auto q = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    r0[0] = p[0]; r0[1] = p[1]; r1[0] = q[0]; r1[1] = q[1];
+  }
+  a = as_d((unsigned long long)r1[0] << 32 | r0[0]);
+  b = as_d((unsigned long long)r1[1] << 32 | r0[1]);
+}
+
 template <int kOff, int kHave>
 __device__ __forceinline__ void halve_acc(tap_acc* v, int lane) {
   constexpr int kKeep = (kHave + 1) / 2;
-  const bool up = lane & kOff;
 #pragma unroll
   for (int i = 0; i < kKeep; ++i) {
-    const tap_acc lo = v[i];
-    tap_acc hi{0.0, 0.0};
+    tap_acc lo = v[i], hi{0.0, 0.0};
     if (kKeep + i < kHave) hi = v[kKeep + i];
-    const tap_acc give = up ? lo : hi;
-    tap_acc keep = up ? hi : lo, got;
-    got.s = __shfl_xor(give.s, kOff);
-    got.c = __shfl_xor(give.c, kOff);
-    tap_acc_merge(&keep, got);
-    v[i] = keep;
+    if constexpr (kOff >= 16) {
+      swap_halves<kOff>(lo.s, hi.s);
+      swap_halves<kOff>(lo.c, hi.c);
+      tap_acc_merge(&lo, hi);
+      v[i] = lo;
+    } else {
+      const bool up = lane & kOff;
+      const tap_acc give = up ? lo : hi;
+      tap_acc keep = up ? hi : lo, got;
+      got.s = xchg<kOff>(give.s);
+      got.c = xchg<kOff>(give.c);
+      tap_acc_merge(&keep, got);
+      v[i] = keep;
+    }
   }
+}
+
+// One sum, whose shares are in both lanes of a pair: merged in both, the
+// lower lane's share first.
+template <int kOff>
+__device__ __forceinline__ void pair_acc(tap_acc* v, int lane) {
+  tap_acc got;
+  got.s = xchg<kOff>(v->s);
+  got.c = xchg<kOff>(v->c);
+  tap_acc a = (lane & kOff) ? got : *v;
+  tap_acc_merge(&a, (lane & kOff) ? *v : got);
+  *v = a;
 }
 
 template <int kWaves>
@@ -1595,15 +1648,7 @@ __device__ void block_reduce_acc(tap_acc* v, tap_acc* sh /* [kWaves][kQ] */, tap
   halve_acc<8, 5>(v, lane);        // 3 and 2
   halve_acc<4, 3>(v, lane);        // 2 and 1
   halve_acc<2, 2>(v, lane);        // 1 and 1
-  {
-    tap_acc got;
-    got.s = __shfl_xor(v[0].s, 1);
-    got.c = __shfl_xor(v[0].c, 1);
-    // (the lower lane's share first in both lanes)
-    tap_acc a = (lane & 1) ? got : v[0];
-    tap_acc_merge(&a, (lane & 1) ? v[0] : got);
-    v[0] = a;
-  }
+  pair_acc<1>(v, lane);
   const int b5 = lane >> 5 & 1, b4 = lane >> 4 & 1, b3 = lane >> 3 & 1, b2 = lane >> 2 & 1, b1 = lane >> 1 & 1;
   const int in5 = 3 * b3 + 2 * b2 + b1;                       // of the 5 sums of this 8-lane group
   const int q = 10 * b5 + 5 * b4 + in5;
@@ -1651,20 +1696,18 @@ __device__ __forceinline__ void link_sums(tap_acc* acc, const Links& K, size_t i
 // Per variant: lambda (first 2^-j with g <= 0, the reference's rule), then
 // gap, objective, lower bound, relative gap, average excess cost, trace
 // record, stop test.
-// The decision of one window for one variant from its merged sums acc[kQ]
-// (thread 0 of the caller): on the first window the iteration's scalars
-// and trace record, then lambda = the first 2^-j with g <= 0, or a request
-// for the next window (need_more, jnext).
+// The decision of one window for one variant from its merged sums acc[kQ],
+// by one wavefront (all its lanes keep the same state; lane 0 writes): on
+// the first window the iteration's scalars and trace record, then lambda =
+// the first 2^-j with g <= 0 (a lane looks at each j), or a request for the
+// next window (need_more, jnext).
 __device__ __forceinline__ void decide_window(VarState& s, const tap_acc* acc, int only_g,
-                                              const FwParams* prm, int var) {
-  tapgpu_iter* const trace = prm->trace;
-  const int trace_cap = prm->trace_cap, max_iters = prm->max_iters;
-  const double target = prm->target;
-  const int jwin = prm->jwin;
-  double gj[kJ];
-#pragma unroll
-  for (int j = 0; j < kJ; ++j) gj[j] = tap_acc_value(acc[3 + j]);
+                                              const FwParams& prm, int var) {
+  const int lane = lane_id();
   const int jbase = only_g ? s.jnext : 0;
+  const int jl = min(lane, kJ - 1);
+  const unsigned long long neg = ballot(tap_acc_value(acc[3 + jl]) <= 0) & ((1ull << kJ) - 1ull);
+  tapgpu_iter* const rec = s.iter < prm.trace_cap ? prm.trace + (size_t)var * prm.trace_cap + s.iter : nullptr;
   if (!only_g) {
     const double g0 = tap_acc_value(acc[0]);
     s.objective = tap_acc_value(acc[1]);
@@ -1673,7 +1716,7 @@ __device__ __forceinline__ void decide_window(VarState& s, const tap_acc* acc, i
     s.need_more = 0;
     if (g0 >= 0) {
       s.lambda = 0.0; s.found = 1;
-    } else if (gj[0] <= 0) {
+    } else if (neg & 1ull) {
       s.lambda = 1.0; s.found = 1;
     }
     // record the iteration's scalars (lambda filled below)
@@ -1681,37 +1724,35 @@ __device__ __forceinline__ void decide_window(VarState& s, const tap_acc* acc, i
     const double lb = s.objective - gap;
     if (lb > s.best_lb) s.best_lb = lb;
     if (s.best_lb != 0) s.relgap = (s.objective - s.best_lb) / fabs(s.best_lb);
-    if (s.iter < trace_cap) {
+    if (rec && lane == 0) {
       tapgpu_iter t;
       t.lambda = 0.0; t.gap = gap; t.objective = s.objective; t.lowerbound = lb;
       t.best_lowerbound = s.best_lb; t.relgap = s.relgap;
       t.avg_excess = -g0 / s.total_demand; t.vht = s.vht;
-      trace[(size_t)var * trace_cap + s.iter] = t;
+      *rec = t;
     }
   }
   if (!s.found) {
-    for (int j = std::max(jbase, 1); j < jbase + jwin && j <= kMaxHalvings; ++j) {
-      if (gj[j - jbase] <= 0) {
-        s.lambda = ldexp(1.0, -j);
-        s.found = 1;
-        break;
-      }
-    }
-    if (!s.found) {
-      if (jbase + jwin > kMaxHalvings) {
-        s.lambda = 0.0;            // bisection cap reached: lambda_left == 0
-        s.found = 1;
-      } else {
-        s.need_more = 1;
-        s.jnext = jbase + jwin;
-      }
+    // steps jbase .. jbase + jwin - 1, from 2^-1 on and down to 2^-kMaxHalvings
+    const int n = min(prm.jwin, kMaxHalvings + 1 - jbase);
+    unsigned long long m = neg & ((1ull << n) - 1ull);
+    if (jbase == 0) m &= ~1ull;
+    if (m) {
+      s.lambda = ldexp(1.0, -(jbase + __ffsll((long long)m) - 1));
+      s.found = 1;
+    } else if (jbase + prm.jwin > kMaxHalvings) {
+      s.lambda = 0.0;            // bisection cap reached: lambda_left == 0
+      s.found = 1;
+    } else {
+      s.need_more = 1;
+      s.jnext = jbase + prm.jwin;
     }
   }
   if (s.found) {
     s.need_more = 0;
-    if (s.iter < trace_cap) trace[(size_t)var * trace_cap + s.iter].lambda = s.lambda;
+    if (rec && lane == 0) rec->lambda = s.lambda;
     s.iter += 1;
-    s.active = (max_iters <= 0 || s.iter < max_iters) && (target <= 0 || s.relgap > target);
+    s.active = (prm.max_iters <= 0 || s.iter < prm.max_iters) && (prm.target <= 0 || s.relgap > prm.target);
   }
 }
 
@@ -1822,14 +1863,17 @@ __global__ __launch_bounds__(kBlock) void k_link_search(Links K, VarState* st, u
   };
   window(0, true, blockIdx.x * kBlock + tid, nb * kBlock);
   if (nb > 1 && !merge_blocks(sums, sh, part + (size_t)var * nb * kQ, &done[var])) return;
-  VarState s;                                                // (thread 0's)
-  if (tid == 0) s = st[var];
+  VarState s{};                                              // (kept by wavefront 0)
+  FwParams p{};
+  if (tid < kWave) { s = st[var]; p = *prm; }
   for (int only_g = 0;; only_g = 1) {
-    if (tid == 0) {
-      decide_window(s, sums, only_g, prm, var);
-      s_more = s.need_more;
-      s_jnext = s.jnext;
-      s_lambda = s.lambda;
+    if (tid < kWave) {
+      decide_window(s, sums, only_g, p, var);
+      if (tid == 0) {
+        s_more = s.need_more;
+        s_jnext = s.jnext;
+        s_lambda = s.lambda;
+      }
     }
     __syncthreads();
     if (!s_more) break;
@@ -2014,6 +2058,8 @@ struct tapgpu_ctx {
   size_t iter_bytes = 0;
   // lanes kernel (batched loading, variants in wavefront lanes)
   int lanes_min = 0;                  // active variants needed to use it (0: never)
+  bool lanes_auto = true;             // lanes_min is the default
+  bool tiny_ok = false;               // the one-workgroup kernel holds this network
   bool lanes_ok = false;              // its LDS (bitmaps + queues) fits
   int lanes_qcap = 0;                 // LDS frontier queue entries per round
   int lanes_qcap_max = 0;             // entries its LDS allocation holds
@@ -2034,6 +2080,8 @@ struct tapgpu_ctx {
   bool profiling = false;
   hipEvent_t ev[2 * 8] = {};
   std::vector<void*> allocs;
+  unsigned char* block_at = nullptr;  // balloc: the rest of the current block
+  size_t block_left = 0;
 
   int fail(int code, const char* fmt, ...) {
     char buf[512];
@@ -2068,6 +2116,29 @@ int dalloc(tapgpu_ctx* ctx, T** p, size_t n) {
                      hipGetErrorString(e));
   }
   ctx->allocs.push_back(*p);
+  return TAPGPU_OK;
+}
+
+// dalloc for the arrays a context keeps for life: carved out of blocks, so
+// that creating a small context costs a few device allocations.
+template <class T>
+int balloc(tapgpu_ctx* ctx, T** p, size_t n) {
+  constexpr size_t kBlockBytes = 4ull << 20;
+  const size_t bytes = (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255;
+  *p = nullptr;
+  if (bytes > ctx->block_left) {
+    unsigned char* b = nullptr;
+    if (int rc = dalloc(ctx, &b, std::max(bytes, kBlockBytes))) return rc;
+    if (bytes >= kBlockBytes) {                  // (a block of its own)
+      *p = (T*)b;
+      return TAPGPU_OK;
+    }
+    ctx->block_at = b;
+    ctx->block_left = kBlockBytes;
+  }
+  *p = (T*)ctx->block_at;
+  ctx->block_at += bytes;
+  ctx->block_left -= bytes;
   return TAPGPU_OK;
 }
 
@@ -2744,6 +2815,7 @@ int aon_hbm(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
 }
 
 #include "taplanes.inc"
+#include "taptiny.inc"
 
 // The lanes kernel loads a batch when at least lanes_min of its variants
 // are active (lanes_min 0: never).
@@ -2752,6 +2824,14 @@ bool use_lanes(tapgpu_ctx* c, int v0, int Vn, const unsigned char* h_on) {
   int n = 0;
   for (int v = v0; v < v0 + Vn; ++v) n += (!h_on || h_on[v]) ? 1 : 0;
   return n >= c->lanes_min;
+}
+
+// Whether iterations run in the one-workgroup kernel: a network it holds, on
+// the LDS strategy and the default link passes (h_on as for use_lanes; a
+// batch for which the lanes kernel was asked for keeps it).
+bool use_tiny(tapgpu_ctx* c, const unsigned char* h_on) {
+  return c->tiny_ok && c->graphs && !c->profiling && use_lds(c) && c->split == 0 && c->link_mode == 0 &&
+         (c->lanes_auto || !use_lanes(c, 0, c->V, h_on));
 }
 
 // All-or-nothing loading of variants [v0, v0 + Vn) (groups of those
@@ -2974,6 +3054,10 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
       c->qcap = c->qcap_max;
       c->lds_bytes = origin_lds_bytes(c->N, c->qcap_max);
     }
+    bool pow4 = true;
+    for (int64_t j = 0; j < (pw_v ? V * E : E); ++j) pow4 = pow4 && (pw_v ? pw_v : net->power)[j] == 4.0;
+    c->tiny_ok = c->lds_ok && pow4 && tiny_fits(c->N, c->E, c->Z) &&
+                 tiny_lds_bytes(c->N, c->E) + 128 <= (size_t)lds_max;
     c->hbm_lds = origin_hbm_lds_bytes(N, 0);
     c->hbm_ok = c->hbm_lds + 256 <= (size_t)lds_max;
     if (c->hbm_ok) {
@@ -3079,7 +3163,7 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
     c->pin_on = b + 144 + sizeof(VarState) * (size_t)V;
   }
   int rc;
-#define ALLOC(ptr, n) if ((rc = dalloc(c, &c->ptr, (n)))) return rc
+#define ALLOC(ptr, n) if ((rc = balloc(c, &c->ptr, (n)))) return rc
   ALLOC(fw_off, N + 1); ALLOC(fw_dst, E); ALLOC(rv_off, N + 1); ALLOC(rv_src, E);
   ALLOC(rv_eid, E); ALLOC(tail, E); ALLOC(rvpos, E);
   ALLOC(t0, VE); ALLOC(cap, VE); ALLOC(B, VE); ALLOC(pw, VE); ALLOC(present, VE);
@@ -3089,7 +3173,7 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
   ALLOC(flags, c->flags_cap);
   {
     c->iter_bytes = 16 + 128 + sizeof(VarState) * (size_t)V + (size_t)V;
-    if ((rc = dalloc(c, &c->iter_dev, c->iter_bytes))) return rc;
+    if ((rc = balloc(c, &c->iter_dev, c->iter_bytes))) return rc;
     c->err_dev = (int*)c->iter_dev;
     c->counters = (unsigned long long*)(c->iter_dev + 16);
     c->st = (VarState*)(c->iter_dev + 144);
@@ -3142,12 +3226,15 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
     HIPCHK(c, hipGetLastError());
   }
   c->h_odc = std::move(odc);
-  if ((rc = dalloc(c, &c->od_start, Z + 1))) return rc;
-  if ((rc = dalloc(c, &c->od_dest, h_od_dest.size()))) return rc;
-  if ((rc = dalloc(c, &c->od_val, h_od_val.size()))) return rc;
+  if ((rc = balloc(c, &c->od_start, Z + 1))) return rc;
+  if ((rc = balloc(c, &c->od_dest, h_od_dest.size()))) return rc;
+  if ((rc = balloc(c, &c->od_val, h_od_val.size()))) return rc;
   if ((rc = upload(c, c->od_start, h_od_start.data(), Z + 1))) return rc;
   if ((rc = upload(c, c->od_dest, h_od_dest.data(), h_od_dest.size()))) return rc;
   if ((rc = upload(c, c->od_val, h_od_val.data(), h_od_val.size()))) return rc;
+  if (c->tiny_ok)
+    HIPCHK(c, hipFuncSetAttribute(tiny_kernel(c->N), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)tiny_lds_bytes(c->N, c->E)));
   if (c->lds_ok) {
     HIPCHK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(k_origin_lds<1024>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->lds_bytes));
@@ -3581,6 +3668,13 @@ int tapgpu_fw_init(tapgpu_ctx* c, const double* warm_volumes) {
   HIPCHK(c, hipMemsetAsync(c->var_on, 1, c->V, c->stream));
   if (warm_volumes) {
     if ((rc = upload(c, c->x, warm_volumes, (size_t)c->V * c->E))) return rc;
+  } else if (use_tiny(c, nullptr)) {
+    // the loading, x = y and c = BPR(x) in one launch
+    hipLaunchKernelGGL(k_iter_begin, dim3(1), dim3(kBlock), 0, c->stream, c->err_dev, c->counters, c->y, 0ll);
+    if ((rc = launch_tiny(c, 1))) return rc;
+    if ((rc = finish_origin(c, c->V, std::chrono::steady_clock::now()))) return rc;
+    c->initialised = true;
+    return TAPGPU_OK;
   } else {
     if ((rc = launch_costs(c, 0, nullptr, 0, c->V))) return rc;   // Wa = t0
     if ((rc = load_variants(c, 0, c->V, nullptr, nullptr))) return rc;
@@ -3777,12 +3871,29 @@ int tapgpu_fw_run(tapgpu_ctx* c, int max_iters, double target_relgap, tapgpu_res
     if (c->trace_cap < 1 << 30) {
       int maxit = 0;
       for (int v = 0; v < c->V; ++v) maxit = std::max(maxit, hs[v].iter);
-      if (maxit + kMaxGraphIters >= c->trace_cap) {
-        if ((rc = ensure_trace(c, std::max(2 * c->trace_cap, maxit + kMaxGraphIters + 1)))) return rc;
+      const int ahead = std::max(kMaxGraphIters, kTinyIters);       // iterations before the next look
+      if (maxit + ahead >= c->trace_cap) {
+        if ((rc = ensure_trace(c, std::max(2 * c->trace_cap, maxit + ahead + 1)))) return rc;
         if ((rc = upload_params(c, max_iters, target_relgap))) return rc;
       }
     }
     auto t_it = std::chrono::steady_clock::now();
+    if (use_tiny(c, hon.data())) {
+      // up to kTinyIters iterations of every variant in one launch
+      hipLaunchKernelGGL(k_iter_begin, dim3(1), dim3(kBlock), 0, c->stream, c->err_dev, c->counters, c->y, 0ll);
+      if ((rc = launch_tiny(c, 0))) return rc;
+      HIPCHK(c, hipMemcpyAsync(c->pin_block, c->iter_dev, c->iter_bytes, hipMemcpyDeviceToHost, c->stream));
+      HIPCHK(c, hipStreamSynchronize(c->stream));
+      int64_t done = 0;
+      for (int v = 0; v < c->V; ++v) done += c->pin_st[v].iter - hs[v].iter;
+      if ((rc = absorb_origin(c, c->pin_err, c->pin_cnt, 0, std::chrono::steady_clock::now()))) return rc;
+      c->stats.origin_blocks += (int64_t)c->Z * done;
+      c->stats.link_passes += done / c->V;
+      std::copy(c->pin_st, c->pin_st + c->V, hs.begin());
+      std::copy(c->pin_on, c->pin_on + c->V, hon.begin());
+      c->stats.link_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_it).count();
+      continue;
+    }
     if ((rc = origin_order_update(c))) return rc;      // (before any capture)
     // with the schedule already tuned, one kernel opens the iteration and
     // clears what the loading would clear
@@ -4120,6 +4231,7 @@ int tapgpu_set_lanes(tapgpu_ctx* c, int min_active) {
   if (min_active != 0 && !c->lanes_ok)
     return c->fail(TAPGPU_E_ARG, "frontier bitmaps of this network do not fit LDS");
   c->lanes_min = min_active < 0 ? (c->V > 1 ? kLanesMinDefault : 0) : min_active;
+  c->lanes_auto = min_active < 0;
   return TAPGPU_OK;
 }
 

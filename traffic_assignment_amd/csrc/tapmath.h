@@ -29,13 +29,13 @@ TAP_HD double tap_pow4(double x)
 {
   const double h1 = x * x;
   const double h2 = h1 * h1;
-  if (!(h2 < 1e300) || h2 < 1e-280)      /* overflow, zero or near-subnormal */
-    return h2;
   const double l1 = TAP_FMA(x, x, -h1);
   const double l2 = TAP_FMA(h1, h1, -h2);
   double t = TAP_FMA(2.0 * h1, l1, l2);
   t = TAP_FMA(l1, l1, t);
-  return h2 + t;
+  /* overflow, zero or near-subnormal: h2 as it is (a select, not a branch:
+     the step sizes of a line search are evaluated side by side) */
+  return (!(h2 < 1e300) || h2 < 1e-280) ? h2 : h2 + t;
 }
 
 /* any other power: the platform pow, kept out of line so that the loops
