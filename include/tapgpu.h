@@ -269,7 +269,7 @@ int tapgpu_set_strategy(tapgpu_ctx *ctx, int strategy);
    many labels a thread lowers and then expands itself, in a chain, within
    one round (0: every lowered node waits for the next round).  -1 (the
    default): tuned on the next loading by timing each candidate
-   (0, 2, 4, 8, 16, 32) on the real launch.  Results do not depend on it. */
+   (0, 2, 4, 8, 16, 32) on the real launch, if any of its rounds scans.  Results do not depend on it. */
 int tapgpu_set_origin_chase(tapgpu_ctx *ctx, int chase);
 int tapgpu_get_origin_chase(const tapgpu_ctx *ctx);
 
@@ -317,7 +317,9 @@ int tapgpu_get_strategy(const tapgpu_ctx *ctx);
    wavefront (one workgroup per (origin, group of up to 64 variants), labels
    node-major in HBM, predecessors taken along the demand walks).  A loading
    of a batch uses it when at least min_active of its variants are active;
-   0: never; -1 (the default): 16 for batched contexts, never for plain ones.
+   0: never; -1 (the default): 16 for batched contexts, never for plain ones,
+   and on networks whose labels fit LDS only where the network's size and
+   the number of active variants make it the faster one.
    A loading that meets a node whose tight in-links all come from tails with
    its own label (zero-cost links) is redone by the per-origin strategy.
    Results do not depend on it (same trees, same volumes bit for bit). */

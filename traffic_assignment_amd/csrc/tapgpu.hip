@@ -523,7 +523,8 @@ struct OriginArgs {
                                      //     relax rounds, longest loading walk,
                                      //     tree links loaded, walk steps, -,
                                      //     wall-clock ticks of relaxation,
-                                     //     predecessors, loading
+                                     //     predecessors, loading; [12] rounds
+                                     //     that overflowed the LDS queue
   // block x handles origin src_list[x] (shortest-path-only mode: start
   // nodes; LDS loadings: origins longest first)
   const int* src_list;
@@ -745,7 +746,7 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
   const int jq = min(j0, qcap);
   const int pass = min(kPass, qcap);
   int r = 0, qn;
-  unsigned n_listed = 0;                   // (wave-uniform)
+  unsigned n_listed = 0, n_scans = 0;      // (wave-uniform)
   for (;;) {
     unsigned pf = 0;
     if (pf_node >= 0)
@@ -770,6 +771,7 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
       for (int j = j0; j < qn; j += kPass) expand(qr[j]);
       n_listed += (unsigned)qn;
     } else {
+      ++n_scans;
       for (int v0 = tid; v0 < N; v0 += BLOCK) {
         if (!(__hip_atomic_load(&key[v0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & 1ull)) continue;
         int x = v0;
@@ -794,6 +796,7 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
     pf_sink ^= pf;
   }
   if (tid == 0) n_exp += n_listed;
+  if (n_scans && tid == 0 && A.counters) atomicAdd(&A.counters[12], (unsigned long long)n_scans);
   if (qn) {                     // only possible with negative costs
     if (tid == 0 && atomicCAS(&A.err[0], 0, 2) == 0) { A.err[1] = src; A.err[2] = 0; }
     return;
@@ -2059,6 +2062,7 @@ struct tapgpu_ctx {
   // lanes kernel (batched loading, variants in wavefront lanes)
   int lanes_min = 0;                  // active variants needed to use it (0: never)
   bool lanes_auto = true;             // lanes_min is the default
+  int cus = 0;                        // compute units of the device
   bool tiny_ok = false;               // the one-workgroup kernel holds this network
   bool lanes_ok = false;              // its LDS (bitmaps + queues) fits
   int lanes_qcap = 0;                 // LDS frontier queue entries per round
@@ -2417,6 +2421,7 @@ void launch_lds(tapgpu_ctx* c, dim3 grid, hipStream_t st, const OriginArgs& A, i
 // fastest (the result is the same for every candidate; the last launch
 // below, with the chosen value, is the one whose volumes are kept).
 constexpr int kChaseCandidates[] = {0, 2, 4, 8, 16, 32};
+constexpr int kTuneBlocks = 4096;              // workgroups of a tuning launch on a batch
 
 int ensure_hbm(tapgpu_ctx* c);
 
@@ -2522,16 +2527,20 @@ int tune_chase(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
     for (auto& e : c->ev) HIPCHK(c, hipEventCreate(&e));
   float best_ms = 0.f;
   int best = kDefaultChase;
+  HIPCHK(c, hipMemsetAsync(c->counters, 0, sizeof(unsigned long long) * 16, c->stream));
   for (int k : kChaseCandidates) {
     c->chase = k;
     float ms = 0.f;
     int rc = launch_origin(c, v0, Vn, var_on, &ms);
     if (rc) return rc;
     int herr = 0;
+    unsigned long long scans = 0;
     HIPCHK(c, hipMemcpyAsync(&herr, c->err_dev, sizeof herr, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(&scans, c->counters + 12, sizeof scans, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (herr) break;                    // reported by the caller's launch
     if (best_ms == 0.f || ms < best_ms) { best_ms = ms; best = k; }
+    if (!scans) break;                  // every round ran from the queue: the length plays no part
   }
   c->chase = best;
   c->stats.origin_tune_ms += best_ms;
@@ -2669,12 +2678,14 @@ int aon_lds(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
   auto t0 = std::chrono::steady_clock::now();
   if (int rc = origin_order_update(c)) return rc;
   if (!c->pre_cleared) HIPCHK(c, hipMemsetAsync(c->err_dev, 0, sizeof(int) * 3, c->stream));
+  // candidates run on as many variants as fill the chip several times over
+  const int Vt = var_on ? Vn : (int)std::min<long long>(Vn, 1 + kTuneBlocks / std::max(c->Z, 1));
   if (c->lds_block < 0 && c->Z > 0) {
     // workgroup and queue size first, then the chain length, on the LDS
     // kernel alone
     const int keep = c->split;
     c->split = 0;
-    int rc = tune_lds_shape(c, v0, Vn, var_on);
+    int rc = tune_lds_shape(c, v0, Vt, var_on);
     c->split = keep;
     if (rc) return rc;
     HIPCHK(c, hipMemsetAsync(c->err_dev, 0, sizeof(int) * 3, c->stream));
@@ -2682,7 +2693,7 @@ int aon_lds(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
   if (c->chase < 0 && c->Z > 0) {
     const int keep = c->split;
     c->split = 0;
-    int rc = tune_chase(c, v0, Vn, var_on);
+    int rc = tune_chase(c, v0, Vt, var_on);
     c->split = keep;
     if (rc) return rc;
     HIPCHK(c, hipMemsetAsync(c->err_dev, 0, sizeof(int) * 3, c->stream));
@@ -2817,13 +2828,34 @@ int aon_hbm(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
 #include "taplanes.inc"
 #include "taptiny.inc"
 
+// Whether the lanes kernel is the faster loading of n variants, where the
+// labels fit LDS.  A lanes task walks its network at ~1.1 us a node however
+// few of its lanes are used, and 1,024 tasks run at once; an LDS workgroup
+// takes ~10 ns a node (23 us at least), one variant and origin each, over
+// the CUs.  So few variants or few origins leave the lanes kernel waiting
+// on its own latency.  Measured ms a loading, lanes and per-origin: 990
+// nodes, 90 zones, 40 variants 1.06 and 0.39, 256 variants 1.43 and 2.11;
+// 2,750 nodes, 250 zones, 64 variants 3.1 and 1.8, 256 variants 5.0 and 6.5;
+// 5,390 nodes, 490 zones, 40 variants 7.1 and 3.6, 128 variants 9.4 and
+// 11.1; metro (11,000 nodes, 1,000 zones) 16 variants 14.9 and 7.0, 64
+// variants 17.1 and 27.4.  Networks with denser nodes cost the LDS kernel
+// up to 1.7 times this estimate (8,460 nodes with shortcuts, 360 zones, 64
+// variants: 8.9 and 12.7), hence the factor.
+bool lanes_pay(const tapgpu_ctx* c, int n) {
+  const double nodes = c->N, tasks = (double)c->Z * ((n + kWave - 1) / kWave);
+  const double lanes = 1.1e-6 * nodes + 0.9e-9 * nodes * tasks;
+  const double origin = (double)n * c->Z * std::max(23e-6, 10e-9 * nodes) / std::max(c->cus, 1);
+  return 1.6 * origin >= lanes;
+}
+
 // The lanes kernel loads a batch when at least lanes_min of its variants
-// are active (lanes_min 0: never).
+// are active (lanes_min 0: never) and, unless the number was asked for, it
+// is the faster one.
 bool use_lanes(tapgpu_ctx* c, int v0, int Vn, const unsigned char* h_on) {
   if (c->lanes_min <= 0 || !c->lanes_ok) return false;
   int n = 0;
   for (int v = v0; v < v0 + Vn; ++v) n += (!h_on || h_on[v]) ? 1 : 0;
-  return n >= c->lanes_min;
+  return n >= c->lanes_min && (!c->lanes_auto || !use_lds(c) || lanes_pay(c, n));
 }
 
 // Whether iterations run in the one-workgroup kernel: a network it holds, on
@@ -3074,6 +3106,7 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
     }
     int ncu = 0, per_cu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) ncu = 1;
+    c->cus = ncu;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_origin_hbm, kHbmBlock, c->hbm_lds) !=
         hipSuccess || per_cu < 1)
       per_cu = 1;
