@@ -168,3 +168,42 @@ def test_line_search_blocks(engine_mod, E):
             eng.fw_run(max_iters=20)
             res.append(([eng.flows()], [eng.trace()]))
     _same(*res)
+
+
+@pytest.mark.parametrize("M", [2, 17, 512, 513, 514, 1500])
+def test_gradient_rows_of_parallel_routes(engine_mod, M):
+    """M equal-time routes from a hub: M - 1 cycles, all through the tree's
+    route, so two links' rows have M - 1 entries (512 is the longest that
+    takes lanes, longer ones a workgroup).  Volumes of half the capacity are
+    the equilibrium in exact arithmetic.  Tolerance as for the other
+    comparisons with the dense solve; a repeat gives the same bits."""
+    from oracle import gradient as G
+    from traffic_assignment_amd import synth
+    print(f"case gradient rows M={M}", flush=True)
+    rng = np.random.default_rng(M)
+    mid = np.arange(4, 4 + M)
+    cap = 2.0 * rng.integers(5, 40, M)
+    init = np.concatenate([[1], np.full(M, 3), mid])
+    term = np.concatenate([[3], mid, np.full(M, 2)])
+    E = init.size
+    capacity = np.concatenate([[cap.sum()], cap, cap])
+    net = synth.Network(num_zones=2, num_nodes=3 + M, first_thru_node=3, init=init, term=term,
+                        capacity=capacity, length=np.ones(E), fftime=np.ones(E), B=np.full(E, 0.15),
+                        power=np.full(E, 4.0), speed=np.zeros(E), toll=np.zeros(E),
+                        ltype=np.ones(E, np.int16))
+    x = capacity / 2
+    dem = synth.Demand(2, np.array([0, 1, 1]), np.array([2]), np.array([x[0]]))
+    links = np.stack([np.zeros(M, np.int64), 1 + np.arange(M), 1 + M + np.arange(M)], 1)
+    ref = G.reference_gradient(net, x, dict(od=np.zeros(M, np.int64), flow=cap / 2,
+                                            off=3 * np.arange(M + 1), links=links.ravel()))
+    assert ref["rank"] == M - 1
+    with engine_mod.TapEngine(net, dem) as eng:
+        eng.fw_init(x)
+        g = eng.gradient(eps=1e-9, cg_tol=1e-13)
+        h = eng.gradient(eps=1e-9, cg_tol=1e-13)
+    assert g["info"]["cg_status"] == 1 and g["info"]["cycles"] == M - 1
+    for k in ("dobj_dt0", "dobj_dcap"):
+        np.testing.assert_allclose(g[k], ref[k], rtol=1e-12, atol=1e-300)
+    for k in ("dvht_dcap", "dvht_dt0"):
+        np.testing.assert_allclose(g[k], ref[k], rtol=1e-7, atol=1e-9 * np.abs(ref[k]).max())
+        assert np.array_equal(g[k].view(np.int64), h[k].view(np.int64))
