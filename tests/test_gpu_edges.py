@@ -207,3 +207,32 @@ def test_gradient_rows_of_parallel_routes(engine_mod, M):
     for k in ("dvht_dcap", "dvht_dt0"):
         np.testing.assert_allclose(g[k], ref[k], rtol=1e-7, atol=1e-9 * np.abs(ref[k]).max())
         assert np.array_equal(g[k].view(np.int64), h[k].view(np.int64))
+
+
+@pytest.mark.parametrize("N,starts,strategy", [(300, 582, "lds"), (300, 583, "lds"), (1100, 400, "hbm"),
+                                               (4097, 45, "lds"), (4097, 1060, "lds")])
+def test_shortest_paths_in_slabs(engine_mod, N, starts, strategy):
+    """Results of one copy, of several slabs placed by the caller and of
+    slabs placed by threads, with more starts than a launch takes: the
+    columns equal calls of 40 starts (one copy each), in both layouts and
+    with either array left out."""
+    import ctypes as C
+    from conftest import empty_demand
+    print(f"case slabs N={N} starts={starts} {strategy}", flush=True)
+    net, rng = small_network(N + starts, N, 20, 21, 2 * N, "cont", 30)
+    s = rng.integers(1, N + 1, starts).astype(np.int64)
+    with engine_mod.TapEngine(net, empty_demand(20)) as eng:
+        eng.set_strategy(strategy)
+        d, p = eng.sssp(s)
+        for j in range(0, starts, 40):
+            dj, pj = eng.sssp(s[j:j + 40])
+            assert np.array_equal(d[:, j:j + 40].view(np.int64), dj.view(np.int64))
+            assert np.array_equal(p[:, j:j + 40], pj)
+        L = engine_mod.lib()
+        vp = C.c_void_p
+        ld = starts + 3
+        d2, p2 = np.full((N + 1, ld), 7.0), np.full((N + 1, ld), 7, np.int64)
+        assert L.tapgpu_sssp(eng._h, 0, vp(s.ctypes.data), starts, vp(d2.ctypes.data), None, ld, 2) == 0
+        assert L.tapgpu_sssp(eng._h, 0, vp(s.ctypes.data), starts, None, vp(p2.ctypes.data), ld, 2) == 0
+    assert np.array_equal(d2[:, 2:-1], d) and np.array_equal(p2[:, 2:-1], p)
+    assert (d2[:, [0, 1, -1]] == 7).all() and (p2[:, [0, 1, -1]] == 7).all()

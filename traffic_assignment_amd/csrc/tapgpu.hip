@@ -32,7 +32,10 @@
 
 #include <hip/hip_runtime.h>
 
+#include <sched.h>
+
 #include <algorithm>
+#include <atomic>
 #include <cfloat>
 #include <climits>
 #include <chrono>
@@ -43,6 +46,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/tapgpu.h"
@@ -1943,6 +1947,8 @@ struct DevBuf {
 
 }  // namespace
 
+constexpr int kStageSlots = 8;          // slabs of results in flight to the host
+
 struct tapgpu_ctx {
   std::string err;
   hipStream_t stream = nullptr;
@@ -2040,6 +2046,13 @@ struct tapgpu_ctx {
   bool initialised = false;
   // pinned host scratch
   int* h_int = nullptr;
+  // results on their way to the caller's arrays (tapstage.inc)
+  char* stage_dev = nullptr;
+  size_t stage_dev_bytes = 0;
+  char* stage_pin = nullptr;
+  size_t stage_pin_bytes = 0;
+  hipEvent_t stage_ev[kStageSlots] = {};
+  unsigned char* aon_on = nullptr;    // [V] the variant that an all-or-nothing call loads
   // pinned readback of one FW iteration: error flag, origin-kernel
   // counters, variant states and flags (one synchronisation per iteration)
   int* pin_err = nullptr;                   // [4]
@@ -2826,6 +2839,7 @@ int aon_hbm(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
 }
 
 #include "taplanes.inc"
+#include "tapstage.inc"
 #include "taptiny.inc"
 
 // Whether the lanes kernel is the faster loading of n variants, where the
@@ -3338,6 +3352,10 @@ void tapgpu_destroy(tapgpu_ctx* c) {
   if (c->trace) (void)hipFree(c->trace);
   if (c->h_int) (void)hipHostFree(c->h_int);
   if (c->pin_block) (void)hipHostFree(c->pin_block);
+  if (c->stage_pin) (void)hipHostFree(c->stage_pin);
+  if (c->stage_dev) (void)hipFree(c->stage_dev);
+  for (auto& e : c->stage_ev)
+    if (e) (void)hipEventDestroy(e);
   for (auto& e : c->ev)
     if (e) (void)hipEventDestroy(e);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -3357,7 +3375,9 @@ int tapgpu_set_costs(tapgpu_ctx* c, int64_t variant, const double* costs) {
   if (!c || !costs) return TAPGPU_E_ARG;
   int rc = check_variant(c, variant);
   if (rc) return rc;
-  for (int k = 0; k < c->E; ++k)
+  int bad = 0;                                   // (no early exit: the loop takes vectors)
+  for (int k = 0; k < c->E; ++k) bad |= !(costs[k] >= 0.0);
+  for (int k = 0; bad && k < c->E; ++k)
     if (!(costs[k] >= 0.0))
       return c->fail(TAPGPU_E_ARG, "link %d: negative or NaN cost", k);
   if ((rc = upload(c, c->c + (size_t)variant * c->E, costs, c->E))) return rc;
@@ -3392,75 +3412,28 @@ int tapgpu_sssp(tapgpu_ctx* c, int64_t variant, const int64_t* start_nodes, int6
     const bool hbm = !use_lds(c);
     if (hbm && (rc = ensure_hbm(c))) return rc;
     const int64_t chunk = std::min<int64_t>(std::max<int64_t>(num_start, 1), 1024);
-    int* d_src = nullptr;
-    double* d_dist = nullptr;
-    int* d_pred = nullptr;
-    if ((rc = dalloc(c, &d_src, chunk))) return rc;
-    if ((rc = dalloc(c, &d_dist, (size_t)c->N * chunk))) return rc;
-    if ((rc = dalloc(c, &d_pred, (size_t)c->N * chunk))) return rc;
-    std::vector<int> hs(chunk);
-    std::vector<double> hd((size_t)c->N * chunk);
-    std::vector<int> hp((size_t)c->N * chunk);
+    SsspStage S;
+    rc = stage_sssp(c, chunk, &S);
     for (int64_t s0 = 0; !rc && s0 < num_start; s0 += chunk) {
-      const int64_t ns = std::min<int64_t>(chunk, num_start - s0);
-      for (int64_t j = 0; j < ns; ++j) hs[j] = (int)(start_nodes[s0 + j] - 1);
-      if ((rc = upload(c, d_src, hs.data(), ns))) break;
-      // a failed launch must not hand back stale links: predecessors start
-      // at -1 and the error flag at 0 for every chunk
-      if (hipMemsetAsync(d_pred, 0xFF, sizeof(int) * (size_t)c->N * chunk, c->stream) != hipSuccess ||
-          hipMemsetAsync(c->err_dev, 0, sizeof(int) * 3, c->stream) != hipSuccess) {
-        rc = c->fail(TAPGPU_E_HIP, "clearing the shortest-path outputs failed");
-        break;
-      }
+      const int ns = (int)std::min<int64_t>(chunk, num_start - s0);
+      for (int j = 0; j < ns; ++j) S.src[j] = (int)(start_nodes[s0 + j] - 1);
       OriginArgs A = make_origin_args(c, nullptr);
       advance_variant(c, A, variant);
-      A.src_list = d_src; A.out_dist = d_dist; A.out_pred = d_pred; A.ld = chunk;
+      A.src_list = S.src; A.err = S.err; A.out_dist = S.dist; A.out_pred = S.pred; A.ld = ns;
+      hipLaunchKernelGGL(k_sssp_begin, dim3(grid_for((long long)c->N * ns / kWave + 1)), dim3(kBlock), 0,
+                         c->stream, S.pred, (long long)c->N * ns, S.err);
       if (hbm)
-        hipLaunchKernelGGL(k_origin_hbm, dim3((unsigned)std::min<int64_t>(ns, c->hbm_grid)),
-                           dim3(kHbmBlock), c->hbm_lds, c->stream, A, 0, (int)ns);
+        hipLaunchKernelGGL(k_origin_hbm, dim3(std::min(ns, c->hbm_grid)), dim3(kHbmBlock), c->hbm_lds,
+                           c->stream, A, 0, ns);
       else
-        launch_lds(c, dim3((unsigned)ns, 1), c->stream, A, 0);
-      int herr[3] = {0, 0, 0};
-      const hipError_t e0 = hipGetLastError();
-      const hipError_t e1 = hipMemcpyAsync(hd.data(), d_dist, sizeof(double) * c->N * chunk,
-                                           hipMemcpyDeviceToHost, c->stream);
-      const hipError_t e2 = hipMemcpyAsync(hp.data(), d_pred, sizeof(int) * c->N * chunk,
-                                           hipMemcpyDeviceToHost, c->stream);
-      const hipError_t e4 = hipMemcpyAsync(herr, c->err_dev, sizeof herr, hipMemcpyDeviceToHost,
-                                           c->stream);
-      const hipError_t e3 = hipStreamSynchronize(c->stream);
-      if (e0 != hipSuccess || e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess ||
-          e4 != hipSuccess) {
-        const hipError_t e = e0 != hipSuccess ? e0 : e1 != hipSuccess ? e1 : e2 != hipSuccess ? e2
-                             : e4 != hipSuccess ? e4 : e3;
+        launch_lds(c, dim3(ns, 1), c->stream, A, 0);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess)
         rc = c->fail(TAPGPU_E_HIP, "shortest-path launch failed: %s", hipGetErrorString(e));
-        break;
-      }
-      if (herr[0] == 2) {
-        rc = c->fail(TAPGPU_E_LIMIT, "label-correcting rounds exceeded from origin %d (negative costs?)",
-                     herr[1] + 1);
-        break;
-      }
-      if (herr[0] == 3) {
-        rc = c->fail(TAPGPU_E_LIMIT, "predecessor cycle in the tree of origin %d", herr[1] + 1);
-        break;
-      }
-      if (herr[0] != 0) {
-        rc = c->fail(TAPGPU_E_LIMIT, "shortest-path kernel reported error %d at origin %d", herr[0],
-                     herr[1] + 1);
-        break;
-      }
-      for (int64_t v = 1; v < N1; ++v)
-        for (int64_t j = 0; j < ns; ++j) {
-          const size_t o = (size_t)v * ld + col_base + s0 + j;
-          if (dist) dist[o] = hd[(size_t)(v - 1) * chunk + j];
-          if (pred) pred[o] = hp[(size_t)(v - 1) * chunk + j];
-        }
+      else
+        rc = deliver_sssp(c, S, ns, dist, pred, ld, col_base + s0);
     }
-    for (void* q : {(void*)d_src, (void*)d_dist, (void*)d_pred}) {
-      c->allocs.erase(std::remove(c->allocs.begin(), c->allocs.end(), q), c->allocs.end());
-      (void)hipFree(q);
-    }
+    stage_trim(c);
     return rc;
   }
   // chunks of the variant's columns; groups [0, Gv) of a private mapping
@@ -3633,15 +3606,7 @@ int tapgpu_sssp_noalloc(tapgpu_ctx* c, int64_t variant, const int64_t* d_start_n
   const int* herr = c->h_int;
   if (herr[0] == 5)
     return c->fail(TAPGPU_E_ARG, "start node %d of the list is out of range", herr[1]);
-  if (herr[0] == 2)
-    return c->fail(TAPGPU_E_LIMIT, "label-correcting rounds exceeded from origin %d (negative costs?)",
-                   herr[1] + 1);
-  if (herr[0] == 3)
-    return c->fail(TAPGPU_E_LIMIT, "predecessor cycle in the tree of origin %d", herr[1] + 1);
-  if (herr[0] != 0)
-    return c->fail(TAPGPU_E_LIMIT, "shortest-path kernel reported error %d at origin %d", herr[0],
-                   herr[1] + 1);
-  return TAPGPU_OK;
+  return sssp_error(c, herr);
 }
 
 int tapgpu_aon(tapgpu_ctx* c, int64_t variant, double* volumes) {
@@ -3651,18 +3616,15 @@ int tapgpu_aon(tapgpu_ctx* c, int64_t variant, double* volumes) {
   const int v = (int)variant;
   std::vector<unsigned char> on(c->V, 0);
   on[v] = 1;
-  unsigned char* d_on = nullptr;
-  if ((rc = dalloc(c, &d_on, c->V))) return rc;
-  rc = upload(c, d_on, on.data(), c->V);
-  if (!rc) rc = load_variants(c, v, 1, d_on, on.data());
-  if (!rc && volumes) {
+  if (!c->aon_on && (rc = dalloc(c, &c->aon_on, c->V))) return rc;
+  if ((rc = upload(c, c->aon_on, on.data(), c->V))) return rc;
+  if ((rc = load_variants(c, v, 1, c->aon_on, on.data()))) return rc;
+  if (volumes) {
     const hipError_t e = hipMemcpy(volumes, c->y + (size_t)v * c->E, sizeof(double) * c->E,
                                    hipMemcpyDeviceToHost);
-    if (e != hipSuccess) rc = c->fail(TAPGPU_E_HIP, "copy of volumes failed");
+    if (e != hipSuccess) return c->fail(TAPGPU_E_HIP, "copy of volumes failed");
   }
-  c->allocs.erase(std::remove(c->allocs.begin(), c->allocs.end(), (void*)d_on), c->allocs.end());
-  (void)hipFree(d_on);
-  return rc;
+  return TAPGPU_OK;
 }
 
 static int ensure_trace(tapgpu_ctx* c, int need) {
