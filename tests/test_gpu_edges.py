@@ -236,3 +236,24 @@ def test_shortest_paths_in_slabs(engine_mod, N, starts, strategy):
         assert L.tapgpu_sssp(eng._h, 0, vp(s.ctypes.data), starts, None, vp(p2.ctypes.data), ld, 2) == 0
     assert np.array_equal(d2[:, 2:-1], d) and np.array_equal(p2[:, 2:-1], p)
     assert (d2[:, [0, 1, -1]] == 7).all() and (p2[:, [0, 1, -1]] == 7).all()
+
+
+@pytest.mark.parametrize("threads", [512, 1024])
+def test_lds_rounds_of_several_workgroups_per_cu(engine_mod, threads):
+    """Workgroups that share a CU and its LDS, 24 x 397 searches: equal
+    labels and trees every time."""
+    from conftest import network
+    print(f"case lds shared CU {threads}", flush=True)
+    net, dem = network("metro", 0.63)
+    origins = np.tile(np.arange(1, net.num_zones + 1), 4)
+    with engine_mod.TapEngine(net, dem) as eng:
+        eng.set_strategy("hbm")
+        d0, p0 = eng.sssp(origins[:net.num_zones])
+        eng.set_strategy("lds")
+        eng.set_origin_block(threads)
+        for q in (-1, 1024, 256) * 2:
+            eng.set_origin_queue(q)
+            eng.set_origin_block(threads)
+            d, p = eng.sssp(origins)
+            assert np.array_equal(d.view(np.int64), np.tile(d0.view(np.int64), 4))
+            assert np.array_equal(p, np.tile(p0, 4))

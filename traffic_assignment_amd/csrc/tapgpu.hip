@@ -494,6 +494,16 @@ constexpr int kSellWidth = 16;
 constexpr int kSellFetch = 4;        // rows of a slice loaded ahead
 constexpr unsigned kSellNone = 0xFFFF0000u;
 
+// A barrier in a loop whose LDS writes of one pass are read in the next.  The
+// wait is written out: the compiler drops its own where the writes reach the
+// barrier over the loop's back edge only, and another wavefront's read can
+// then overtake a write (seen with 512 threads: one label in 10^7 stayed
+// too high).
+__device__ __forceinline__ void loop_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
 // LDS atomicAdd by one lane.  The address is made to look divergent: for a
 // uniform one the compiler adds a wave-wide reduction around the atomic.
 __device__ __forceinline__ int lds_add(int* p, int n) {
@@ -757,7 +767,7 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
       pf = __hip_atomic_load((const unsigned*)(recb + (unsigned)pf_node * 64u), __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_WAVEFRONT);
     pf_node = -1;
-    __syncthreads();
+    loop_barrier();
     int u0 = queue0[qoff + jq], n0 = s_qn[c_now];
     asm volatile("" : "+v"(u0), "+v"(n0));              // (both read before either is used)
     qn = uniform(n0);
