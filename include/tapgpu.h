@@ -260,7 +260,7 @@ int tapgpu_set_profiling(tapgpu_ctx *ctx, int on);
    fits, else 3), 1 = node-major multi-origin sweeps (any size), 2 = one
    origin per workgroup with labels in LDS (networks whose labels fit a
    workgroup's LDS: about 13k nodes, fewer than 65535 links), 3 = one origin
-   per workgroup with labels in HBM (frontier bitmaps in LDS: up to about
+   per workgroup with labels in HBM (a node bitmap in LDS: up to about
    430k nodes).  tapgpu_get_strategy returns the one in use (1, 2 or 3). */
 int tapgpu_set_strategy(tapgpu_ctx *ctx, int strategy);
 
@@ -281,7 +281,8 @@ int tapgpu_get_origin_chase(const tapgpu_ctx *ctx);
    the LDS path, where the next loading picks it with the workgroup size
    (the most, 1024 or 256: a shorter queue takes less LDS, so more
    workgroups share a CU); 0: bitmap scans only; larger values are clamped
-   to that most.  tapgpu_get_origin_queue returns the value of the kernel in
+   to that most.  The labels-in-HBM kernel scans nothing: its queues have at
+   least 64 entries, and nodes that find no room wait for a later bucket.  tapgpu_get_origin_queue returns the value of the kernel in
    use.  Results do not depend on it. */
 int tapgpu_set_origin_queue(tapgpu_ctx *ctx, int entries);
 int tapgpu_get_origin_queue(const tapgpu_ctx *ctx);
@@ -296,9 +297,10 @@ int tapgpu_get_origin_block(const tapgpu_ctx *ctx);
 
 /* Worklist schedule of the labels-in-HBM path (strategy 3): bucket width of
    its label-ordered rounds, as a multiple of the mean free-flow link time
-   (0: no buckets, every queued node is expanded each round).  -1 (the
-   default): tuned on the first loading: each candidate (0, 1, 2, 4, 8,
-   16) runs one wave of workgroups, and the smallest busy time summed over
+   (0: none given; the width then follows the number of nodes in a bucket,
+   as it does before tuning).  -1 (the default): tuned on the first loading:
+   the candidates 1, 2, 4, 8 and 16 run one wave of workgroups each, up to
+   the first that is clearly slower, and the smallest busy time summed over
    the workgroups wins.  Results do not depend on it. */
 int tapgpu_set_origin_delta(tapgpu_ctx *ctx, double mult);
 double tapgpu_get_origin_delta(const tapgpu_ctx *ctx);

@@ -257,3 +257,30 @@ def test_lds_rounds_of_several_workgroups_per_cu(engine_mod, threads):
             d, p = eng.sssp(origins)
             assert np.array_equal(d.view(np.int64), np.tile(d0.view(np.int64), 4))
             assert np.array_equal(p, np.tile(p0, 4))
+
+
+@pytest.mark.parametrize("N,ft,hub", [(63, 1, 5), (129, 64, 16), (1000, 90, 60), (4097, 300, 700)])
+@pytest.mark.parametrize("kind", ["cont", "ints"])
+def test_hbm_kernel_queues_and_records(engine_mod, N, ft, hub, kind):
+    """Nodes with more links than a record or an in-link slice holds, queues
+    of 64 entries (they overflow) to the largest, bucket widths from one
+    bucket per label to all in one: labels, trees and loads equal the LDS
+    kernel's."""
+    print(f"case hbm edges N={N} ft={ft} hub={hub} {kind}", flush=True)
+    Z = min(max(ft - 1, 12), 40)
+    net, rng = small_network(3 * N + hub, N, Z, ft, N, kind, hub)
+    dem = random_demand(net, rng)
+    starts = rng.integers(1, N + 1, 50)
+    with engine_mod.TapEngine(net, dem) as eng:
+        eng.set_strategy("lds")
+        d0, p0 = eng.sssp(starts)
+        y0 = eng.aon()
+        eng.set_strategy("hbm")
+        for q in (0, 64, 200, -1):
+            for width in (0.0, 1e-3, 1.0, 1e6):
+                eng.set_origin_queue(q)
+                eng.set_origin_delta(width)
+                d, p = eng.sssp(starts)
+                assert np.array_equal(d.view(np.int64), d0.view(np.int64)), (q, width)
+                assert np.array_equal(p, p0), (q, width)
+                assert np.array_equal(eng.aon().view(np.int64), y0.view(np.int64)), (q, width)

@@ -521,6 +521,12 @@ struct OriginArgs {
   const double* sellw;               // [V][sell_n] sliced in-link costs
   const unsigned* sell_id;           // [sell_n] link id << 16 | tail
   const int* sell_ptr;               // [ceil(N/64) + 1] first entry of each slice
+  const struct HbmRec* hrec;         // [V][N] out-link records (labels-in-HBM kernel)
+  const uint2* hsell_id;             // [hsell_n] tail, link id
+  const double* hsellw;              // [V][hsell_n]
+  const int* hsell_ptr;
+  long long hsell_n;
+  const int *place, *node;           // its numbering: node -> place, place -> node
   long long sell_n;
   const long long* od_start;         // [Z + 1]
   const int* od_dest;                // 0-based zone
@@ -528,7 +534,7 @@ struct OriginArgs {
   const unsigned char* var_on;       // [V] or null
   int chase;                         // expansions a thread chains per round
   int qcap;                          // LDS frontier queue entries per round (0: bitmap scan only)
-  int hqcap;                         // labels-in-HBM kernel: queue entries per round (0: bitmap scan only)
+  int hqcap;                         // labels-in-HBM kernel: entries of a queue
   double delta;                      // labels-in-HBM kernel: bucket width (<= 0: none)
   int z0, zn;                        // labels-in-HBM kernel: origins [z0, z0 + zn) of each variant
   double* y;                         // [V * E], zeroed by the caller
@@ -1080,18 +1086,17 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
 // ---------------------------------------------------------------------------
 //
 // The same three phases as k_origin_lds for networks whose labels do not fit
-// LDS: only the three frontier bitmaps (3 x 8 x ceil(N/64) bytes) live in
-// LDS; labels, predecessors and flows are a per-workgroup scratch
-// row in HBM (L2 / infinity cache resident while the workgroup runs).  A
-// persistent grid loops over (origin, variant) items.  A row is private to
-// its workgroup, whose waves share one CU, so every scratch access is a
-// workgroup-scope atomic: loads skip the CU's L1 and read the XCD's L2,
-// where the atomics execute, and the barrier closing a round orders them.
-// (Device-scope accesses would have to be coherent across the XCDs' L2s and
-// cost an L2 writeback and invalidation per round.)
-// Relaxation within a round may read a label another thread is lowering;
-// the lowered node is queued for the next round, so the fixed point is the
-// same as with strict rounds.
+// LDS: only a node bitmap (8 x ceil(N/64) bytes) and the frontier
+// queues live in LDS; labels, predecessors and flows are a per-workgroup
+// scratch row in HBM (L2 / infinity cache resident while the workgroup
+// runs).  A persistent grid loops over (origin, variant) items.  A row is
+// private to its workgroup, whose waves share one CU, so every scratch
+// access is a workgroup-scope atomic: loads skip the CU's L1 and read the
+// XCD's L2, and the barrier closing a round orders them.  (Device-scope
+// accesses would have to be coherent across the XCDs' L2s and cost an L2
+// writeback and invalidation per round.)  Relaxation within a round may read
+// a label another thread is lowering; the lowered node is queued for the
+// next round, so the fixed point is the same as with strict rounds.
 
 #ifndef TAPGPU_HBM_BLOCK
 #define TAPGPU_HBM_BLOCK 512
@@ -1101,21 +1106,92 @@ constexpr int kHbmBlock = TAPGPU_HBM_BLOCK;    // 512: 2 workgroups per CU, each
 #define TAPGPU_HBM_PER_CU (1024 / TAPGPU_HBM_BLOCK)
 #endif
 constexpr int kHbmPerCu = TAPGPU_HBM_PER_CU;    // workgroups sharing a CU's LDS (registers: <= 128 VGPRs)
-constexpr int kHbmQueueMax = 4096;              // frontier queue entries per round
+constexpr int kHbmQueueMax = 4096;              // entries of a frontier queue
 
 __global__ void k_zero_i32(int* p) { *p = 0; }
 
-// LDS of the labels-in-HBM kernel: three bitmaps 3*8W | two queues of
-// (label 8 B, node 4 B) entries 2*12Q.
+// LDS of the labels-in-HBM kernel: a bitmap 8W | the table, two near queues
+// and a far queue of twice their size, of (label 8 B, node 4 B) entries; the
+// predecessors' second bitmap takes the place of these.
+constexpr int kHbmQueueMin = 64;                // entries, whatever size is asked for
+constexpr size_t kHbmQueueBytes = 48;           // per entry of the queue size
+constexpr int kHbmGroup = 2;                    // lanes per expanded node
+constexpr int kHbmCand = (5 + kHbmGroup - 1) / kHbmGroup;   // links per lane, at most
+constexpr int kHbmRedo = 64;                    // places kept for entries to be followed up again
+constexpr int kHbmSlots = 1024;                 // of the table that settles which lane lowers a label
 size_t origin_hbm_lds_bytes(int N, int hqcap) {
-  return 24ull * (size_t)((N + 63) / 64) + 24ull * (size_t)hqcap;
+  const size_t bitmap = 8ull * (size_t)((N + 63) / 64);
+  return bitmap + std::max<size_t>(bitmap, 12 * kHbmSlots + kHbmQueueBytes * (size_t)hqcap);
+}
+
+// Mirrors of the graph and of each variant's costs that the labels-in-HBM
+// kernel reads, written before each of its launches (a pass over the links:
+// 20 us on regional, against 40 ms): the LDS kernel's records and sliced
+// in-links with 32-bit nodes and links.  A record is one 64-byte line of
+// kHrecLinks links to through nodes, self-loops left out; a node with more
+// of them has none in its record and `more` set, and is read from the CSR.
+// The kernel has a numbering of its own: zones keep their numbers, through
+// nodes get places such that each 128-byte line of labels (16 nodes) holds
+// neighbours of each other (hbm_places).  A search's front is a ring; with
+// nodes numbered along rows of a city every node of it brings a line of its
+// own, which 64 workgroups an XCD cannot keep in 4 MB of L2.  Ties are
+// broken by node numbers, not places, so the trees do not depend on it.
+constexpr int kHrecLinks = 5;
+struct __align__(64) HbmRec {
+  double w[kHrecLinks];
+  int head[kHrecLinks];
+  int more;
+};
+static_assert(sizeof(HbmRec) == 64 && kHrecLinks <= kHbmCand * kHbmGroup, "an out-link record is one 64-byte line");
+
+// a thread per (variant, node), and per padding lane of the last slice
+__global__ __launch_bounds__(kBlock) void k_hbm_mirrors(OriginArgs A, int Vn, HbmRec* hrec,
+                                                        uint2* sell_id, double* sellw_all) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;       // place
+  const int N = A.N, sl = i / kWave;
+  if (sl >= (N + kWave - 1) / kWave) return;
+  const int v = i < N ? A.node[i] : -1;
+  const int begin = A.hsell_ptr[sl] + i % kWave, end = A.hsell_ptr[sl + 1];
+  for (int var = blockIdx.y; var < Vn; var += gridDim.y) {
+    const double* fw = A.fww + (size_t)var * A.E;
+    const double* rw = A.rvw + (size_t)var * A.E;
+    double* sellw = sellw_all + (size_t)var * A.hsell_n;
+    int at = begin;
+    if (v >= 0) {
+      HbmRec R;
+      int n = 0;
+#pragma unroll
+      for (int g = 0; g < kHrecLinks; ++g) { R.w[g] = INFINITY; R.head[g] = i; }
+      for (int k = A.fw_off[v]; k < A.fw_off[v + 1]; ++k) {
+        const int d = A.fw_dst[k];
+        if (d < A.ft0 || d == v) continue;
+#pragma unroll
+        for (int g = 0; g < kHrecLinks; ++g)
+          if (g == n) { R.w[g] = fw[k]; R.head[g] = A.place[d]; }
+        ++n;
+      }
+      R.more = n > kHrecLinks;
+      if (R.more)
+#pragma unroll
+        for (int g = 0; g < kHrecLinks; ++g) { R.w[g] = INFINITY; R.head[g] = i; }
+      hrec[(size_t)var * N + i] = R;
+      for (int k = A.rv_off[v]; k < A.rv_off[v + 1] && at < end; ++k) {
+        const int u = A.rv_src[k];
+        if (v < A.ft0 || u < A.ft0 || u == v) continue;
+        if (var == 0) sell_id[at] = make_uint2((unsigned)A.place[u], (unsigned)A.rv_eid[k]);
+        sellw[at] = rw[k];
+        at += kWave;
+      }
+    }
+    for (; at < end; at += kWave) {
+      if (var == 0) sell_id[at] = make_uint2((unsigned)min(i, N - 1), 0u);
+      sellw[at] = INFINITY;
+    }
+  }
 }
 
 // workgroup-scope loads of a workgroup's private scratch row
 __device__ __forceinline__ unsigned long long ldg_u64(const unsigned long long* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ unsigned ldg_u32(const unsigned* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 __device__ __forceinline__ int ldg_i32(const int* p) {
@@ -1124,22 +1200,26 @@ __device__ __forceinline__ int ldg_i32(const int* p) {
 
 __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void k_origin_hbm(OriginArgs A, int load, int items) {
   extern __shared__ unsigned long long sm[];
-  const int N = A.N;
+  constexpr int kWaves = kHbmBlock / kWave;
+  const int N = A.N, ft0 = A.ft0, qcap = A.hqcap;
   const int W = (N + 63) >> 6;
   unsigned long long* bmA = sm;
-  unsigned long long* bmB = bmA + W;
-  unsigned long long* bmC = bmB + W;
-  unsigned long long* qlab0 = bmC + W;                  // 2 x [hqcap] labels when listed
-  unsigned long long* qlab1 = qlab0 + A.hqcap;
-  unsigned* qnode0 = (unsigned*)(qlab1 + A.hqcap);      // 2 x [hqcap] nodes
-  unsigned* qnode1 = qnode0 + A.hqcap;
+  unsigned long long* bmB = bmA;                        // (the predecessors' use of the two bitmaps)
+  unsigned long long* bmC = bmA + W;
+  const int fcap = 2 * qcap;
+  unsigned long long* tab_lab = bmA + W;                // [kHbmSlots] smallest label offered
+  unsigned long long* far_lab = tab_lab + kHbmSlots;    // [fcap] labels when listed
+  unsigned long long* near_lab = far_lab + fcap;        // 2 x [qcap]
+  unsigned* far_node = (unsigned*)(near_lab + 2 * (size_t)qcap);
+  unsigned* near_node = far_node + fcap;
+  unsigned* tab_node = near_node + 2 * (size_t)qcap;    // [kHbmSlots] node + 1, 0: free
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-  __shared__ int s_qn[3], s_exp[3];
-  __shared__ unsigned long long s_minq[3];
+  __shared__ int s_near[3], s_redo[3], s_far[2], s_over[2], s_lost;
+  __shared__ unsigned long long s_min[2];
   __shared__ unsigned long long s_cnt[8];
   __shared__ int s_maxlen;
   __shared__ int s_level_ties, s_left, s_added;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, wave = uniform(tid / kWave);
   const unsigned long long kMax = as_b(DBL_MAX);
   unsigned long long* dist = A.h_dist + (size_t)blockIdx.x * N;
   int* pred = A.h_pred + (size_t)blockIdx.x * N;
@@ -1147,8 +1227,8 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
   double* flow = (double*)dist;
   if (tid < 8) s_cnt[tid] = 0;
   if (tid == 0) s_maxlen = 0;
-  unsigned long long n_exp = 0, n_scan = 0, n_upd = 0, n_rounds = 0, n_steps = 0, n_loaded = 0;
-  unsigned long long n_def = 0;
+  unsigned n_exp = 0, n_scan = 0, n_upd = 0, n_steps = 0, n_loaded = 0, n_def = 0;   // (a lane's share)
+  unsigned long long n_rounds = 0;
   unsigned long long c_relax = 0, c_pred = 0, c_load = 0;
 
   __shared__ int s_item;
@@ -1157,234 +1237,456 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
     // takes it), or block-strided
     if (tid == 0) s_item = A.next ? atomicAdd(A.next, 1) : (int)blockIdx.x + k * (int)gridDim.x;
     __syncthreads();
-    const int item = s_item;
+    const int item = uniform(s_item);
     __syncthreads();
     if (item >= items) break;
-    int var, src;
+    int var, origin;
     if (A.src_list) {
       var = 0;
-      src = A.src_list[item];
+      origin = A.src_list[item];
     } else if (A.order) {                     // longest origins first, all variants of each
       const int rank = item / A.vn;
       var = item - rank * A.vn;
-      src = A.order[rank];
+      origin = A.order[rank];
     } else {
       var = item / A.zn;
-      src = A.z0 + item - var * A.zn;
+      origin = A.z0 + item - var * A.zn;
     }
     if (A.var_on && !A.var_on[var]) continue;
+    const int src = A.place[origin];          // (nodes below are places, unless they come from the CSR)
     const double* __restrict__ fw = A.fww + (size_t)var * A.E;
     const double* __restrict__ rw = A.rvw + (size_t)var * A.E;
+    const char* recb = (const char*)(A.hrec + (size_t)var * N);
+    const double* __restrict__ sellw = A.hsellw + (size_t)var * A.hsell_n;
     const long long clk0 = wall_clock64();
+    // ---- label-correcting rounds in buckets.  Round r expands the near
+    //      nodes: those lowered below T in round r-1, listed in an LDS queue
+    //      with their label.  A node lowered to T or above goes to the far
+    //      queue.  A round that leaves nothing near moves T to the smallest
+    //      far label plus the bucket width and the far entries below it over.
+    //      The width is delta; where none is set (delta < 0) it doubles when
+    //      a bucket has fewer nodes than half a pass and halves when one has
+    //      more than two passes.
+    //      Labels are lowered with plain stores: an atomic at L2 is forwarded
+    //      to memory (it must be seen by the other XCDs) and takes the line
+    //      out of this one's L2, which made 0.57 G memory atomics and as many
+    //      misses a loading of regional.  Two lanes that lower a label in the
+    //      same round may leave the larger value, so every store is followed
+    //      up: its queue entry (v, lab) is compared with v's label when it is
+    //      taken out, in a later round.  Equal: v is expanded (once a round:
+    //      `taken` flags).  The label is smaller: another entry stands for
+    //      it.  Larger: it is stored again, with a new entry.  An entry is
+    //      thus dropped only where the label at most equals its own, and a
+    //      round never leaves a label above what it was at its start, so the
+    //      labels that are left are the least.  Most such races are settled
+    //      before the store, in a table of labels offered in the round: only
+    //      the smallest offered to a node goes on (a node that finds no slot
+    //      goes on anyway).  Without it the larger value wins half of the
+    //      races and is expanded: 2.6 times the rounds on regional.
+    //      Nodes that find the near queue full go to the far one; no store
+    //      without an entry: where that is full too, the link's tail is
+    //      flagged (in pred's row, which is free until the predecessors
+    //      are chosen) and expanded again when T moves.  Entries to be
+    //      followed up once more grow from the end of the near queue, where
+    //      kHbmRedo places are kept for them; should a round have more, the
+    //      search starts again, `safe`: with as many places kept as the
+    //      round has entries.
+    //      A round is a chain of trips to the XCD's L2 and beyond, so what
+    //      counts is their number and the lines they touch: kHbmGroup lanes
+    //      share an expanded node, whose links are one line that is read
+    //      beside its label; the labels of the heads are next.  Links to
+    //      zones are left out (their labels are pulled at the end), and
+    //      keeping a node for a later bucket costs nothing in the rounds
+    //      between.  Measured on regional (4,000 origins, 94,000 nodes, 500
+    //      rounds an origin): 3.1 ms an origin and workgroup for the labels,
+    //      0.9 for the predecessors, 0.5 for the loading, 38 ms a loading;
+    //      with one lane a node, CSR reads, an L2 atomic a lowered label and
+    //      queued nodes looked at in every round 6.0, 1.2 and 0.8, 66 ms. ----
+    const bool adapt = A.delta < 0.0;
+    double width = fabs(A.delta);
+    unsigned long long T = 0;
+    int r = 1, fb = 0, lim = qcap;             // lim: places of the near queue for lowered nodes
+    constexpr int kPass = kHbmBlock / kHbmGroup;     // nodes taken at once
+    const int g = lane & (kHbmGroup - 1), grp = lane / kHbmGroup;
+    // this lane's place among the lanes with `want`, counted on *n
+    auto place = [&](bool want, int* n) {
+      const unsigned long long bal = __ballot(want);
+      int b0 = 0;
+      if (bal) {
+        const int leader = __ffsll((long long)bal) - 1;
+        if (lane == leader) b0 = lds_add(n, __popcll(bal));
+        b0 = __builtin_amdgcn_readlane(b0, leader);
+      }
+      return b0 + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
+                                                 __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
+    };
+    auto put = [&](unsigned long long* lab, unsigned* node, int at, unsigned long long l, int v) {
+      lab[at] = l;
+      node[at] = (unsigned)v;
+    };
+    auto set_label = [&](int v, unsigned long long lab) {
+      __hip_atomic_store(&dist[v], lab, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    // offers v the label cb; the slot it went to, -1: none of its two
+    auto offer_label = [&](int v, unsigned long long cb) {
+      const unsigned h = ((unsigned)v * 0x9E3779B1u) >> 22;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int s = (int)(h ^ k);
+        const unsigned old = atomicCAS(&tab_node[s], 0u, (unsigned)v + 1u);
+        if (old == 0u || old == (unsigned)v + 1u) {
+          atomicMin(&tab_lab[s], cb);
+          return s;
+        }
+      }
+      return -1;
+    };
+    // u -> v[i] gives v[i] the label cb[i] where low[i]: lowers and lists
+    // them, one LDS atomic for both queues and all of the wavefront's
+    auto relax = [&](auto& v, auto& cb, auto& low, int u, int room) {
+      constexpr int K = sizeof(low) / sizeof(low[0]);
+      unsigned long long bn[K], bf[K];
+      int nn = 0, nf = 0;
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        bn[i] = __ballot(low[i] && cb[i] < T);
+        bf[i] = __ballot(low[i] && cb[i] >= T);
+        nn += __popcll(bn[i]);
+        nf += __popcll(bf[i]);
+      }
+      if (!(nn + nf)) return;
+      int base = 0;
+      if (lane < 2) base = lds_add(lane ? &s_far[fb] : &s_near[r % 3], lane ? nf : nn);
+      int pn = __builtin_amdgcn_readlane(base, 0), pf = __builtin_amdgcn_readlane(base, 1);
+      auto rank = [&](unsigned long long m) {
+        return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+      };
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        const bool near = low[i] && cb[i] < T && pn + rank(bn[i]) < room;
+        int at = pf + rank(bf[i]);
+        if (pn + __popcll(bn[i]) > room) {             // the rest of the near ones to the far queue
+          const bool rest = low[i] && cb[i] < T && !near;
+          const int k = place(rest, &s_far[fb]);
+          if (rest) at = k;
+        }
+        if (near) {
+          put(near_lab, near_node, (r & 1) * qcap + pn + rank(bn[i]), cb[i], v[i]);
+        } else if (low[i] && at < fcap) {
+          put(far_lab, far_node, at, cb[i], v[i]);
+          ++n_def;
+        } else if (low[i]) {
+          __hip_atomic_store(&pred[u], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          s_over[fb] = 1;
+          low[i] = false;
+        }
+        if (low[i]) {
+          set_label(v[i], cb[i]);
+          ++n_upd;
+        }
+        pn += __popcll(bn[i]);
+        pf += __popcll(bf[i]);
+      }
+    };
+    for (bool safe = false;; safe = true) {
+#pragma unroll 4
     for (int v = tid; v < N; v += kHbmBlock) {
       __hip_atomic_store(&dist[v], kMax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_store(&pred[v], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    for (int w = tid; w < 3 * W; w += kHbmBlock) bmA[w] = 0;
-    if (tid < 3) { s_qn[tid] = tid == 0 ? 1 : 0; s_exp[tid] = 0; s_minq[tid] = ~0ull; }
+    for (int w = tid; w < W; w += kHbmBlock) bmA[w] = 0;
+    if (tid < 3) { s_near[tid] = tid == 0 ? 1 : 0; s_redo[tid] = 0; }
+    if (tid < 2) { s_far[tid] = 0; s_over[tid] = 0; s_min[tid] = ~0ull; }
+    if (tid == 0) s_lost = 0;
     __syncthreads();
     if (tid == 0) {
       __hip_atomic_store(&dist[src], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      bmA[src >> 6] = 1ull << (src & 63);
-      if (A.hqcap > 0) { qnode0[0] = (unsigned)src; qlab0[0] = 0ull; }
+      near_node[0] = (unsigned)src;
+      near_lab[0] = 0ull;
     }
     __syncthreads();
-
-    // ---- label-correcting rounds, bucketed: a round expands the queued
-    //      nodes whose label is below T and keeps the others queued; a
-    //      round that expands nothing moves T to the smallest queued label
-    //      plus delta (delta <= 0: no buckets, every queued node expands).
-    //      The nodes queued for round r (lowered or kept in round r-1) are
-    //      listed in an LDS queue with their label when listed (count
-    //      s_qn[(r-1)%3], buffer (r-1)&1), one node per thread, so keeping a
-    //      node needs no HBM read; the label only decides the bucket (the
-    //      current label, never higher, is read to expand).  When more were
-    //      queued than the queue holds, the round scans their bitmap `cur`
-    //      instead.  A node is listed once per round: the lane whose
-    //      atomicOr sets its bit in `nxt` appends it, one LDS atomicAdd per
-    //      wave for all of the wave's appends. ----
-    unsigned long long *cur = bmA, *nxt = bmB, *clr = bmC;
-    const bool buckets = A.delta > 0.0;
-    double T = buckets ? A.delta : INFINITY;
-    int r = 1;
-    // sets v's bit in nxt; the lane that set it appends (v, lab)
-    auto list = [&](bool want, int v, unsigned long long lab) {
-      bool first = false;
-      if (want) {
-        const unsigned long long bit = 1ull << (v & 63);
-        first = !(atomicOr(&nxt[v >> 6], bit) & bit);
-      }
-      const unsigned long long bal = __ballot(first);
-      if (bal) {
-        const int leader = __ffsll((long long)bal) - 1;
-        int b0 = 0;
-        if (lane == leader) b0 = atomicAdd(&s_qn[r % 3], __popcll(bal));
-        b0 = __builtin_amdgcn_readlane(b0, leader);
-        if (first) {
-          const int pos = b0 + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
-                                                              __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
-          if (pos < A.hqcap) {
-            ((r & 1) ? qlab1 : qlab0)[pos] = lab;
-            ((r & 1) ? qnode1 : qnode0)[pos] = (unsigned)v;
+    T = as_b(width);
+    r = 1; fb = 0; lim = qcap;
+    for (;;) {
+      const int n1 = min(uniform(s_near[(r - 1) % 3]), lim);
+      const int qn = n1 + min(uniform(s_redo[(r - 1) % 3]), qcap - lim);
+      const int from = ((r - 1) & 1) * qcap, to = (r & 1) * qcap;
+      const int room = qcap - (safe ? qn : min(qn, kHbmRedo));
+      for (int s = tid; s < kHbmSlots; s += kHbmBlock) { tab_node[s] = 0u; tab_lab[s] = ~0ull; }
+      for (int j0 = 0; j0 < qn; j0 += kPass) {
+        // ---- the lanes of a group take an entry (all lanes come here) ----
+        const int j = j0 + wave * (kWave / kHbmGroup) + grp;
+        const bool on = j < qn;
+        const int at = from + (j < n1 ? j : qcap - 1 - (j - n1));
+        const int u = on ? (int)near_node[at] : src;
+        const unsigned long long lab = on ? near_lab[at] : kMax;
+        const unsigned ro = (unsigned)u * 64u;
+        // (no load is masked: a merge with a default waits for each of them)
+        double w[kHbmCand];
+        int v[kHbmCand];
+        const unsigned long long have = ldg_u64(&dist[u]);
+        int more = *(const int*)(recb + (ro + 12u * kHrecLinks));
+#pragma unroll
+        for (int i = 0; i < kHbmCand; ++i) {
+          const unsigned k = min((unsigned)(g + i * kHbmGroup), (unsigned)(kHrecLinks - 1));
+          w[i] = *(const double*)(recb + (ro + k * 8u));
+          v[i] = *(const int*)(recb + (ro + 8u * kHrecLinks + k * 4u));
+        }
+        if (j0 == 0) __syncthreads();                  // (the table is clear; the loads are on their way)
+        const bool lost = on && g == 0 && have > lab;
+        if (__builtin_expect(__ballot(lost) != 0, 0)) {
+          const int k = place(lost, &s_redo[r % 3]);
+          if (lost && k < qcap - room) {
+            set_label(u, lab);
+            put(near_lab, near_node, to + qcap - 1 - k, lab, u);
+          } else if (lost) {
+            s_lost = 1;
+          }
+        }
+        bool first = on && g == 0 && have == lab;
+        const unsigned long long bit = 1ull << (u & 63);
+        if (first) first = !(atomicOr(&bmA[u >> 6], bit) & bit);
+        const bool go = (__ballot(first) >> (lane & ~(kHbmGroup - 1))) & 1ull;
+        n_exp += first;
+        unsigned long long cb[kHbmCand], hv[kHbmCand];
+        bool low[kHbmCand];
+        int slot[kHbmCand];
+#pragma unroll
+        for (int i = 0; i < kHbmCand; ++i) {
+          cb[i] = as_b(as_d(lab) + w[i]);
+          hv[i] = ldg_u64(&dist[v[i]]);
+        }
+#pragma unroll
+        for (int i = 0; i < kHbmCand; ++i) {
+          const bool in = go && cb[i] < kMax && g + i * kHbmGroup < kHrecLinks;
+          n_scan += in;
+          low[i] = in && cb[i] < hv[i];
+          slot[i] = -1;
+          if (low[i]) slot[i] = offer_label(v[i], cb[i]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kHbmCand; ++i)
+          if (slot[i] >= 0) low[i] = tab_lab[slot[i]] == cb[i];   // else a smaller one is stored
+        relax(v, cb, low, u, room);
+        if (!go) more = 0;
+        if (__ballot(more)) {                          // more links than the record holds
+          const int nu = A.node[u], ee = more ? A.fw_off[nu + 1] : 0;
+          for (int e = (more ? A.fw_off[nu] : 0) + g; __ballot(e < ee); e += kHbmGroup) {
+            int x[1] = {u};
+            double we = INFINITY;
+            if (e < ee) { x[0] = A.place[A.fw_dst[e]]; we = fw[e]; }
+            unsigned long long c[1] = {as_b(as_d(lab) + we)};
+            const bool ok = e < ee && x[0] >= ft0 && c[0] < kMax;
+            n_scan += ok;
+            bool lo[1] = {c[0] < (ok ? ldg_u64(&dist[x[0]]) : 0ull)};
+            relax(x, c, lo, u, room);
           }
         }
       }
-    };
-    // u (listed with label lab) either stays queued (lab >= T) or expands;
-    // the smallest label kept queued by this lane in the round is min_kept
-    unsigned long long min_kept = ~0ull;
-    auto visit = [&](int u, unsigned long long lab) {
-      const int sl = r % 3;
-      if (!(as_d(lab) < T)) lab = ldg_u64(&dist[u]);   // the listed label may be stale
-      if (!(as_d(lab) < T)) {                 // later bucket: stays queued
-        min_kept = min(min_kept, lab);
-        ++n_def;
-        list(true, u, lab);
-        return;
-      }
-      s_exp[sl] = 1;
-      const double du = as_d(ldg_u64(&dist[u]));
-      const int eb = A.fw_off[u], ee = A.fw_off[u + 1];
-      ++n_exp;
-      n_scan += (unsigned long long)(ee - eb);
-      for (int e0 = eb; e0 < ee; e0 += 8) {
-        int hv[8];
-        double hw[8];
-        unsigned long long hd[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (e0 + k < ee) { hv[k] = A.fw_dst[e0 + k]; hw[k] = fw[e0 + k]; }
-        // the heads' labels are read first: most links lower nothing, and an
-        // L2 atomic costs more than a read
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (e0 + k < ee) hd[k] = ldg_u64(&dist[hv[k]]);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          if (e0 + k >= ee) break;
-          const int v = hv[k];
-          const unsigned long long cb = as_b(du + hw[k]);
-          bool low = false;
-          if (cb < hd[k]) {
-            // no wait for the old value: a head whose label this lowers is
-            // listed (a node listed twice is deduplicated by the bitmap, and
-            // its key -- cb, at or above the label -- is re-read before a
-            // bucket decision), so the atomic need not return
-            (void)__hip_atomic_fetch_min(&dist[v], cb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            ++n_upd;
-            low = v >= A.ft0;
-          }
-          list(low, v, cb);
-        }
-      }
-    };
-    for (;; ++r) {
-      const int sl = r % 3;
-      const int qn = s_qn[(r - 1) % 3];
-      if (qn <= A.hqcap) {
-        const unsigned* qn_r = (r & 1) ? qnode0 : qnode1;
-        const unsigned long long* ql_r = (r & 1) ? qlab0 : qlab1;
-        for (int i = tid; i < qn; i += kHbmBlock) visit((int)qn_r[i], ql_r[i]);
-      } else {
-        for (int slot = tid; slot < 4 * W; slot += kHbmBlock) {
-          const int w = slot >> 2, q = slot & 3;
-          unsigned bits = (unsigned)((cur[w] >> (16 * q)) & 0xFFFFull);
-          while (bits) {
-            const int b = __ffs(bits) - 1;
-            bits &= bits - 1;
-            const int u = (w << 6) + 16 * q + b;
-            visit(u, ldg_u64(&dist[u]));
-          }
-        }
-      }
-      // one LDS atomic per wavefront for the round's smallest kept label
-      for (int o = kWave / 2; o > 0; o >>= 1) min_kept = min(min_kept, __shfl_xor(min_kept, o));
-      if (lane == 0 && min_kept != ~0ull) atomicMin(&s_minq[sl], min_kept);
-      min_kept = ~0ull;
-      for (int w = tid; w < W; w += kHbmBlock) clr[w] = 0;
-      if (tid == 0) {
-        const int sn = (r + 1) % 3;
-        s_qn[sn] = 0;
-        s_exp[sn] = 0;
-        s_minq[sn] = ~0ull;
-      }
+      // (every entry is taken: the last pass's barrier)
+      for (int j = tid; j < qn; j += kHbmBlock) bmA[near_node[from + (j < n1 ? j : qcap - 1 - (j - n1))] >> 6] = 0ull;
+      if (tid == 0) { s_near[(r + 1) % 3] = 0; s_redo[(r + 1) % 3] = 0; }
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // (the round's stores are done)
       __syncthreads();
-      if (!s_qn[sl]) break;
-      if (buckets && !s_exp[sl]) T = as_d(s_minq[sl]) + A.delta;
-      if (r > 64 * N + 64) {
-        if (tid == 0 && atomicCAS(&A.err[0], 0, 2) == 0) { A.err[1] = src; A.err[2] = 0; }
-        break;
-      }
-      unsigned long long* t = cur; cur = nxt; nxt = clr; clr = t;
-    }
-    n_rounds += (unsigned long long)r;
-    if (A.work && tid == 0 && var == 0) A.work[src] = r;
-    const long long clk1 = wall_clock64();
-
-    // ---- predecessor links: smallest tail label below the node's, then
-    //      tail id; nodes with none join by attach_level_ties.  Tails,
-    //      costs and link ids of up to 4 in-links are loaded together, then
-    //      the tails' labels. ----
-    for (int w = tid; w < W; w += kHbmBlock) bmB[w] = 0;     // nodes left for attach_level_ties
-    if (tid == 0) s_level_ties = 0;
-    __syncthreads();
-    for (int v = tid; v < N; v += kHbmBlock) {
-      int p = -1, pt = -1;
-      const unsigned long long dv = ldg_u64(&dist[v]);
-      if (v != src && dv != kMax) {
-        unsigned long long best_du = dv;      // only tails with a smaller label can win
-        const int kb = A.rv_off[v], ke = A.rv_off[v + 1];
-        for (int k0 = kb; k0 < ke; k0 += 4) {
-          int hu[4], he[4];
-          double hw[4];
-          unsigned long long hd[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (k0 + i < ke) { hu[i] = A.rv_src[k0 + i]; hw[i] = rw[k0 + i]; he[i] = A.rv_eid[k0 + i]; }
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (k0 + i < ke) hd[i] = ldg_u64(&dist[hu[i]]);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if (k0 + i >= ke) break;
-            const int u = hu[i];
-            if (u == v || (u < A.ft0 && u != src)) continue;
-            const unsigned long long du = hd[i];
-            if (du == kMax) continue;
-            if (as_b(as_d(du) + hw[i]) != dv) continue;
-            bool take = du < best_du;
-            if (!take && du == best_du && pt >= 0) take = u < pt;
-            if (take) {
-              best_du = du;
-              p = he[i];
-              pt = u;
+      lim = room;
+      bool done = false;
+      while (!(min(uniform(s_near[r % 3]), lim) + uniform(s_redo[r % 3]))) {   // T moves
+        const int fn = uniform(s_far[fb]), fc = min(fn, fcap);
+        const bool over = uniform(s_over[fb]) != 0;
+        done = fn == 0 && !over;
+        if (done) break;
+        unsigned long long m = ~0ull;
+        for (int i = tid; i < fc; i += kHbmBlock) m = min(m, far_lab[i]);
+        for (int o = kWave / 2; o > 0; o >>= 1) m = min(m, __shfl_xor(m, o));
+        if (lane == 0 && m != ~0ull) atomicMin(&s_min[fb], m);
+        if (tid == 0) { s_far[fb ^ 1] = 0; s_over[fb ^ 1] = 0; s_near[r % 3] = 0; }
+        __syncthreads();
+        // 7/8 of the near queue at most, so that the entries find room for what
+        // they lower; far entries first, so that the far queue empties
+        const int fill = qcap - qcap / 8;
+        lim = fill;
+        const unsigned long long mn = s_min[fb];
+        // (above the smallest label also where delta is below its last bit)
+        if (mn != ~0ull) T = max(T, max(as_b(as_d(mn) + width), mn + 1));
+        if (tid == 0) s_min[fb ^ 1] = ~0ull;
+        for (int i0 = 0; i0 < fc; i0 += kHbmBlock) {   // (what stays closes up in place)
+          const int i = i0 + tid;
+          const bool on = i < fc;
+          const unsigned long long lab = on ? far_lab[i] : 0ull;
+          const int v = on ? (int)far_node[i] : src;
+          __syncthreads();
+          const bool near = on && lab < T;
+          const int pn = place(near, &s_near[r % 3]);
+          const bool keep = on && !(near && pn < fill);
+          if (near && pn < fill) put(near_lab, near_node, to + pn, lab, v);
+          const int pf = place(keep, &s_far[fb ^ 1]);
+          if (keep) put(far_lab, far_node, pf, lab, v);
+        }
+        if (over) {
+          __syncthreads();
+          for (int u0 = wave * kWave; u0 < N; u0 += kHbmBlock) {
+            const int u = u0 + lane;
+            const bool on = u < N && ldg_i32(&pred[min(u, N - 1)]) != 0;
+            const int pn = place(on, &s_near[r % 3]);
+            if (on && pn < fill) {
+              __hip_atomic_store(&pred[u], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              put(near_lab, near_node, to + pn, ldg_u64(&dist[u]), u);
+            } else if (on) {
+              s_over[fb ^ 1] = 1;
             }
           }
         }
+        fb ^= 1;
+        __syncthreads();
+        if (adapt) {
+          const int moved = uniform(s_near[r % 3]);
+          if (moved > 2 * kPass)
+            width *= 0.5;
+          else if (moved < kPass / 2)
+            width *= 2.0;
+        }
       }
+      if (done) break;
+      if (r > 64 * N + 64) {
+        if (tid == 0 && atomicCAS(&A.err[0], 0, 2) == 0) { A.err[1] = origin; A.err[2] = 0; }
+        break;
+      }
+      ++r;
+    }
+    if (safe || !uniform(s_lost)) break;
+    __syncthreads();
+    }
+    n_rounds += (unsigned long long)r;
+    if (A.work && tid == 0 && var == 0) A.work[origin] = r;
+    const long long clk1 = wall_clock64();
+
+    // ---- predecessor links: smallest tail label below the node's, then
+    //      tail id; nodes with none join by attach_level_ties.  Through
+    //      nodes by slices of 64, whose in-links are contiguous row by row;
+    //      the next slice's rows are on their way while a slice's tails are
+    //      looked up.  The links of an origin that is a zone are in no slice
+    //      and come first (label 0 and the smallest id: they win where they
+    //      are tight).  Then the zones, whose labels are the minimum over
+    //      their in-links. ----
+    for (int w = tid; w < 2 * W; w += kHbmBlock) bmB[w] = 0;   // level ties | chosen
+    if (tid == 0) s_level_ties = 0;
+    __syncthreads();
+    auto choose = [&](int v, int p, int pt, unsigned long long dv) {
       __hip_atomic_store(&pred[v], p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       __hip_atomic_store(&ptail[v], pt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       // reached, not the origin, and no tight tail with a smaller label
       const bool level_tie = p < 0 && v != src && dv != kMax;
-      if (level_tie) {
-        atomicOr(&bmB[v >> 6], 1ull << (v & 63));
+      if (level_tie) {                                 // (by node)
+        const int n = A.node[v];
+        atomicOr(&bmB[n >> 6], 1ull << (n & 63));
         s_level_ties = 1;
       }
       if (A.out_dist) {
-        const size_t o = (size_t)v * A.ld + item;
+        const size_t o = (size_t)A.node[v] * A.ld + item;
         A.out_dist[o] = as_d(dv);
         if (!level_tie) A.out_pred[o] = p;
       }
+    };
+    if (src < ft0)
+      for (int e = A.fw_off[src] + tid; e < A.fw_off[src + 1]; e += kHbmBlock) {
+        const int v = A.place[A.fw_dst[e]];
+        const unsigned long long wb = as_b(0.0 + fw[e]);
+        if (v < ft0 || wb == 0ull || wb >= kMax || ldg_u64(&dist[v]) != wb) continue;
+        bool first = true;                             // of equal parallel links
+        for (int k = A.fw_off[src]; k < e; ++k) first = first && !(A.fw_dst[k] == A.fw_dst[e] && fw[k] == fw[e]);
+        if (!first) continue;
+        choose(v, e, src, wb);
+        atomicOr(&bmC[v >> 6], 1ull << (v & 63));      // chosen
+      }
+    __syncthreads();
+    {
+      constexpr int kFetch = 5;                        // rows of a slice loaded ahead
+      struct Rows { uint2 id[kFetch]; double w[kFetch]; unsigned long long dv; int at, rows; };
+      auto fetch = [&](int sl, Rows& R) {
+        const int p0 = A.hsell_ptr[sl];
+        R.at = p0 + lane;
+        R.rows = (A.hsell_ptr[sl + 1] - p0) / kWave;
+#pragma unroll
+        for (int i = 0; i < kFetch; ++i)
+          if (i < R.rows) { R.id[i] = A.hsell_id[R.at + i * kWave]; R.w[i] = sellw[R.at + i * kWave]; }
+        const int v = sl * kWave + lane;
+        R.dv = v < N && v >= ft0 ? ldg_u64(&dist[v]) : kMax;
+      };
+      auto select = [&](int sl, const Rows& R) {
+        const int v = sl * kWave + lane;
+        const unsigned long long dv = R.dv;
+        unsigned long long best_du = dv, du[kFetch];   // only tails with a smaller label can win
+        int p = -1, pt = INT_MAX;
+        auto offer = [&](int u, int e, double w, unsigned long long d) {
+          const bool tight = as_b(as_d(d) + w) == dv;
+          if (tight && (d < best_du || (d == best_du && p >= 0 && A.node[u] < A.node[pt]))) {
+            best_du = d; p = e; pt = u;
+          }
+        };
+#pragma unroll
+        for (int i = 0; i < kFetch; ++i)
+          if (i < R.rows) du[i] = ldg_u64(&dist[R.id[i].x]);
+#pragma unroll
+        for (int i = 0; i < kFetch; ++i)
+          if (i < R.rows) offer((int)R.id[i].x, (int)R.id[i].y, R.w[i], du[i]);
+        for (int i = kFetch; i < R.rows; ++i) {
+          const uint2 id = A.hsell_id[R.at + i * kWave];
+          offer((int)id.x, (int)id.y, sellw[R.at + i * kWave], ldg_u64(&dist[id.x]));
+        }
+        if (v >= N || v < ft0) return;
+        if (R.rows == kSellWidth)
+          for (int n = A.node[v], e = A.rv_off[n]; e < A.rv_off[n + 1]; ++e) {
+            const int u = A.place[A.rv_src[e]];
+            if (u >= ft0 && u != v) offer(u, A.rv_eid[e], rw[e], ldg_u64(&dist[u]));
+          }
+        if ((bmC[sl] >> lane) & 1ull) return;          // chosen
+        if (dv == kMax || v == src) p = -1;
+        choose(v, p, p < 0 ? -1 : pt, dv);
+      };
+      for (int sl = ft0 / kWave + wave; sl < W; sl += kWaves) {
+        Rows R;
+        fetch(sl, R);
+        select(sl, R);
+      }
+    }
+    for (int v = tid; v < ft0 && v < N; v += kHbmBlock) {
+      int p = -1, pt = -1;
+      unsigned long long dk = v == src ? 0ull : kMax;
+      if (v != src) {
+        auto tails = [&](auto&& f) {                   // f(tail, link, its label, label through it)
+          for (int e = A.rv_off[v]; e < A.rv_off[v + 1]; ++e) {
+            const int u = A.place[A.rv_src[e]];
+            if (u == v || (u < ft0 && u != src)) continue;
+            const unsigned long long du = u == src ? 0ull : ldg_u64(&dist[u]);
+            if (du != kMax) f(u, A.rv_eid[e], du, as_b(as_d(du) + rw[e]));
+          }
+        };
+        tails([&](int, int, unsigned long long, unsigned long long c) { dk = min(dk, c); });
+        unsigned long long best_du = dk;
+        if (dk != kMax)
+          tails([&](int u, int e, unsigned long long du, unsigned long long c) {
+            if (c == dk && (du < best_du || (du == best_du && p >= 0 && A.node[u] < A.node[pt]))) {
+              best_du = du;
+              p = e;
+              pt = u;
+            }
+          });
+        __hip_atomic_store(&dist[v], dk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      choose(v, p, pt, dk);
     }
     __syncthreads();
     if (s_level_ties) {
       const bool ok = attach_level_ties<kHbmBlock>(
-          A, rw, src, bmB, bmC, &s_left, &s_added, [&](int v) { return ldg_u64(&dist[v]); },
-          [&](int v, int e, int u) {
-            __hip_atomic_store(&pred[v], e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_store(&ptail[v], u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          A, rw, origin, bmB, bmC, &s_left, &s_added, [&](int v) { return ldg_u64(&dist[A.place[v]]); },
+          [&](int v, int e, int u) {                   // (v and u are nodes here)
+            const int i = A.place[v];
+            __hip_atomic_store(&pred[i], e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_store(&ptail[i], A.place[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             if (A.out_dist) A.out_pred[(size_t)v * A.ld + item] = e;
           });
-      if (!ok && tid == 0 && atomicCAS(&A.err[0], 0, 3) == 0) { A.err[1] = src; A.err[2] = 0; }
+      if (!ok && tid == 0 && atomicCAS(&A.err[0], 0, 3) == 0) { A.err[1] = origin; A.err[2] = 0; }
       __syncthreads();
     }
     // every label read is done: the row now holds flows
@@ -1394,50 +1696,59 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
     if (!load) continue;
 
     // ---- loading: destination walks, then tree links with flow ----
+#pragma unroll 4
     for (int v = tid; v < N; v += kHbmBlock)
       __hip_atomic_store(&dist[v], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // +0.0
     __syncthreads();
     int maxlen = 0;
-    for (long long i = A.od_start[src] + tid; i < A.od_start[src + 1]; i += kHbmBlock) {
-      const int d = A.od_dest[i];
+    for (long long i = A.od_start[origin] + tid; i < A.od_start[origin + 1]; i += kHbmBlock) {
+      const int d = A.place[A.od_dest[i]];
       const double f = A.od_val[i];
       if (d == src || !(f > 0.0)) continue;
       if (ldg_i32(&pred[d]) < 0) {
-        if (atomicCAS(&A.err[0], 0, 1) == 0) { A.err[1] = src; A.err[2] = d; }
+        if (atomicCAS(&A.err[0], 0, 1) == 0) { A.err[1] = origin; A.err[2] = A.od_dest[i]; }
         continue;
       }
       int v = d, len = 0;
       while (v != src) {
         if (len > N || v < 0) {
-          if (atomicCAS(&A.err[0], 0, 3) == 0) { A.err[1] = src; A.err[2] = 0; }
+          if (atomicCAS(&A.err[0], 0, 3) == 0) { A.err[1] = origin; A.err[2] = 0; }
           break;
         }
         __hip_atomic_fetch_add(&flow[v], f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         v = ldg_i32(&ptail[v]);
         ++len;
       }
-      n_steps += (unsigned long long)len;
+      n_steps += (unsigned)len;
       maxlen = max(maxlen, len);
     }
     if (maxlen) atomicMax(&s_maxlen, maxlen);
     __syncthreads();
     double* __restrict__ yv = A.y + (size_t)var * A.E;
-    for (int v = tid; v < N; v += kHbmBlock) {
-      const double f = as_d(ldg_u64(&dist[v]));
-      if (f != 0.0) {
-        const int p = ldg_i32(&pred[v]);
-        if (p >= 0) {
-          unsafeAtomicAdd(&yv[p], f);
+    constexpr int kScan = 4;                           // nodes a thread has in flight
+    for (int v0 = tid; v0 < N; v0 += kScan * kHbmBlock) {
+      double f[kScan];
+      int p[kScan];
+#pragma unroll
+      for (int i = 0; i < kScan; ++i)
+        f[i] = v0 + i * kHbmBlock < N ? as_d(ldg_u64(&dist[v0 + i * kHbmBlock])) : 0.0;
+#pragma unroll
+      for (int i = 0; i < kScan; ++i) p[i] = f[i] != 0.0 ? ldg_i32(&pred[v0 + i * kHbmBlock]) : -1;
+#pragma unroll
+      for (int i = 0; i < kScan; ++i)
+        if (p[i] >= 0) {
+          unsafeAtomicAdd(&yv[p[i]], f[i]);
           ++n_loaded;
         }
-      }
     }
     __syncthreads();          // the row is reused by the next item
     c_load += (unsigned long long)(wall_clock64() - clk2);
   }
   if (A.counters) {
-    atomicAdd(&s_cnt[0], n_exp); atomicAdd(&s_cnt[1], n_scan); atomicAdd(&s_cnt[2], n_upd);
-    atomicAdd(&s_cnt[5], n_loaded); atomicAdd(&s_cnt[6], n_steps); atomicAdd(&s_cnt[7], n_def);
+    const unsigned long long cnt[8] = {n_exp, n_scan, n_upd, 0, 0, n_loaded, n_steps, n_def};
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < 3 || i > 4) atomicAdd(&s_cnt[i], cnt[i]);
     __syncthreads();
     if (tid == 0) {
       atomicAdd(&A.counters[7], s_cnt[7]);
@@ -1977,6 +2288,11 @@ struct tapgpu_ctx {
   // the LDS kernel's mirrors of the graph and the costs
   double *rec = nullptr, *sellw = nullptr;
   int *recpos = nullptr, *sellpos = nullptr, *sell_ptr = nullptr;
+  HbmRec* hrec = nullptr;             // the labels-in-HBM kernel's mirrors (ensure_hbm_mirrors)
+  uint2* hsell_id = nullptr;
+  double* hsellw = nullptr;
+  int* hplace = nullptr;              // [N] place of a node | [N] node of a place | slices
+  long long hsell_n = 0;
   unsigned* sell_id = nullptr;
   long long sell_n = 0;
   bool mirrors_stale = false;         // not kept since the last lanes loading
@@ -2390,13 +2706,16 @@ OriginArgs make_origin_args(tapgpu_ctx* c, const unsigned char* var_on) {
   A.rv_eid = c->rv_eid; A.tail = c->tail; A.fww = c->fww; A.rvw = c->rvw;
   A.rec = c->rec; A.sellw = c->sellw; A.sell_id = c->sell_id; A.sell_ptr = c->sell_ptr;
   A.sell_n = c->sell_n;
+  A.hrec = c->hrec; A.hsell_id = c->hsell_id; A.hsellw = c->hsellw; A.hsell_n = c->hsell_n;
+  A.place = c->hplace; A.node = c->hplace + c->N; A.hsell_ptr = c->hplace + 2 * (size_t)c->N;
   A.od_start = c->od_start; A.od_dest = c->od_dest; A.od_val = c->od_val;
   A.var_on = var_on; A.y = c->y; A.err = c->err_dev; A.counters = c->counters;
   A.chase = c->chase >= 0 ? c->chase : kDefaultChase;
   A.qcap = c->qcap;
-  A.hqcap = c->hqcap;
+  A.hqcap = std::max(c->hqcap, kHbmQueueMin);
   A.h_dist = c->h_dist; A.h_pred = c->h_pred; A.h_ptail = c->h_ptail;
-  A.delta = c->delta_mult > 0 ? c->delta_mult * c->mean_t0 : 0.0;
+  // (negative: a width to start from; before tuning, or without buckets)
+  A.delta = c->delta_mult > 0 ? c->delta_mult * c->mean_t0 : c->mean_t0 > 0 ? -4.0 * c->mean_t0 : -1.0;
   A.z0 = 0;
   A.zn = c->Z;
   return A;
@@ -2406,6 +2725,10 @@ OriginArgs make_origin_args(tapgpu_ctx* c, const unsigned char* var_on) {
 void advance_variant(tapgpu_ctx* c, OriginArgs& A, int64_t v) {
   A.fww += (size_t)v * c->E;
   A.rvw += (size_t)v * c->E;
+  if (c->hrec) {
+    A.hrec += (size_t)v * c->N;
+    A.hsellw += (size_t)v * c->hsell_n;
+  }
   if (c->rec) {
     A.rec += (size_t)v * c->N * kRecDoubles;
     A.sellw += (size_t)v * c->sell_n;
@@ -2447,6 +2770,7 @@ constexpr int kChaseCandidates[] = {0, 2, 4, 8, 16, 32};
 constexpr int kTuneBlocks = 4096;              // workgroups of a tuning launch on a batch
 
 int ensure_hbm(tapgpu_ctx* c);
+void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn);
 
 // Per-origin round counts of the recording loading (zeroed: origins a
 // loading skips keep 0 and go last).
@@ -2475,7 +2799,9 @@ int launch_origin(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, fl
     if (zh > 0) {
       int rc = ensure_hbm(c);
       if (rc) return rc;
-      A.h_dist = c->h_dist; A.h_pred = c->h_pred; A.h_ptail = c->h_ptail;
+      A = make_origin_args(c, var_on);            // (with what ensure_hbm has made)
+      advance_variant(c, A, v0); A.y += (size_t)v0 * c->E;
+      if (var_on) A.var_on = var_on + v0;
     }
     if (zh == 0) {
       if (c->origin_order_ready) {
@@ -2491,6 +2817,7 @@ int launch_origin(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, fl
     }
     if (ms) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
     if (zh > 0) {
+      launch_hbm_mirrors(c, A, Vn);
       HIPCHK(c, hipEventRecord(c->ev_fork, c->stream));
       HIPCHK(c, hipStreamWaitEvent(c->stream2, c->ev_fork, 0));
       OriginArgs B = A;
@@ -2737,9 +3064,95 @@ int aon_lds(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
   return finish_origin(c, Vn, t0);
 }
 
+// Places of the nodes in the labels-in-HBM kernel's rows: zones first, as
+// they are numbered; then, line by line, groups of through nodes grown from
+// a node beside the last ones, each time by the node with the most links to
+// the group.
+void hbm_places(int N, int ft0, const std::vector<int>& off, const std::vector<int>& dst,
+                const std::vector<int>& roff, const std::vector<int>& rsrc, int* place) {
+  constexpr int kLine = 16;                            // labels in 128 bytes
+  std::vector<char> done(N, 0);
+  std::vector<int> beside, links(N, 0), group;
+  size_t head = 0;
+  int next = std::min(ft0, N), scan = next;
+  for (int v = 0; v < next; ++v) { place[v] = v; done[v] = 1; }
+  while (next < N) {
+    int left = kLine - next % kLine;
+    while (left > 0 && next < N) {
+      while (head < beside.size() && done[beside[head]]) ++head;
+      if (head == beside.size())
+        while (done[scan]) ++scan;
+      group.assign(1, head < beside.size() ? beside[head] : scan);
+      while (!group.empty() && left > 0) {
+        size_t best = 0;
+        for (size_t i = 1; i < group.size(); ++i)
+          if (links[group[i]] > links[group[best]]) best = i;
+        const int v = group[best];
+        group.erase(group.begin() + best);
+        links[v] = 0;
+        done[v] = 1;
+        place[v] = next++;
+        --left;
+        auto grow = [&](int u) {
+          if (u < ft0 || done[u]) return;
+          if (links[u]++ == 0) group.push_back(u);
+        };
+        for (int k = off[v]; k < off[v + 1]; ++k) grow(dst[k]);
+        for (int k = roff[v]; k < roff[v + 1]; ++k) grow(rsrc[k]);
+      }
+      for (int u : group) { links[u] = 0; beside.push_back(u); }
+    }
+  }
+}
+
+// The labels-in-HBM kernel's mirrors: made with the context where its labels
+// do not fit LDS, otherwise when the kernel is chosen or first runs.
+int alloc_hbm_mirrors(tapgpu_ctx* c) {
+  if (c->hsellw) return TAPGPU_OK;
+  const int N = c->N, W = (N + kWave - 1) / kWave;
+  std::vector<int> off(N + 1), dst(c->E), roff(N + 1), rsrc(c->E);
+  auto get = [&](std::vector<int>& h, const int* d) {
+    return hipMemcpyAsync(h.data(), d, sizeof(int) * h.size(), hipMemcpyDeviceToHost, c->stream);
+  };
+  HIPCHK(c, get(off, c->fw_off));
+  HIPCHK(c, get(dst, c->fw_dst));
+  HIPCHK(c, get(roff, c->rv_off));
+  HIPCHK(c, get(rsrc, c->rv_src));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  std::vector<int> h(2 * (size_t)N + W + 1, 0);
+  hbm_places(N, c->ft0, off, dst, roff, rsrc, h.data());
+  for (int v = 0; v < N; ++v) h[(size_t)N + h[v]] = v;
+  int* ptr = h.data() + 2 * (size_t)N;
+  for (int v = c->ft0; v < N; ++v) {
+    int n = 0;
+    for (int k = roff[v]; k < roff[v + 1]; ++k) n += rsrc[k] != v && rsrc[k] >= c->ft0;
+    int& rows = ptr[h[v] / kWave + 1];
+    rows = std::max(rows, std::min(kSellWidth, n));
+  }
+  for (int i = 0; i < W; ++i) ptr[i + 1] = ptr[i] + ptr[i + 1] * kWave;
+  c->hsell_n = ptr[W];
+  int rc;
+  if (!c->hplace && (rc = dalloc(c, &c->hplace, h.size()))) return rc;
+  if (!c->hrec && (rc = dalloc(c, &c->hrec, (size_t)c->V * N))) return rc;
+  if (!c->hsell_id && (rc = dalloc(c, &c->hsell_id, (size_t)c->hsell_n))) return rc;
+  if ((rc = upload(c, c->hplace, h.data(), h.size()))) return rc;
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return dalloc(c, &c->hsellw, (size_t)c->V * c->hsell_n);
+}
+
+// Before a launch of the labels-in-HBM kernel: the mirrors of Vn variants
+// (A is advanced to the first), on the context's stream.
+void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn) {
+  const int per = kBlock, nodes = (c->N + kWave - 1) / kWave * kWave;
+  hipLaunchKernelGGL(k_hbm_mirrors, dim3((nodes + per - 1) / per, std::min(Vn, 65535)), dim3(kBlock), 0,
+                     c->stream, A, Vn, const_cast<HbmRec*>(A.hrec), const_cast<uint2*>(A.hsell_id),
+                     const_cast<double*>(A.hsellw));
+}
+
 // Per-workgroup scratch rows of the labels-in-HBM kernel (allocated on
 // first use: hbm_grid rows of N labels, predecessors and tails).
 int ensure_hbm(tapgpu_ctx* c) {
+  if (int rc = alloc_hbm_mirrors(c)) return rc;
   if (c->h_dist) return TAPGPU_OK;
   const size_t n = (size_t)c->hbm_grid * c->N;
   int rc;
@@ -2758,19 +3171,23 @@ int ensure_hbm(tapgpu_ctx* c) {
 // width, in units of the mean free-flow link time, and keeps the one with
 // the smallest busy time summed over the workgroups; the full launch
 // follows.  Results do not depend on the width.
-constexpr double kDeltaCandidates[] = {0.0, 1.0, 2.0, 4.0, 8.0, 16.0};
+// From narrow to wide, ending with the first that is clearly slower: a width
+// that lists more nodes than the queues hold is many times slower.
+constexpr double kDeltaCandidates[] = {1.0, 2.0, 4.0, 8.0, 16.0};
+constexpr double kDeltaStop = 1.2;
 
 int launch_hbm(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, int items_cap,
                float* ms) {
   if (!c->pre_cleared)
     HIPCHK(c, hipMemsetAsync(c->y + (size_t)v0 * c->E, 0, sizeof(double) * (size_t)Vn * c->E, c->stream));
   if (c->Z == 0) return TAPGPU_OK;
+  if (int rc = ensure_hbm(c)) return rc;        // (no allocation once made)
   OriginArgs A = make_origin_args(c, var_on);
   advance_variant(c, A, v0); A.y += (size_t)v0 * c->E;
   if (var_on) A.var_on = var_on + v0;
   const int items = std::min(c->Z * Vn, items_cap);
   const int G = std::min(c->hbm_grid, items);
-  if (int rc = ensure_hbm(c)) return rc;        // (the item counter; no allocation once made)
+  launch_hbm_mirrors(c, A, Vn);
   if (c->origin_order_ready) {
     A.order = c->d_origin_order;
     A.vn = Vn;
@@ -2824,6 +3241,7 @@ int tune_delta(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
     if ((rc = tuning_work(c, &work, &herr))) return rc;
     if (herr) break;
     if (best_work == 0.0 || work < best_work) { best_work = work; best_ms = ms; best = m; }
+    if (work > kDeltaStop * best_work) break;
   }
   c->delta_mult = best;
   c->stats.origin_tune_ms += best_ms;
@@ -3114,8 +3532,8 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
     for (int64_t j = 0; j < (pw_v ? V * E : E); ++j) pow4 = pow4 && (pw_v ? pw_v : net->power)[j] == 4.0;
     c->tiny_ok = c->lds_ok && pow4 && tiny_fits(c->N, c->E, c->Z) &&
                  tiny_lds_bytes(c->N, c->E) + 128 <= (size_t)lds_max;
-    c->hbm_lds = origin_hbm_lds_bytes(N, 0);
-    c->hbm_ok = c->hbm_lds + 256 <= (size_t)lds_max;
+    // (the networks it takes: 24 bytes of LDS for 64 nodes)
+    c->hbm_ok = 24 * (((size_t)N + 63) / 64) + 256 <= (size_t)lds_max;
     if (c->hbm_ok) {
       // queues from the LDS share of one of the kHbmPerCu workgroups on a CU
       int lds_cu = 0;
@@ -3123,8 +3541,9 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
               hipSuccess || lds_cu <= 0)
         lds_cu = lds_max;
       const size_t share = std::min<size_t>((size_t)lds_cu / kHbmPerCu, (size_t)lds_max) - 256;
-      const size_t spare = share > c->hbm_lds ? share - c->hbm_lds : 0;
-      c->hqcap_max = (int)std::min<size_t>(kHbmQueueMax, spare / 24) & ~63;
+      const size_t fixed = 8 * (((size_t)N + 63) / 64) + 12 * kHbmSlots;
+      const size_t spare = share > fixed ? share - fixed : 0;
+      c->hqcap_max = std::max((int)std::min<size_t>(kHbmQueueMax, spare / kHbmQueueBytes) & ~63, kHbmQueueMin);
       c->hqcap = c->hqcap_max;
       c->hbm_lds = origin_hbm_lds_bytes(N, c->hqcap_max);
     }
@@ -3276,6 +3695,7 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
   if ((rc = upload(c, c->present, hpres.data(), VE))) return rc;
   if ((rc = upload(c, c->col_src, col_src.data(), c->P))) return rc;
   if ((rc = upload(c, c->grp_var, grp_var.data(), c->Galloc))) return rc;
+  if (!c->lds_ok && c->hbm_ok && (rc = alloc_hbm_mirrors(c))) return rc;   // (tapgpu_sssp_noalloc allocates nothing)
   if (c->lds_ok) {
     if ((rc = upload(c, c->sell_ptr, sell_ptr.data(), sell_ptr.size()))) return rc;
     hipLaunchKernelGGL(k_mirrors, dim3((W * kWave + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream,
@@ -3432,10 +3852,11 @@ int tapgpu_sssp(tapgpu_ctx* c, int64_t variant, const int64_t* start_nodes, int6
       A.src_list = S.src; A.err = S.err; A.out_dist = S.dist; A.out_pred = S.pred; A.ld = ns;
       hipLaunchKernelGGL(k_sssp_begin, dim3(grid_for((long long)c->N * ns / kWave + 1)), dim3(kBlock), 0,
                          c->stream, S.pred, (long long)c->N * ns, S.err);
-      if (hbm)
+      if (hbm) {
+        if (s0 == 0) launch_hbm_mirrors(c, A, 1);
         hipLaunchKernelGGL(k_origin_hbm, dim3(std::min(ns, c->hbm_grid)), dim3(kHbmBlock), c->hbm_lds,
                            c->stream, A, 0, ns);
-      else
+      } else
         launch_lds(c, dim3(ns, 1), c->stream, A, 0);
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess)
@@ -3605,11 +4026,13 @@ int tapgpu_sssp_noalloc(tapgpu_ctx* c, int64_t variant, const int64_t* d_start_n
   const long long npred = (long long)c->N * ld;
   hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(npred / kWave + 1)), dim3(kBlock), 0, c->stream,
                      d_pred, npred, -1);
-  if (lds)
+  if (lds) {
     launch_lds(c, dim3((unsigned)num_start, 1), c->stream, A, 0);
-  else
+  } else {
+    launch_hbm_mirrors(c, A, 1);
     hipLaunchKernelGGL(k_origin_hbm, dim3((unsigned)std::min<int64_t>(num_start, rows)),
                        dim3(kHbmBlock), c->hbm_lds, c->stream, A, 0, (int)num_start);
+  }
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipMemcpyAsync(c->h_int, c->err_dev, sizeof(int) * 3, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -4157,7 +4580,14 @@ int tapgpu_set_strategy(tapgpu_ctx* c, int strategy) {
     return c->fail(TAPGPU_E_ARG, "network does not fit the one-origin-per-workgroup path");
   if (strategy == 3 && !c->hbm_ok)
     return c->fail(TAPGPU_E_ARG, "frontier bitmaps of this network do not fit LDS");
+  const int before = c->strategy;
   c->strategy = strategy;
+  // (tapgpu_sssp_noalloc allocates nothing, and takes this kernel then)
+  if (!use_lds(c) && c->hbm_ok)
+    if (int rc = alloc_hbm_mirrors(c)) {
+      c->strategy = before;
+      return rc;
+    }
   return TAPGPU_OK;
 }
 
