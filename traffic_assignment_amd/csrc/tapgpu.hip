@@ -1390,172 +1390,172 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
     };
     for (bool safe = false;; safe = true) {
 #pragma unroll 4
-    for (int v = tid; v < N; v += kHbmBlock) {
-      __hip_atomic_store(&dist[v], kMax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      __hip_atomic_store(&pred[v], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    for (int w = tid; w < W; w += kHbmBlock) bmA[w] = 0;
-    if (tid < 3) { s_near[tid] = tid == 0 ? 1 : 0; s_redo[tid] = 0; }
-    if (tid < 2) { s_far[tid] = 0; s_over[tid] = 0; s_min[tid] = ~0ull; }
-    if (tid == 0) s_lost = 0;
-    __syncthreads();
-    if (tid == 0) {
-      __hip_atomic_store(&dist[src], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      near_node[0] = (unsigned)src;
-      near_lab[0] = 0ull;
-    }
-    __syncthreads();
-    T = as_b(width);
-    r = 1; fb = 0; lim = qcap;
-    for (;;) {
-      const int n1 = min(uniform(s_near[(r - 1) % 3]), lim);
-      const int qn = n1 + min(uniform(s_redo[(r - 1) % 3]), qcap - lim);
-      const int from = ((r - 1) & 1) * qcap, to = (r & 1) * qcap;
-      const int room = qcap - (safe ? qn : min(qn, kHbmRedo));
-      for (int s = tid; s < kHbmSlots; s += kHbmBlock) { tab_node[s] = 0u; tab_lab[s] = ~0ull; }
-      for (int j0 = 0; j0 < qn; j0 += kPass) {
-        // ---- the lanes of a group take an entry (all lanes come here) ----
-        const int j = j0 + wave * (kWave / kHbmGroup) + grp;
-        const bool on = j < qn;
-        const int at = from + (j < n1 ? j : qcap - 1 - (j - n1));
-        const int u = on ? (int)near_node[at] : src;
-        const unsigned long long lab = on ? near_lab[at] : kMax;
-        const unsigned ro = (unsigned)u * 64u;
-        // (no load is masked: a merge with a default waits for each of them)
-        double w[kHbmCand];
-        int v[kHbmCand];
-        const unsigned long long have = ldg_u64(&dist[u]);
-        int more = *(const int*)(recb + (ro + 12u * kHrecLinks));
-#pragma unroll
-        for (int i = 0; i < kHbmCand; ++i) {
-          const unsigned k = min((unsigned)(g + i * kHbmGroup), (unsigned)(kHrecLinks - 1));
-          w[i] = *(const double*)(recb + (ro + k * 8u));
-          v[i] = *(const int*)(recb + (ro + 8u * kHrecLinks + k * 4u));
-        }
-        if (j0 == 0) __syncthreads();                  // (the table is clear; the loads are on their way)
-        const bool lost = on && g == 0 && have > lab;
-        if (__builtin_expect(__ballot(lost) != 0, 0)) {
-          const int k = place(lost, &s_redo[r % 3]);
-          if (lost && k < qcap - room) {
-            set_label(u, lab);
-            put(near_lab, near_node, to + qcap - 1 - k, lab, u);
-          } else if (lost) {
-            s_lost = 1;
-          }
-        }
-        bool first = on && g == 0 && have == lab;
-        const unsigned long long bit = 1ull << (u & 63);
-        if (first) first = !(atomicOr(&bmA[u >> 6], bit) & bit);
-        const bool go = (__ballot(first) >> (lane & ~(kHbmGroup - 1))) & 1ull;
-        n_exp += first;
-        unsigned long long cb[kHbmCand], hv[kHbmCand];
-        bool low[kHbmCand];
-        int slot[kHbmCand];
-#pragma unroll
-        for (int i = 0; i < kHbmCand; ++i) {
-          cb[i] = as_b(as_d(lab) + w[i]);
-          hv[i] = ldg_u64(&dist[v[i]]);
-        }
-#pragma unroll
-        for (int i = 0; i < kHbmCand; ++i) {
-          const bool in = go && cb[i] < kMax && g + i * kHbmGroup < kHrecLinks;
-          n_scan += in;
-          low[i] = in && cb[i] < hv[i];
-          slot[i] = -1;
-          if (low[i]) slot[i] = offer_label(v[i], cb[i]);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < kHbmCand; ++i)
-          if (slot[i] >= 0) low[i] = tab_lab[slot[i]] == cb[i];   // else a smaller one is stored
-        relax(v, cb, low, u, room);
-        if (!go) more = 0;
-        if (__ballot(more)) {                          // more links than the record holds
-          const int nu = A.node[u], ee = more ? A.fw_off[nu + 1] : 0;
-          for (int e = (more ? A.fw_off[nu] : 0) + g; __ballot(e < ee); e += kHbmGroup) {
-            int x[1] = {u};
-            double we = INFINITY;
-            if (e < ee) { x[0] = A.place[A.fw_dst[e]]; we = fw[e]; }
-            unsigned long long c[1] = {as_b(as_d(lab) + we)};
-            const bool ok = e < ee && x[0] >= ft0 && c[0] < kMax;
-            n_scan += ok;
-            bool lo[1] = {c[0] < (ok ? ldg_u64(&dist[x[0]]) : 0ull)};
-            relax(x, c, lo, u, room);
-          }
-        }
+      for (int v = tid; v < N; v += kHbmBlock) {
+        __hip_atomic_store(&dist[v], kMax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_store(&pred[v], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
-      // (every entry is taken: the last pass's barrier)
-      for (int j = tid; j < qn; j += kHbmBlock) bmA[near_node[from + (j < n1 ? j : qcap - 1 - (j - n1))] >> 6] = 0ull;
-      if (tid == 0) { s_near[(r + 1) % 3] = 0; s_redo[(r + 1) % 3] = 0; }
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // (the round's stores are done)
+      for (int w = tid; w < W; w += kHbmBlock) bmA[w] = 0;
+      if (tid < 3) { s_near[tid] = tid == 0 ? 1 : 0; s_redo[tid] = 0; }
+      if (tid < 2) { s_far[tid] = 0; s_over[tid] = 0; s_min[tid] = ~0ull; }
+      if (tid == 0) s_lost = 0;
       __syncthreads();
-      lim = room;
-      bool done = false;
-      while (!(min(uniform(s_near[r % 3]), lim) + uniform(s_redo[r % 3]))) {   // T moves
-        const int fn = uniform(s_far[fb]), fc = min(fn, fcap);
-        const bool over = uniform(s_over[fb]) != 0;
-        done = fn == 0 && !over;
-        if (done) break;
-        unsigned long long m = ~0ull;
-        for (int i = tid; i < fc; i += kHbmBlock) m = min(m, far_lab[i]);
-        for (int o = kWave / 2; o > 0; o >>= 1) m = min(m, __shfl_xor(m, o));
-        if (lane == 0 && m != ~0ull) atomicMin(&s_min[fb], m);
-        if (tid == 0) { s_far[fb ^ 1] = 0; s_over[fb ^ 1] = 0; s_near[r % 3] = 0; }
-        __syncthreads();
-        // 7/8 of the near queue at most, so that the entries find room for what
-        // they lower; far entries first, so that the far queue empties
-        const int fill = qcap - qcap / 8;
-        lim = fill;
-        const unsigned long long mn = s_min[fb];
-        // (above the smallest label also where delta is below its last bit)
-        if (mn != ~0ull) T = max(T, max(as_b(as_d(mn) + width), mn + 1));
-        if (tid == 0) s_min[fb ^ 1] = ~0ull;
-        for (int i0 = 0; i0 < fc; i0 += kHbmBlock) {   // (what stays closes up in place)
-          const int i = i0 + tid;
-          const bool on = i < fc;
-          const unsigned long long lab = on ? far_lab[i] : 0ull;
-          const int v = on ? (int)far_node[i] : src;
+      if (tid == 0) {
+        __hip_atomic_store(&dist[src], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        near_node[0] = (unsigned)src;
+        near_lab[0] = 0ull;
+      }
+      __syncthreads();
+      T = as_b(width);
+      r = 1; fb = 0; lim = qcap;
+      for (;;) {
+        const int n1 = min(uniform(s_near[(r - 1) % 3]), lim);
+        const int qn = n1 + min(uniform(s_redo[(r - 1) % 3]), qcap - lim);
+        const int from = ((r - 1) & 1) * qcap, to = (r & 1) * qcap;
+        const int room = qcap - (safe ? qn : min(qn, kHbmRedo));
+        for (int s = tid; s < kHbmSlots; s += kHbmBlock) { tab_node[s] = 0u; tab_lab[s] = ~0ull; }
+        for (int j0 = 0; j0 < qn; j0 += kPass) {
+          // ---- the lanes of a group take an entry (all lanes come here) ----
+          const int j = j0 + wave * (kWave / kHbmGroup) + grp;
+          const bool on = j < qn;
+          const int at = from + (j < n1 ? j : qcap - 1 - (j - n1));
+          const int u = on ? (int)near_node[at] : src;
+          const unsigned long long lab = on ? near_lab[at] : kMax;
+          const unsigned ro = (unsigned)u * 64u;
+          // (no load is masked: a merge with a default waits for each of them)
+          double w[kHbmCand];
+          int v[kHbmCand];
+          const unsigned long long have = ldg_u64(&dist[u]);
+          int more = *(const int*)(recb + (ro + 12u * kHrecLinks));
+#pragma unroll
+          for (int i = 0; i < kHbmCand; ++i) {
+            const unsigned k = min((unsigned)(g + i * kHbmGroup), (unsigned)(kHrecLinks - 1));
+            w[i] = *(const double*)(recb + (ro + k * 8u));
+            v[i] = *(const int*)(recb + (ro + 8u * kHrecLinks + k * 4u));
+          }
+          if (j0 == 0) __syncthreads();                  // (the table is clear; the loads are on their way)
+          const bool lost = on && g == 0 && have > lab;
+          if (__builtin_expect(__ballot(lost) != 0, 0)) {
+            const int k = place(lost, &s_redo[r % 3]);
+            if (lost && k < qcap - room) {
+              set_label(u, lab);
+              put(near_lab, near_node, to + qcap - 1 - k, lab, u);
+            } else if (lost) {
+              s_lost = 1;
+            }
+          }
+          bool first = on && g == 0 && have == lab;
+          const unsigned long long bit = 1ull << (u & 63);
+          if (first) first = !(atomicOr(&bmA[u >> 6], bit) & bit);
+          const bool go = (__ballot(first) >> (lane & ~(kHbmGroup - 1))) & 1ull;
+          n_exp += first;
+          unsigned long long cb[kHbmCand], hv[kHbmCand];
+          bool low[kHbmCand];
+          int slot[kHbmCand];
+#pragma unroll
+          for (int i = 0; i < kHbmCand; ++i) {
+            cb[i] = as_b(as_d(lab) + w[i]);
+            hv[i] = ldg_u64(&dist[v[i]]);
+          }
+#pragma unroll
+          for (int i = 0; i < kHbmCand; ++i) {
+            const bool in = go && cb[i] < kMax && g + i * kHbmGroup < kHrecLinks;
+            n_scan += in;
+            low[i] = in && cb[i] < hv[i];
+            slot[i] = -1;
+            if (low[i]) slot[i] = offer_label(v[i], cb[i]);
+          }
           __syncthreads();
-          const bool near = on && lab < T;
-          const int pn = place(near, &s_near[r % 3]);
-          const bool keep = on && !(near && pn < fill);
-          if (near && pn < fill) put(near_lab, near_node, to + pn, lab, v);
-          const int pf = place(keep, &s_far[fb ^ 1]);
-          if (keep) put(far_lab, far_node, pf, lab, v);
-        }
-        if (over) {
-          __syncthreads();
-          for (int u0 = wave * kWave; u0 < N; u0 += kHbmBlock) {
-            const int u = u0 + lane;
-            const bool on = u < N && ldg_i32(&pred[min(u, N - 1)]) != 0;
-            const int pn = place(on, &s_near[r % 3]);
-            if (on && pn < fill) {
-              __hip_atomic_store(&pred[u], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-              put(near_lab, near_node, to + pn, ldg_u64(&dist[u]), u);
-            } else if (on) {
-              s_over[fb ^ 1] = 1;
+#pragma unroll
+          for (int i = 0; i < kHbmCand; ++i)
+            if (slot[i] >= 0) low[i] = tab_lab[slot[i]] == cb[i];   // else a smaller one is stored
+          relax(v, cb, low, u, room);
+          if (!go) more = 0;
+          if (__ballot(more)) {                          // more links than the record holds
+            const int nu = A.node[u], ee = more ? A.fw_off[nu + 1] : 0;
+            for (int e = (more ? A.fw_off[nu] : 0) + g; __ballot(e < ee); e += kHbmGroup) {
+              int x[1] = {u};
+              double we = INFINITY;
+              if (e < ee) { x[0] = A.place[A.fw_dst[e]]; we = fw[e]; }
+              unsigned long long c[1] = {as_b(as_d(lab) + we)};
+              const bool ok = e < ee && x[0] >= ft0 && c[0] < kMax;
+              n_scan += ok;
+              bool lo[1] = {c[0] < (ok ? ldg_u64(&dist[x[0]]) : 0ull)};
+              relax(x, c, lo, u, room);
             }
           }
         }
-        fb ^= 1;
+        // (every entry is taken: the last pass's barrier)
+        for (int j = tid; j < qn; j += kHbmBlock) bmA[near_node[from + (j < n1 ? j : qcap - 1 - (j - n1))] >> 6] = 0ull;
+        if (tid == 0) { s_near[(r + 1) % 3] = 0; s_redo[(r + 1) % 3] = 0; }
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // (the round's stores are done)
         __syncthreads();
-        if (adapt) {
-          const int moved = uniform(s_near[r % 3]);
-          if (moved > 2 * kPass)
-            width *= 0.5;
-          else if (moved < kPass / 2)
-            width *= 2.0;
+        lim = room;
+        bool done = false;
+        while (!(min(uniform(s_near[r % 3]), lim) + uniform(s_redo[r % 3]))) {   // T moves
+          const int fn = uniform(s_far[fb]), fc = min(fn, fcap);
+          const bool over = uniform(s_over[fb]) != 0;
+          done = fn == 0 && !over;
+          if (done) break;
+          unsigned long long m = ~0ull;
+          for (int i = tid; i < fc; i += kHbmBlock) m = min(m, far_lab[i]);
+          for (int o = kWave / 2; o > 0; o >>= 1) m = min(m, __shfl_xor(m, o));
+          if (lane == 0 && m != ~0ull) atomicMin(&s_min[fb], m);
+          if (tid == 0) { s_far[fb ^ 1] = 0; s_over[fb ^ 1] = 0; s_near[r % 3] = 0; }
+          __syncthreads();
+          // 7/8 of the near queue at most, so that the entries find room for what
+          // they lower; far entries first, so that the far queue empties
+          const int fill = qcap - qcap / 8;
+          lim = fill;
+          const unsigned long long mn = s_min[fb];
+          // (above the smallest label also where delta is below its last bit)
+          if (mn != ~0ull) T = max(T, max(as_b(as_d(mn) + width), mn + 1));
+          if (tid == 0) s_min[fb ^ 1] = ~0ull;
+          for (int i0 = 0; i0 < fc; i0 += kHbmBlock) {   // (what stays closes up in place)
+            const int i = i0 + tid;
+            const bool on = i < fc;
+            const unsigned long long lab = on ? far_lab[i] : 0ull;
+            const int v = on ? (int)far_node[i] : src;
+            __syncthreads();
+            const bool near = on && lab < T;
+            const int pn = place(near, &s_near[r % 3]);
+            const bool keep = on && !(near && pn < fill);
+            if (near && pn < fill) put(near_lab, near_node, to + pn, lab, v);
+            const int pf = place(keep, &s_far[fb ^ 1]);
+            if (keep) put(far_lab, far_node, pf, lab, v);
+          }
+          if (over) {
+            __syncthreads();
+            for (int u0 = wave * kWave; u0 < N; u0 += kHbmBlock) {
+              const int u = u0 + lane;
+              const bool on = u < N && ldg_i32(&pred[min(u, N - 1)]) != 0;
+              const int pn = place(on, &s_near[r % 3]);
+              if (on && pn < fill) {
+                __hip_atomic_store(&pred[u], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                put(near_lab, near_node, to + pn, ldg_u64(&dist[u]), u);
+              } else if (on) {
+                s_over[fb ^ 1] = 1;
+              }
+            }
+          }
+          fb ^= 1;
+          __syncthreads();
+          if (adapt) {
+            const int moved = uniform(s_near[r % 3]);
+            if (moved > 2 * kPass)
+              width *= 0.5;
+            else if (moved < kPass / 2)
+              width *= 2.0;
+          }
         }
+        if (done) break;
+        if (r > 64 * N + 64) {
+          if (tid == 0 && atomicCAS(&A.err[0], 0, 2) == 0) { A.err[1] = origin; A.err[2] = 0; }
+          break;
+        }
+        ++r;
       }
-      if (done) break;
-      if (r > 64 * N + 64) {
-        if (tid == 0 && atomicCAS(&A.err[0], 0, 2) == 0) { A.err[1] = origin; A.err[2] = 0; }
-        break;
-      }
-      ++r;
-    }
-    if (safe || !uniform(s_lost)) break;
-    __syncthreads();
+      if (safe || !uniform(s_lost)) break;
+      __syncthreads();
     }
     n_rounds += (unsigned long long)r;
     if (A.work && tid == 0 && var == 0) A.work[origin] = r;
@@ -3143,8 +3143,8 @@ int alloc_hbm_mirrors(tapgpu_ctx* c) {
 // Before a launch of the labels-in-HBM kernel: the mirrors of Vn variants
 // (A is advanced to the first), on the context's stream.
 void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn) {
-  const int per = kBlock, nodes = (c->N + kWave - 1) / kWave * kWave;
-  hipLaunchKernelGGL(k_hbm_mirrors, dim3((nodes + per - 1) / per, std::min(Vn, 65535)), dim3(kBlock), 0,
+  const int nodes = (c->N + kWave - 1) / kWave * kWave;
+  hipLaunchKernelGGL(k_hbm_mirrors, dim3((nodes + kBlock - 1) / kBlock, std::min(Vn, 65535)), dim3(kBlock), 0,
                      c->stream, A, Vn, const_cast<HbmRec*>(A.hrec), const_cast<uint2*>(A.hsell_id),
                      const_cast<double*>(A.hsellw));
 }
