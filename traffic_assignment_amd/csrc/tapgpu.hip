@@ -45,6 +45,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -3107,7 +3108,7 @@ void hbm_places(int N, int ft0, const std::vector<int>& off, const std::vector<i
 
 // The labels-in-HBM kernel's mirrors: made with the context where its labels
 // do not fit LDS, otherwise when the kernel is chosen or first runs.
-int alloc_hbm_mirrors(tapgpu_ctx* c) {
+int alloc_hbm_mirrors(tapgpu_ctx* c) try {
   if (c->hsellw) return TAPGPU_OK;
   const int N = c->N, W = (N + kWave - 1) / kWave;
   std::vector<int> off(N + 1), dst(c->E), roff(N + 1), rsrc(c->E);
@@ -3138,6 +3139,8 @@ int alloc_hbm_mirrors(tapgpu_ctx* c) {
   if ((rc = upload(c, c->hplace, h.data(), h.size()))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return dalloc(c, &c->hsellw, (size_t)c->V * c->hsell_n);
+} catch (const std::bad_alloc&) {
+  return c->fail(TAPGPU_E_NOMEM, "out of host memory for the node numbering");
 }
 
 // Before a launch of the labels-in-HBM kernel: the mirrors of Vn variants
