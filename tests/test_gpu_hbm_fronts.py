@@ -1,0 +1,79 @@
+"""Searches of the labels-in-HBM kernel whose fronts or far nodes exceed its
+queues.  Labels, trees and volumes equal the LDS kernel's bit for bit, and the
+work stays in proportion: counts of expansions and rounds, not times."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import network, random_demand
+
+pytestmark = pytest.mark.gpu
+
+
+def random_graph(N, degree, Z, seed):
+    """A ring and `degree` links from every node to random ones: a search's
+    front is a large part of the nodes."""
+    from traffic_assignment_amd import synth
+    rng = np.random.default_rng(seed)
+    node = np.arange(1, N + 1)
+    init = np.concatenate([np.repeat(node, degree), node])
+    term = np.concatenate([rng.integers(1, N + 1, N * degree), np.roll(node, -1)])
+    order = np.lexsort((term, init))
+    E = init.size
+    net = synth.Network(num_zones=Z, num_nodes=N, first_thru_node=1, init=init[order].astype(np.int64),
+                        term=term[order].astype(np.int64), capacity=rng.uniform(20.0, 200.0, E),
+                        length=np.ones(E), fftime=rng.uniform(0.5, 3.0, E), B=np.full(E, 0.15),
+                        power=np.full(E, 4.0), speed=np.zeros(E), toll=np.zeros(E),
+                        ltype=np.ones(E, np.int16))
+    return net, rng
+
+
+def _both(eng, costs, starts):
+    """Equal results of both kernels; the labels-in-HBM kernel's counts."""
+    eng.set_costs(costs)
+    eng.set_strategy("lds")
+    d0, p0 = eng.sssp(starts)
+    y0 = eng.aon()
+    eng.set_strategy("hbm")
+    d, p = eng.sssp(starts)
+    a = eng.stats()
+    y = eng.aon()
+    b = eng.stats()
+    assert np.array_equal(d.view(np.int64), d0.view(np.int64))
+    assert np.array_equal(p, p0)
+    assert np.array_equal(y.view(np.int64), y0.view(np.int64))
+    return {k: b[k] - a[k] for k in ("origin_expansions", "origin_relax_rounds")}
+
+
+@pytest.mark.parametrize("N,degree", [(10000, 4), (8000, 6)])      # (fewer than 65,535 links)
+def test_hbm_fronts_beyond_the_queues(engine_mod, N, degree):
+    """Thousands of nodes in a round.  A node is expanded once more for each
+    time its label falls after an expansion, less than twice on average here,
+    whatever the queues hold."""
+    print(f"case hbm wide front N={N} degree={degree}", flush=True)
+    Z = 40
+    net, rng = random_graph(N, degree, Z, degree)
+    dem = random_demand(net, rng)
+    with engine_mod.TapEngine(net, dem) as eng:
+        eng.set_strategy("hbm")
+        eng.aon()                                   # (the bucket width is tuned)
+        for q in (-1, 200, 64):
+            eng.set_origin_queue(q)
+            n = _both(eng, net.fftime, rng.integers(1, net.num_nodes + 1, 20))
+            assert n["origin_expansions"] <= 2.0 * N * Z, q
+
+
+def test_hbm_few_expensive_links(engine_mod):
+    """One link in twenty at a million times its cost: what such links gave
+    nodes long reached otherwise costs no rounds."""
+    print("case hbm expensive links", flush=True)
+    net, dem = network("metro", 0.9)
+    rng = np.random.default_rng(5)
+    dear = net.fftime * np.where(rng.random(net.num_links) < 0.05, 1e6, 1.0)
+    starts = rng.integers(1, net.num_nodes + 1, 20)
+    with engine_mod.TapEngine(net, dem) as eng:
+        eng.set_strategy("hbm")
+        eng.aon()
+        plain = _both(eng, net.fftime, starts)["origin_relax_rounds"]
+        assert _both(eng, dear, starts)["origin_relax_rounds"] <= 1.5 * plain

@@ -1119,6 +1119,7 @@ constexpr size_t kHbmQueueBytes = 48;           // per entry of the queue size
 constexpr int kHbmGroup = 2;                    // lanes per expanded node
 constexpr int kHbmCand = (5 + kHbmGroup - 1) / kHbmGroup;   // links per lane, at most
 constexpr int kHbmRedo = 64;                    // places kept for entries to be followed up again
+constexpr int kHbmFew = 32;                     // entries brought near at once, below which the far queue is weeded
 constexpr int kHbmSlots = 1024;                 // of the table that settles which lane lowers a label
 size_t origin_hbm_lds_bytes(int N, int hqcap) {
   const size_t bitmap = 8ull * (size_t)((N + 63) / 64);
@@ -1215,8 +1216,8 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
   unsigned* near_node = far_node + fcap;
   unsigned* tab_node = near_node + 2 * (size_t)qcap;    // [kHbmSlots] node + 1, 0: free
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-  __shared__ int s_near[3], s_redo[3], s_far[2], s_over[2], s_lost;
-  __shared__ unsigned long long s_min[2];
+  __shared__ int s_near[3], s_redo[3], s_far[2], s_wide[2];
+  __shared__ unsigned long long s_min[3];
   __shared__ unsigned long long s_cnt[8];
   __shared__ int s_maxlen;
   __shared__ int s_level_ties, s_left, s_added;
@@ -1285,13 +1286,18 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
     //      goes on anyway).  Without it the larger value wins half of the
     //      races and is expanded: 2.6 times the rounds on regional.
     //      Nodes that find the near queue full go to the far one; no store
-    //      without an entry: where that is full too, the link's tail is
-    //      flagged (in pred's row, which is free until the predecessors
-    //      are chosen) and expanded again when T moves.  Entries to be
-    //      followed up once more grow from the end of the near queue, where
-    //      kHbmRedo places are kept for them; should a round have more, the
-    //      search starts again, `safe`: with as many places kept as the
-    //      round has entries.
+    //      without an entry: where that is full too, the search turns wide
+    //      (below), with the nodes of every entry flagged, the round's own
+    //      among them.  Entries to be followed up once more grow from the end
+    //      of the near queue, where kHbmRedo places are kept for them; should
+    //      a round have more, the search turns wide too.
+    //      A far entry whose node has a smaller label by now is of no use.
+    //      When T moves they are weeded out if the far queue is half full or
+    //      the last move brought few entries near: where some links cost far
+    //      more than the others, the search would otherwise end in a move and
+    //      a round for each of thousands of them (regional with 5% of its
+    //      links at a million times their cost: 2,360 moves an origin and
+    //      160 ms a loading, 39 weeded, as without such links).
     //      A round is a chain of trips to the XCD's L2 and beyond, so what
     //      counts is their number and the lines they touch: kHbmGroup lanes
     //      share an expanded node, whose links are one line that is read
@@ -1307,6 +1313,7 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
     double width = fabs(A.delta);
     unsigned long long T = 0;
     int r = 1, fb = 0, lim = qcap;             // lim: places of the near queue for lowered nodes
+    bool wide = false;
     constexpr int kPass = kHbmBlock / kHbmGroup;     // nodes taken at once
     const int g = lane & (kHbmGroup - 1), grp = lane / kHbmGroup;
     // this lane's place among the lanes with `want`, counted on *n
@@ -1342,9 +1349,9 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
       }
       return -1;
     };
-    // u -> v[i] gives v[i] the label cb[i] where low[i]: lowers and lists
-    // them, one LDS atomic for both queues and all of the wavefront's
-    auto relax = [&](auto& v, auto& cb, auto& low, int u, int room) {
+    // gives v[i] the label cb[i] where low[i]: lowers and lists them, one LDS
+    // atomic for both queues and all of the wavefront's
+    auto relax = [&](auto& v, auto& cb, auto& low, int room) {
       constexpr int K = sizeof(low) / sizeof(low[0]);
       unsigned long long bn[K], bf[K];
       int nn = 0, nf = 0;
@@ -1377,8 +1384,7 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
           put(far_lab, far_node, at, cb[i], v[i]);
           ++n_def;
         } else if (low[i]) {
-          __hip_atomic_store(&pred[u], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          s_over[fb] = 1;
+          s_wide[r & 1] = 1;
           low[i] = false;
         }
         if (low[i]) {
@@ -1389,174 +1395,377 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         pf += __popcll(bf[i]);
       }
     };
-    for (bool safe = false;; safe = true) {
 #pragma unroll 4
-      for (int v = tid; v < N; v += kHbmBlock) {
-        __hip_atomic_store(&dist[v], kMax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        __hip_atomic_store(&pred[v], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
-      for (int w = tid; w < W; w += kHbmBlock) bmA[w] = 0;
-      if (tid < 3) { s_near[tid] = tid == 0 ? 1 : 0; s_redo[tid] = 0; }
-      if (tid < 2) { s_far[tid] = 0; s_over[tid] = 0; s_min[tid] = ~0ull; }
-      if (tid == 0) s_lost = 0;
-      __syncthreads();
-      if (tid == 0) {
-        __hip_atomic_store(&dist[src], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        near_node[0] = (unsigned)src;
-        near_lab[0] = 0ull;
-      }
-      __syncthreads();
-      T = as_b(width);
-      r = 1; fb = 0; lim = qcap;
-      for (;;) {
-        const int n1 = min(uniform(s_near[(r - 1) % 3]), lim);
-        const int qn = n1 + min(uniform(s_redo[(r - 1) % 3]), qcap - lim);
-        const int from = ((r - 1) & 1) * qcap, to = (r & 1) * qcap;
-        const int room = qcap - (safe ? qn : min(qn, kHbmRedo));
-        for (int s = tid; s < kHbmSlots; s += kHbmBlock) { tab_node[s] = 0u; tab_lab[s] = ~0ull; }
-        for (int j0 = 0; j0 < qn; j0 += kPass) {
-          // ---- the lanes of a group take an entry (all lanes come here) ----
-          const int j = j0 + wave * (kWave / kHbmGroup) + grp;
-          const bool on = j < qn;
-          const int at = from + (j < n1 ? j : qcap - 1 - (j - n1));
-          const int u = on ? (int)near_node[at] : src;
-          const unsigned long long lab = on ? near_lab[at] : kMax;
-          const unsigned ro = (unsigned)u * 64u;
-          // (no load is masked: a merge with a default waits for each of them)
-          double w[kHbmCand];
-          int v[kHbmCand];
-          const unsigned long long have = ldg_u64(&dist[u]);
-          int more = *(const int*)(recb + (ro + 12u * kHrecLinks));
+    for (int v = tid; v < N; v += kHbmBlock)
+      __hip_atomic_store(&dist[v], kMax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    for (int w = tid; w < W; w += kHbmBlock) bmA[w] = 0;
+    if (tid < 3) { s_near[tid] = tid == 0 ? 1 : 0; s_redo[tid] = 0; s_min[tid] = ~0ull; }
+    if (tid < 2) { s_far[tid] = 0; s_wide[tid] = 0; }
+    __syncthreads();
+    if (tid == 0) {
+      __hip_atomic_store(&dist[src], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      near_node[0] = (unsigned)src;
+      near_lab[0] = 0ull;
+    }
+    __syncthreads();
+    T = as_b(width);
+    bool few = false;                        // the last move of T brought few entries near
+    for (;;) {
+      const int n1 = min(uniform(s_near[(r - 1) % 3]), lim);
+      const int qn = n1 + min(uniform(s_redo[(r - 1) % 3]), qcap - lim);
+      const int from = ((r - 1) & 1) * qcap, to = (r & 1) * qcap;
+      const int room = qcap - min(qn, kHbmRedo);
+      for (int s = tid; s < kHbmSlots; s += kHbmBlock) { tab_node[s] = 0u; tab_lab[s] = ~0ull; }
+      for (int j0 = 0; j0 < qn; j0 += kPass) {
+        // ---- the lanes of a group take an entry (all lanes come here) ----
+        const int j = j0 + wave * (kWave / kHbmGroup) + grp;
+        const bool on = j < qn;
+        const int at = from + (j < n1 ? j : qcap - 1 - (j - n1));
+        const int u = on ? (int)near_node[at] : src;
+        const unsigned long long lab = on ? near_lab[at] : kMax;
+        const unsigned ro = (unsigned)u * 64u;
+        // (no load is masked: a merge with a default waits for each of them)
+        double w[kHbmCand];
+        int v[kHbmCand];
+        const unsigned long long have = ldg_u64(&dist[u]);
+        int more = *(const int*)(recb + (ro + 12u * kHrecLinks));
 #pragma unroll
-          for (int i = 0; i < kHbmCand; ++i) {
-            const unsigned k = min((unsigned)(g + i * kHbmGroup), (unsigned)(kHrecLinks - 1));
-            w[i] = *(const double*)(recb + (ro + k * 8u));
-            v[i] = *(const int*)(recb + (ro + 8u * kHrecLinks + k * 4u));
-          }
-          if (j0 == 0) __syncthreads();                  // (the table is clear; the loads are on their way)
-          const bool lost = on && g == 0 && have > lab;
-          if (__builtin_expect(__ballot(lost) != 0, 0)) {
-            const int k = place(lost, &s_redo[r % 3]);
-            if (lost && k < qcap - room) {
-              set_label(u, lab);
-              put(near_lab, near_node, to + qcap - 1 - k, lab, u);
-            } else if (lost) {
-              s_lost = 1;
-            }
-          }
-          bool first = on && g == 0 && have == lab;
-          const unsigned long long bit = 1ull << (u & 63);
-          if (first) first = !(atomicOr(&bmA[u >> 6], bit) & bit);
-          const bool go = (__ballot(first) >> (lane & ~(kHbmGroup - 1))) & 1ull;
-          n_exp += first;
-          unsigned long long cb[kHbmCand], hv[kHbmCand];
-          bool low[kHbmCand];
-          int slot[kHbmCand];
-#pragma unroll
-          for (int i = 0; i < kHbmCand; ++i) {
-            cb[i] = as_b(as_d(lab) + w[i]);
-            hv[i] = ldg_u64(&dist[v[i]]);
-          }
-#pragma unroll
-          for (int i = 0; i < kHbmCand; ++i) {
-            const bool in = go && cb[i] < kMax && g + i * kHbmGroup < kHrecLinks;
-            n_scan += in;
-            low[i] = in && cb[i] < hv[i];
-            slot[i] = -1;
-            if (low[i]) slot[i] = offer_label(v[i], cb[i]);
-          }
-          __syncthreads();
-#pragma unroll
-          for (int i = 0; i < kHbmCand; ++i)
-            if (slot[i] >= 0) low[i] = tab_lab[slot[i]] == cb[i];   // else a smaller one is stored
-          relax(v, cb, low, u, room);
-          if (!go) more = 0;
-          if (__ballot(more)) {                          // more links than the record holds
-            const int nu = A.node[u], ee = more ? A.fw_off[nu + 1] : 0;
-            for (int e = (more ? A.fw_off[nu] : 0) + g; __ballot(e < ee); e += kHbmGroup) {
-              int x[1] = {u};
-              double we = INFINITY;
-              if (e < ee) { x[0] = A.place[A.fw_dst[e]]; we = fw[e]; }
-              unsigned long long c[1] = {as_b(as_d(lab) + we)};
-              const bool ok = e < ee && x[0] >= ft0 && c[0] < kMax;
-              n_scan += ok;
-              bool lo[1] = {c[0] < (ok ? ldg_u64(&dist[x[0]]) : 0ull)};
-              relax(x, c, lo, u, room);
-            }
+        for (int i = 0; i < kHbmCand; ++i) {
+          const unsigned k = min((unsigned)(g + i * kHbmGroup), (unsigned)(kHrecLinks - 1));
+          w[i] = *(const double*)(recb + (ro + k * 8u));
+          v[i] = *(const int*)(recb + (ro + 8u * kHrecLinks + k * 4u));
+        }
+        if (j0 == 0) __syncthreads();                  // (the table is clear; the loads are on their way)
+        const bool lost = on && g == 0 && have > lab;
+        if (__builtin_expect(__ballot(lost) != 0, 0)) {
+          const int k = place(lost, &s_redo[r % 3]);
+          if (lost && k < qcap - room) {
+            set_label(u, lab);
+            put(near_lab, near_node, to + qcap - 1 - k, lab, u);
+          } else if (lost) {
+            s_wide[r & 1] = 1;
           }
         }
-        // (every entry is taken: the last pass's barrier)
-        for (int j = tid; j < qn; j += kHbmBlock) bmA[near_node[from + (j < n1 ? j : qcap - 1 - (j - n1))] >> 6] = 0ull;
-        if (tid == 0) { s_near[(r + 1) % 3] = 0; s_redo[(r + 1) % 3] = 0; }
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // (the round's stores are done)
+        bool first = on && g == 0 && have == lab;
+        const unsigned long long bit = 1ull << (u & 63);
+        if (first) first = !(atomicOr(&bmA[u >> 6], bit) & bit);
+        const bool go = (__ballot(first) >> (lane & ~(kHbmGroup - 1))) & 1ull;
+        n_exp += first;
+        unsigned long long cb[kHbmCand], hv[kHbmCand];
+        bool low[kHbmCand];
+        int slot[kHbmCand];
+#pragma unroll
+        for (int i = 0; i < kHbmCand; ++i) {
+          cb[i] = as_b(as_d(lab) + w[i]);
+          hv[i] = ldg_u64(&dist[v[i]]);
+        }
+#pragma unroll
+        for (int i = 0; i < kHbmCand; ++i) {
+          const bool in = go && cb[i] < kMax && g + i * kHbmGroup < kHrecLinks;
+          n_scan += in;
+          low[i] = in && cb[i] < hv[i];
+          slot[i] = -1;
+          if (low[i]) slot[i] = offer_label(v[i], cb[i]);
+        }
         __syncthreads();
-        lim = room;
-        bool done = false;
-        while (!(min(uniform(s_near[r % 3]), lim) + uniform(s_redo[r % 3]))) {   // T moves
-          const int fn = uniform(s_far[fb]), fc = min(fn, fcap);
-          const bool over = uniform(s_over[fb]) != 0;
-          done = fn == 0 && !over;
-          if (done) break;
-          unsigned long long m = ~0ull;
-          for (int i = tid; i < fc; i += kHbmBlock) m = min(m, far_lab[i]);
-          for (int o = kWave / 2; o > 0; o >>= 1) m = min(m, __shfl_xor(m, o));
-          if (lane == 0 && m != ~0ull) atomicMin(&s_min[fb], m);
-          if (tid == 0) { s_far[fb ^ 1] = 0; s_over[fb ^ 1] = 0; s_near[r % 3] = 0; }
-          __syncthreads();
-          // 7/8 of the near queue at most, so that the entries find room for what
-          // they lower; far entries first, so that the far queue empties
-          const int fill = qcap - qcap / 8;
-          lim = fill;
-          const unsigned long long mn = s_min[fb];
-          // (above the smallest label also where delta is below its last bit)
-          if (mn != ~0ull) T = max(T, max(as_b(as_d(mn) + width), mn + 1));
-          if (tid == 0) s_min[fb ^ 1] = ~0ull;
-          for (int i0 = 0; i0 < fc; i0 += kHbmBlock) {   // (what stays closes up in place)
-            const int i = i0 + tid;
-            const bool on = i < fc;
-            const unsigned long long lab = on ? far_lab[i] : 0ull;
-            const int v = on ? (int)far_node[i] : src;
-            __syncthreads();
-            const bool near = on && lab < T;
-            const int pn = place(near, &s_near[r % 3]);
-            const bool keep = on && !(near && pn < fill);
-            if (near && pn < fill) put(near_lab, near_node, to + pn, lab, v);
-            const int pf = place(keep, &s_far[fb ^ 1]);
-            if (keep) put(far_lab, far_node, pf, lab, v);
-          }
-          if (over) {
-            __syncthreads();
-            for (int u0 = wave * kWave; u0 < N; u0 += kHbmBlock) {
-              const int u = u0 + lane;
-              const bool on = u < N && ldg_i32(&pred[min(u, N - 1)]) != 0;
-              const int pn = place(on, &s_near[r % 3]);
-              if (on && pn < fill) {
-                __hip_atomic_store(&pred[u], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                put(near_lab, near_node, to + pn, ldg_u64(&dist[u]), u);
-              } else if (on) {
-                s_over[fb ^ 1] = 1;
-              }
-            }
-          }
-          fb ^= 1;
-          __syncthreads();
-          if (adapt) {
-            const int moved = uniform(s_near[r % 3]);
-            if (moved > 2 * kPass)
-              width *= 0.5;
-            else if (moved < kPass / 2)
-              width *= 2.0;
+#pragma unroll
+        for (int i = 0; i < kHbmCand; ++i)
+          if (slot[i] >= 0) low[i] = tab_lab[slot[i]] == cb[i];   // else a smaller one is stored
+        relax(v, cb, low, room);
+        if (!go) more = 0;
+        if (__ballot(more)) {                          // more links than the record holds
+          const int nu = A.node[u], ee = more ? A.fw_off[nu + 1] : 0;
+          for (int e = (more ? A.fw_off[nu] : 0) + g; __ballot(e < ee); e += kHbmGroup) {
+            int x[1] = {u};
+            double we = INFINITY;
+            if (e < ee) { x[0] = A.place[A.fw_dst[e]]; we = fw[e]; }
+            unsigned long long c[1] = {as_b(as_d(lab) + we)};
+            const bool ok = e < ee && x[0] >= ft0 && c[0] < kMax;
+            n_scan += ok;
+            bool lo[1] = {c[0] < (ok ? ldg_u64(&dist[x[0]]) : 0ull)};
+            relax(x, c, lo, room);
           }
         }
+      }
+      // (every entry is taken: the last pass's barrier)
+      for (int j = tid; j < qn; j += kHbmBlock) bmA[near_node[from + (j < n1 ? j : qcap - 1 - (j - n1))] >> 6] = 0ull;
+      if (tid == 0) { s_near[(r + 1) % 3] = 0; s_redo[(r + 1) % 3] = 0; }
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // (the round's stores are done)
+      __syncthreads();
+      lim = room;
+      if (__builtin_expect(uniform(s_wide[r & 1]), 0)) {                    // an entry found no place
+        const int nn = min(uniform(s_near[r % 3]), lim), nr = min(uniform(s_redo[r % 3]), qcap - lim);
+        const int nf = min(uniform(s_far[fb]), fcap);
+        for (int j = tid; j < qn + nn + nr + nf; j += kHbmBlock) {
+          const int k = j - qn, at = j < qn ? from + (j < n1 ? j : qcap - 1 - (j - n1))
+                                            : to + (k < nn ? k : qcap - 1 - (k - nn));
+          const bool near = k < nn + nr;
+          const unsigned long long lab = near ? near_lab[at] : far_lab[k - nn - nr];
+          const int v = (int)(near ? near_node[at] : far_node[k - nn - nr]);
+          if (k >= 0 && ldg_u64(&dist[v]) < lab) continue;   // (another entry stands for it)
+          (void)__hip_atomic_fetch_min(&dist[v], lab, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          atomicOr(&bmA[v >> 6], 1ull << (v & 63));
+        }
+        wide = true;
+        break;
+      }
+      bool done = false;
+      while (!(min(uniform(s_near[r % 3]), lim) + uniform(s_redo[r % 3]))) {   // T moves
+        const int fc = min(uniform(s_far[fb]), fcap);
+        done = fc == 0;
         if (done) break;
+        const bool weed = few || fc > fcap / 2;
+        unsigned long long m = ~0ull;
+        for (int i = tid; i < fc; i += kHbmBlock) {
+          const unsigned long long lab = far_lab[i];
+          if (weed && ldg_u64(&dist[far_node[i]]) < lab)
+            far_lab[i] = ~0ull;
+          else
+            m = min(m, lab);
+        }
+        for (int o = kWave / 2; o > 0; o >>= 1) m = min(m, __shfl_xor(m, o));
+        if (lane == 0 && m != ~0ull) atomicMin(&s_min[fb], m);
+        if (tid == 0) { s_far[fb ^ 1] = 0; s_near[r % 3] = 0; }
+        __syncthreads();
+        // 7/8 of the near queue at most, so that the entries find room for what
+        // they lower; far entries first, so that the far queue empties
+        const int fill = qcap - qcap / 8;
+        lim = fill;
+        const unsigned long long mn = s_min[fb];
+        // (above the smallest label also where delta is below its last bit)
+        if (mn != ~0ull) T = max(T, max(as_b(as_d(mn) + width), mn + 1));
+        if (tid == 0) s_min[fb ^ 1] = ~0ull;
+        for (int i0 = 0; i0 < fc; i0 += kHbmBlock) {   // (what stays closes up in place)
+          const int i = i0 + tid;
+          const unsigned long long lab = i < fc ? far_lab[i] : ~0ull;
+          const bool on = lab != ~0ull;
+          const int v = on ? (int)far_node[i] : src;
+          __syncthreads();
+          const bool near = on && lab < T;
+          const int pn = place(near, &s_near[r % 3]);
+          const bool keep = on && !(near && pn < fill);
+          if (near && pn < fill) put(near_lab, near_node, to + pn, lab, v);
+          const int pf = place(keep, &s_far[fb ^ 1]);
+          if (keep) put(far_lab, far_node, pf, lab, v);
+        }
+        fb ^= 1;
+        __syncthreads();
+        const int moved = uniform(s_near[r % 3]);
+        few = moved < kHbmFew;
+        if (adapt) {
+          if (moved > 2 * kPass)
+            width *= 0.5;
+          else if (moved < kPass / 2)
+            width *= 2.0;
+        }
+      }
+      if (done) break;
+      if (r > 64 * N + 64) {
+        if (tid == 0 && atomicCAS(&A.err[0], 0, 2) == 0) { A.err[1] = origin; A.err[2] = 0; }
+        break;
+      }
+      ++r;
+    }
+    // ---- wide: more nodes wait than the queues hold.  They are flagged in
+    //      bitmaps, one for the round, one for the next and one of those at
+    //      T or above (which are flagged for the next round too where LDS has
+    //      no room for three), and listed by node alone; a round of more
+    //      nodes than its list holds goes by the flags, a wavefront taking
+    //      every 8th word (64 nodes).  A lane expands a node.  Labels are
+    //      lowered by atomics here, so nothing needs to be followed up.
+    //      Measured, ms a loading: a random graph (40,000 nodes of 5 links,
+    //      100 origins, fronts of thousands) 1.8; 4.9 with the tails of links
+    //      that found no place expanded again at each move of T, and 2.1 with
+    //      every listed node looked at in every round.  23,500 nodes of a
+    //      city and 1,000 origins, costs spread by a log-normal factor of
+    //      sigma 2: 4.9, 9.4 and 5.9. ----
+    if (__builtin_expect(wide, 0)) {
+      unsigned long long *cur = bmA, *nxt = bmC;         // (the queues' place)
+      const int room = (int)((12 * kHbmSlots + kHbmQueueBytes * (size_t)qcap) / 8) - W;
+      const bool three = room - W >= kHbmBlock;
+      const int listed = max(0, three ? room - W : room);            // entries of a list
+      unsigned long long* far = nxt + W;
+      int* list = (int*)(three ? far + W : nxt + W);     // 2 x [listed]
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __syncthreads();
+      for (int w = tid; w < (three ? 2 * W : W); w += kHbmBlock) nxt[w] = 0;
+      // in s_near the flagged nodes of a round (the first goes by the flags),
+      // in s_redo the expanded ones, in s_far[0] whether a node waits for T
+      if (tid < 3) { s_near[tid] = tid == r % 3 ? INT_MAX : 0; s_redo[tid] = 0; s_min[tid] = ~0ull; }
+      if (tid == 0) s_far[0] = 0;
+      __syncthreads();
+      // f(node of this lane, flagged, label) for every word of `bm` with a
+      // flag, which are cleared; the next word's labels are on their way
+      // meanwhile
+      auto words = [&](unsigned long long* bm, auto&& f) {
+        for (int w0 = wave; w0 < W; w0 += kWaves * kWave) {
+          const int wi = w0 + lane * kWaves;
+          unsigned long long mine = 0ull;
+          if (wi < W) {
+            mine = bm[wi];
+            if (mine) bm[wi] = 0ull;
+          }
+          auto label = [&](unsigned long long m) {
+            const int k = m ? __ffsll((long long)m) - 1 : 0;
+            return ldg_u64(&dist[min((w0 + k * kWaves) * kWave + lane, N - 1)]);
+          };
+          unsigned long long m = __ballot(mine != 0ull), ahead = label(m);
+          while (m) {
+            const int k = __ffsll((long long)m) - 1;
+            const unsigned long long lab = ahead;
+            m &= m - 1;
+            ahead = label(m);
+            const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)mine, k);
+            const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(mine >> 32), k);
+            f((w0 + k * kWaves) * kWave + lane, ((lane < 32 ? lo : hi) >> (lane & 31)) & 1u, lab);
+          }
+        }
+      };
+      // flags v[i] where want[i] for round r + 1 and lists it there, unless it is
+      auto flag = [&](auto& v, auto& want) {
+        constexpr int K = sizeof(want) / sizeof(want[0]);
+        unsigned long long bal[K];
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          const unsigned long long bit = 1ull << (v[i] & 63);
+          if (want[i]) want[i] = !(atomicOr(&nxt[v[i] >> 6], bit) & bit);
+        }
+#pragma unroll
+        for (int i = 0; i < K; ++i) { bal[i] = __ballot(want[i]); n += __popcll(bal[i]); }
+        if (!n) return;
+        int at = 0;
+        if (lane == 0) at = lds_add(&s_near[r % 3], n);
+        at = __builtin_amdgcn_readlane(at, 0);
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          const int k = at + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bal[i] >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((unsigned)bal[i], 0u));
+          if (want[i] && k < listed) list[(r & 1) * listed + k] = v[i];
+          at += __popcll(bal[i]);
+        }
+      };
+      unsigned long long kept = ~0ull;
+      int taken = 0, since = 0;                          // nodes expanded in this round, since T moved
+      auto lower = [&](auto& v, auto& c, auto& have, bool go) {
+        constexpr int K = sizeof(v) / sizeof(v[0]);
+        bool want[K];
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          const bool in = go && c[i] < kMax, low = in && c[i] < have[i], later = three && c[i] >= T;
+          n_scan += in;
+          n_upd += low;
+          want[i] = low && !later;
+          if (low) (void)__hip_atomic_fetch_min(&dist[v[i]], c[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          if (low && later) {
+            atomicOr(&far[v[i] >> 6], 1ull << (v[i] & 63));
+            s_far[0] = 1;
+          }
+        }
+        flag(v, want);
+      };
+      auto expand = [&](int u, bool on, unsigned long long lab) {    // (all lanes)
+        const bool go = on && lab < T, keep = on && !go;
+        if (__ballot(keep)) {
+          if (three) {
+            if (keep) { atomicOr(&far[u >> 6], 1ull << (u & 63)); s_far[0] = 1; }
+          } else {
+            if (keep) kept = min(kept, lab);
+            int x[1] = {u};
+            bool want[1] = {keep};
+            flag(x, want);
+          }
+        }
+        const unsigned long long m = __ballot(go);
+        if (!m) return;
+        taken += __popcll(m);
+        n_exp += go;
+        if (!go) u = src;
+        const HbmRec* rec = (const HbmRec*)recb + u;
+        int x[kHrecLinks];
+        unsigned long long c[kHrecLinks], have[kHrecLinks];
+        const int more = go ? rec->more : 0;
+#pragma unroll
+        for (int i = 0; i < kHrecLinks; ++i) { x[i] = rec->head[i]; c[i] = as_b(as_d(lab) + rec->w[i]); }
+#pragma unroll
+        for (int i = 0; i < kHrecLinks; ++i) have[i] = ldg_u64(&dist[x[i]]);
+        lower(x, c, have, go);
+        if (__ballot(more)) {
+          int e = 0, e1 = 0;
+          if (more) { e = A.fw_off[A.node[u]]; e1 = A.fw_off[A.node[u] + 1]; }
+          for (; __ballot(e < e1); ++e) {
+            int y[1] = {u};
+            unsigned long long cy[1] = {~0ull};
+            if (e < e1) { y[0] = A.place[A.fw_dst[e]]; cy[0] = as_b(as_d(lab) + fw[e]); }
+            unsigned long long hy[1] = {ldg_u64(&dist[y[0]])};
+            lower(y, cy, hy, e < e1 && y[0] >= ft0 && y[0] != u);
+          }
+        }
+      };
+      for (++r;; ++r) {
+        const int sl = r % 3, n = uniform(s_near[(r - 1) % 3]);
+        taken = 0;
+        if (n <= listed) {
+          const int* q = list + ((r - 1) & 1) * listed;
+          for (int j0 = 0; j0 < n; j0 += kHbmBlock) {
+            const bool on = j0 + tid < n;
+            const int u = on ? q[j0 + tid] : src;
+            if (on) cur[u >> 6] = 0ull;
+            expand(u, on, ldg_u64(&dist[u]));
+          }
+        } else {
+          words(cur, expand);
+        }
+        auto smallest = [&](unsigned long long x) {      // of the wavefront's, to s_min[sl]
+          for (int o = kWave / 2; o > 0; o >>= 1) x = min(x, __shfl_xor(x, o));
+          if (lane == 0 && x != ~0ull) atomicMin(&s_min[sl], x);
+        };
+        if (!three) smallest(kept);
+        kept = ~0ull;
+        if (lane == 0 && taken) atomicAdd(&s_redo[sl], taken);
+        if (tid == 0) { const int sn = (r + 1) % 3; s_near[sn] = 0; s_redo[sn] = 0; s_min[sn] = ~0ull; }
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __syncthreads();
+        const int got = uniform(s_redo[sl]);
+        const bool work = uniform(s_near[sl]) != 0;
+        since += got;
+        if (!work && !(three && uniform(s_far[0]))) break;
+        if (three ? !work : !got) {                      // T moves
+          if (three) {
+            // (a far node below T by now was expanded since)
+            unsigned long long m = ~0ull;
+            words(far, [&](int u, bool on, unsigned long long lab) {
+              const unsigned long long live = __ballot(on && lab >= T);
+              if (on && lab >= T) m = min(m, lab);
+              if (lane == 0) far[u >> 6] = live;
+            });
+            smallest(m);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __syncthreads();
+          }
+          const unsigned long long mn = s_min[sl];
+          if (mn == ~0ull) break;
+          if (adapt) width *= since < kPass ? 2.0 : since > 4 * kHbmBlock ? 0.5 : 1.0;
+          T = max(T, max(as_b(as_d(mn) + width), mn + 1));
+          since = 0;
+          if (three) {
+            words(far, [&](int u, bool on, unsigned long long lab) {
+              const unsigned long long later = __ballot(on && lab >= T);
+              if (lane == 0) far[u >> 6] = later;
+              int x[1] = {u};
+              bool want[1] = {on && lab < T};
+              flag(x, want);
+            });
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __syncthreads();
+          }
+        }
         if (r > 64 * N + 64) {
           if (tid == 0 && atomicCAS(&A.err[0], 0, 2) == 0) { A.err[1] = origin; A.err[2] = 0; }
           break;
         }
-        ++r;
+        unsigned long long* t = cur; cur = nxt; nxt = t;
       }
-      if (safe || !uniform(s_lost)) break;
-      __syncthreads();
     }
     n_rounds += (unsigned long long)r;
     if (A.work && tid == 0 && var == 0) A.work[origin] = r;
