@@ -522,7 +522,9 @@ struct OriginArgs {
   const double* sellw;               // [V][sell_n] sliced in-link costs
   const unsigned* sell_id;           // [sell_n] link id << 16 | tail
   const int* sell_ptr;               // [ceil(N/64) + 1] first entry of each slice
-  const struct HbmRec* hrec;         // [V][N] out-link records (labels-in-HBM kernel)
+  const struct HbmRec* hrec;         // [V][hrec_n] out-link records (labels-in-HBM kernel)
+  const struct HbmRecOf* hrec_of;    // [hrec_n]
+  int hrec_n;
   const uint2* hsell_id;             // [hsell_n] tail, link id
   const double* hsellw;              // [V][hsell_n]
   const int* hsell_ptr;
@@ -1131,7 +1133,16 @@ size_t origin_hbm_lds_bytes(int N, int hqcap) {
 // 20 us on regional, against 40 ms): the LDS kernel's records and sliced
 // in-links with 32-bit nodes and links.  A record is one 64-byte line of
 // kHrecLinks links to through nodes, self-loops left out; a node with more
-// of them has none in its record and `more` set, and is read from the CSR.
+// of them has further records behind those of the nodes, so that its links
+// come in lines too: a search takes them as entries of their own, a round
+// later.  Read from the CSR instead, two links at a time and past the table
+// that settles which label is stored, such nodes held up their wavefronts:
+// grids of 22,500 nodes with 6, 8 and 12 through links each, 200 origins, 3
+// iterations 11.5, 11.3 and 13.2 ms, and 8.5, 8.1 and 9.5 so; 90,000 nodes
+// with 8, 300 origins 66 and 22; regional, where one node in a thousand has
+// more than 5, 39.2 and 36.7 ms a loading.  (Following the records within the
+// round, the workgroup waiting for those that have more: 8.3, 7.6, 10.5, 30
+// and 39.5.)
 // The kernel has a numbering of its own: zones keep their numbers, through
 // nodes get places such that each 128-byte line of labels (16 nodes) holds
 // neighbours of each other (hbm_places).  A search's front is a ring; with
@@ -1145,38 +1156,49 @@ struct __align__(64) HbmRec {
   int more;
 };
 static_assert(sizeof(HbmRec) == 64 && kHrecLinks <= kHbmCand * kHbmGroup, "an out-link record is one 64-byte line");
+// HbmRec::more: the record that follows, whether the one after that follows
+// too (a node's further records are a row that is read as a heap: record k
+// leads to 2k + 1 and 2k + 2), and whether the row goes on
+constexpr int kHrecNext = 0x0FFFFFFF, kHrecRow = 1 << 29, kHrecTwo = 1 << 30;
+static_assert(kHbmGroup == 2, "each lane of a group follows one of the two");
+struct HbmRecOf {
+  int first, end;                    // its links: those of [first, end) to through nodes
+  int more;                          // HbmRec::more
+  int node;                          // place of its node
+};
 
-// a thread per (variant, node), and per padding lane of the last slice
+// a thread per (variant, record), and per padding lane of the last slice
 __global__ __launch_bounds__(kBlock) void k_hbm_mirrors(OriginArgs A, int Vn, HbmRec* hrec,
                                                         uint2* sell_id, double* sellw_all) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;       // place
+  const int i = blockIdx.x * kBlock + threadIdx.x;       // record; below N the place of its node
   const int N = A.N, sl = i / kWave;
-  if (sl >= (N + kWave - 1) / kWave) return;
+  const bool slice = sl < (N + kWave - 1) / kWave;
+  if (!slice && i >= A.hrec_n) return;
   const int v = i < N ? A.node[i] : -1;
-  const int begin = A.hsell_ptr[sl] + i % kWave, end = A.hsell_ptr[sl + 1];
+  const int begin = slice ? A.hsell_ptr[sl] + i % kWave : 0, end = slice ? A.hsell_ptr[sl + 1] : 0;
   for (int var = blockIdx.y; var < Vn; var += gridDim.y) {
     const double* fw = A.fww + (size_t)var * A.E;
     const double* rw = A.rvw + (size_t)var * A.E;
     double* sellw = sellw_all + (size_t)var * A.hsell_n;
     int at = begin;
-    if (v >= 0) {
+    if (i < A.hrec_n) {
+      const HbmRecOf of = A.hrec_of[i];
       HbmRec R;
       int n = 0;
 #pragma unroll
-      for (int g = 0; g < kHrecLinks; ++g) { R.w[g] = INFINITY; R.head[g] = i; }
-      for (int k = A.fw_off[v]; k < A.fw_off[v + 1]; ++k) {
+      for (int g = 0; g < kHrecLinks; ++g) { R.w[g] = INFINITY; R.head[g] = min(i, N - 1); }
+      for (int k = of.first; k < of.end; ++k) {
         const int d = A.fw_dst[k];
-        if (d < A.ft0 || d == v) continue;
+        if (d < A.ft0 || d == A.tail[k]) continue;
 #pragma unroll
         for (int g = 0; g < kHrecLinks; ++g)
           if (g == n) { R.w[g] = fw[k]; R.head[g] = A.place[d]; }
         ++n;
       }
-      R.more = n > kHrecLinks;
-      if (R.more)
-#pragma unroll
-        for (int g = 0; g < kHrecLinks; ++g) { R.w[g] = INFINITY; R.head[g] = i; }
-      hrec[(size_t)var * N + i] = R;
+      R.more = of.more;
+      hrec[(size_t)var * A.hrec_n + i] = R;
+    }
+    if (v >= 0) {
       for (int k = A.rv_off[v]; k < A.rv_off[v + 1] && at < end; ++k) {
         const int u = A.rv_src[k];
         if (v < A.ft0 || u < A.ft0 || u == v) continue;
@@ -1258,7 +1280,7 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
     const int src = A.place[origin];          // (nodes below are places, unless they come from the CSR)
     const double* __restrict__ fw = A.fww + (size_t)var * A.E;
     const double* __restrict__ rw = A.rvw + (size_t)var * A.E;
-    const char* recb = (const char*)(A.hrec + (size_t)var * N);
+    const char* recb = (const char*)(A.hrec + (size_t)var * A.hrec_n);
     const double* __restrict__ sellw = A.hsellw + (size_t)var * A.hsell_n;
     const long long clk0 = wall_clock64();
     // ---- label-correcting rounds in buckets.  Round r expands the near
@@ -1424,11 +1446,12 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         const int u = on ? (int)near_node[at] : src;
         const unsigned long long lab = on ? near_lab[at] : kMax;
         const unsigned ro = (unsigned)u * 64u;
+        // (an entry from N on is a further record of a node that was expanded)
         // (no load is masked: a merge with a default waits for each of them)
         double w[kHbmCand];
         int v[kHbmCand];
-        const unsigned long long have = ldg_u64(&dist[u]);
-        int more = *(const int*)(recb + (ro + 12u * kHrecLinks));
+        const unsigned long long seen = ldg_u64(&dist[min(u, N - 1)]), have = u < N ? seen : lab;
+        const int more = *(const int*)(recb + (ro + 12u * kHrecLinks));
 #pragma unroll
         for (int i = 0; i < kHbmCand; ++i) {
           const unsigned k = min((unsigned)(g + i * kHbmGroup), (unsigned)(kHrecLinks - 1));
@@ -1448,9 +1471,9 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         }
         bool first = on && g == 0 && have == lab;
         const unsigned long long bit = 1ull << (u & 63);
-        if (first) first = !(atomicOr(&bmA[u >> 6], bit) & bit);
+        if (first && u < N) first = !(atomicOr(&bmA[u >> 6], bit) & bit);
         const bool go = (__ballot(first) >> (lane & ~(kHbmGroup - 1))) & 1ull;
-        n_exp += first;
+        n_exp += first && u < N;
         unsigned long long cb[kHbmCand], hv[kHbmCand];
         bool low[kHbmCand];
         int slot[kHbmCand];
@@ -1472,23 +1495,21 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         for (int i = 0; i < kHbmCand; ++i)
           if (slot[i] >= 0) low[i] = tab_lab[slot[i]] == cb[i];   // else a smaller one is stored
         relax(v, cb, low, room);
-        if (!go) more = 0;
-        if (__ballot(more)) {                          // more links than the record holds
-          const int nu = A.node[u], ee = more ? A.fw_off[nu + 1] : 0;
-          for (int e = (more ? A.fw_off[nu] : 0) + g; __ballot(e < ee); e += kHbmGroup) {
-            int x[1] = {u};
-            double we = INFINITY;
-            if (e < ee) { x[0] = A.place[A.fw_dst[e]]; we = fw[e]; }
-            unsigned long long c[1] = {as_b(as_d(lab) + we)};
-            const bool ok = e < ee && x[0] >= ft0 && c[0] < kMax;
-            n_scan += ok;
-            bool lo[1] = {c[0] < (ok ? ldg_u64(&dist[x[0]]) : 0ull)};
-            relax(x, c, lo, room);
-          }
+        const bool rec = go && (g ? more & kHrecTwo : more & kHrecNext);
+        if (__ballot(rec)) {                           // the records that follow
+          int k = place(rec, &s_near[r % 3]);
+          const bool rest = rec && k >= room;
+          const int f = place(rest, &s_far[fb]);
+          if (rec && !rest) put(near_lab, near_node, to + k, lab, (more & kHrecNext) + g);
+          if (rest && f < fcap) put(far_lab, far_node, f, lab, (more & kHrecNext) + g);
+          if (rest && f >= fcap) s_wide[r & 1] = 1;
         }
       }
       // (every entry is taken: the last pass's barrier)
-      for (int j = tid; j < qn; j += kHbmBlock) bmA[near_node[from + (j < n1 ? j : qcap - 1 - (j - n1))] >> 6] = 0ull;
+      for (int j = tid; j < qn; j += kHbmBlock) {
+        const unsigned u = near_node[from + (j < n1 ? j : qcap - 1 - (j - n1))];
+        if (u < (unsigned)N) bmA[u >> 6] = 0ull;
+      }
       if (tid == 0) { s_near[(r + 1) % 3] = 0; s_redo[(r + 1) % 3] = 0; }
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // (the round's stores are done)
       __syncthreads();
@@ -1501,7 +1522,8 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
                                             : to + (k < nn ? k : qcap - 1 - (k - nn));
           const bool near = k < nn + nr;
           const unsigned long long lab = near ? near_lab[at] : far_lab[k - nn - nr];
-          const int v = (int)(near ? near_node[at] : far_node[k - nn - nr]);
+          int v = (int)(near ? near_node[at] : far_node[k - nn - nr]);
+          if (v >= N) v = A.hrec_of[v].node;
           if (k >= 0 && ldg_u64(&dist[v]) < lab) continue;   // (another entry stands for it)
           (void)__hip_atomic_fetch_min(&dist[v], lab, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
           atomicOr(&bmA[v >> 6], 1ull << (v & 63));
@@ -1518,7 +1540,7 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         unsigned long long m = ~0ull;
         for (int i = tid; i < fc; i += kHbmBlock) {
           const unsigned long long lab = far_lab[i];
-          if (weed && ldg_u64(&dist[far_node[i]]) < lab)
+          if (weed && far_node[i] < (unsigned)N && ldg_u64(&dist[far_node[i]]) < lab)
             far_lab[i] = ~0ull;
           else
             m = min(m, lab);
@@ -1665,7 +1687,8 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         flag(v, want);
       };
       auto expand = [&](int u, bool on, unsigned long long lab) {    // (all lanes)
-        const bool go = on && lab < T, keep = on && !go;
+        bool go = on && lab < T;
+        const bool keep = on && !go;
         if (__ballot(keep)) {
           if (three) {
             if (keep) { atomicOr(&far[u >> 6], 1ull << (u & 63)); s_far[0] = 1; }
@@ -1680,26 +1703,19 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         if (!m) return;
         taken += __popcll(m);
         n_exp += go;
-        if (!go) u = src;
-        const HbmRec* rec = (const HbmRec*)recb + u;
-        int x[kHrecLinks];
-        unsigned long long c[kHrecLinks], have[kHrecLinks];
-        const int more = go ? rec->more : 0;
+        for (int q = go ? u : src;;) {                   // its records
+          const HbmRec* rec = (const HbmRec*)recb + q;
+          int x[kHrecLinks];
+          unsigned long long c[kHrecLinks], have[kHrecLinks];
+          const int more = rec->more;
 #pragma unroll
-        for (int i = 0; i < kHrecLinks; ++i) { x[i] = rec->head[i]; c[i] = as_b(as_d(lab) + rec->w[i]); }
+          for (int i = 0; i < kHrecLinks; ++i) { x[i] = rec->head[i]; c[i] = as_b(as_d(lab) + rec->w[i]); }
 #pragma unroll
-        for (int i = 0; i < kHrecLinks; ++i) have[i] = ldg_u64(&dist[x[i]]);
-        lower(x, c, have, go);
-        if (__ballot(more)) {
-          int e = 0, e1 = 0;
-          if (more) { e = A.fw_off[A.node[u]]; e1 = A.fw_off[A.node[u] + 1]; }
-          for (; __ballot(e < e1); ++e) {
-            int y[1] = {u};
-            unsigned long long cy[1] = {~0ull};
-            if (e < e1) { y[0] = A.place[A.fw_dst[e]]; cy[0] = as_b(as_d(lab) + fw[e]); }
-            unsigned long long hy[1] = {ldg_u64(&dist[y[0]])};
-            lower(y, cy, hy, e < e1 && y[0] >= ft0 && y[0] != u);
-          }
+          for (int i = 0; i < kHrecLinks; ++i) have[i] = ldg_u64(&dist[x[i]]);
+          lower(x, c, have, go);
+          go = go && more & kHrecRow;
+          if (!__ballot(go)) break;
+          if (go) q = q < N ? more & kHrecNext : q + 1;
         }
       };
       for (++r;; ++r) {
@@ -2498,7 +2514,9 @@ struct tapgpu_ctx {
   // the LDS kernel's mirrors of the graph and the costs
   double *rec = nullptr, *sellw = nullptr;
   int *recpos = nullptr, *sellpos = nullptr, *sell_ptr = nullptr;
-  HbmRec* hrec = nullptr;             // the labels-in-HBM kernel's mirrors (ensure_hbm_mirrors)
+  HbmRec* hrec = nullptr;             // the labels-in-HBM kernel's mirrors (alloc_hbm_mirrors)
+  HbmRecOf* hrec_of = nullptr;
+  int hrec_n = 0;
   uint2* hsell_id = nullptr;
   double* hsellw = nullptr;
   int* hplace = nullptr;              // [N] place of a node | [N] node of a place | slices
@@ -2916,7 +2934,7 @@ OriginArgs make_origin_args(tapgpu_ctx* c, const unsigned char* var_on) {
   A.rv_eid = c->rv_eid; A.tail = c->tail; A.fww = c->fww; A.rvw = c->rvw;
   A.rec = c->rec; A.sellw = c->sellw; A.sell_id = c->sell_id; A.sell_ptr = c->sell_ptr;
   A.sell_n = c->sell_n;
-  A.hrec = c->hrec; A.hsell_id = c->hsell_id; A.hsellw = c->hsellw; A.hsell_n = c->hsell_n;
+  A.hrec = c->hrec; A.hrec_of = c->hrec_of; A.hrec_n = c->hrec_n; A.hsell_id = c->hsell_id; A.hsellw = c->hsellw; A.hsell_n = c->hsell_n;
   A.place = c->hplace; A.node = c->hplace + c->N; A.hsell_ptr = c->hplace + 2 * (size_t)c->N;
   A.od_start = c->od_start; A.od_dest = c->od_dest; A.od_val = c->od_val;
   A.var_on = var_on; A.y = c->y; A.err = c->err_dev; A.counters = c->counters;
@@ -2936,7 +2954,7 @@ void advance_variant(tapgpu_ctx* c, OriginArgs& A, int64_t v) {
   A.fww += (size_t)v * c->E;
   A.rvw += (size_t)v * c->E;
   if (c->hrec) {
-    A.hrec += (size_t)v * c->N;
+    A.hrec += (size_t)v * c->hrec_n;
     A.hsellw += (size_t)v * c->hsell_n;
   }
   if (c->rec) {
@@ -3341,9 +3359,31 @@ int alloc_hbm_mirrors(tapgpu_ctx* c) try {
   }
   for (int i = 0; i < W; ++i) ptr[i + 1] = ptr[i] + ptr[i + 1] * kWave;
   c->hsell_n = ptr[W];
+  // a node's records: the first at its place, further ones in a row behind
+  // all places
+  std::vector<HbmRecOf> of(N);
+  for (int i = 0; i < N; ++i) {
+    const int v = h[(size_t)N + i], base = (int)of.size() - 1;
+    int at = i, n = 0;
+    of[i] = {off[v], off[v + 1], 0, i};
+    for (int k = off[v]; k < off[v + 1]; ++k) {
+      if (dst[k] < c->ft0 || dst[k] == v || n++ < kHrecLinks) continue;
+      n = 1;
+      of[at].end = k;
+      at = (int)of.size();
+      of.push_back({k, off[v + 1], 0, i});
+    }
+    const int m = (int)of.size() - 1 - base;           // records after the first
+    for (int k = 0; k <= m; ++k)
+      of[k ? base + k : i].more = (2 * k + 1 <= m ? base + 2 * k + 1 : 0) | (2 * k + 2 <= m ? kHrecTwo : 0) |
+                                  (k < m ? kHrecRow : 0);
+  }
+  c->hrec_n = (int)of.size();
   int rc;
   if (!c->hplace && (rc = dalloc(c, &c->hplace, h.size()))) return rc;
-  if (!c->hrec && (rc = dalloc(c, &c->hrec, (size_t)c->V * N))) return rc;
+  if (!c->hrec_of && (rc = dalloc(c, &c->hrec_of, of.size()))) return rc;
+  if ((rc = upload(c, c->hrec_of, of.data(), of.size()))) return rc;
+  if (!c->hrec && (rc = dalloc(c, &c->hrec, (size_t)c->V * c->hrec_n))) return rc;
   if (!c->hsell_id && (rc = dalloc(c, &c->hsell_id, (size_t)c->hsell_n))) return rc;
   if ((rc = upload(c, c->hplace, h.data(), h.size()))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -3355,7 +3395,7 @@ int alloc_hbm_mirrors(tapgpu_ctx* c) try {
 // Before a launch of the labels-in-HBM kernel: the mirrors of Vn variants
 // (A is advanced to the first), on the context's stream.
 void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn) {
-  const int nodes = (c->N + kWave - 1) / kWave * kWave;
+  const int nodes = std::max((c->N + kWave - 1) / kWave * kWave, c->hrec_n);
   hipLaunchKernelGGL(k_hbm_mirrors, dim3((nodes + kBlock - 1) / kBlock, std::min(Vn, 65535)), dim3(kBlock), 0,
                      c->stream, A, Vn, const_cast<HbmRec*>(A.hrec), const_cast<uint2*>(A.hsell_id),
                      const_cast<double*>(A.hsellw));
