@@ -284,3 +284,34 @@ def test_hbm_kernel_queues_and_records(engine_mod, N, ft, hub, kind):
                 assert np.array_equal(d.view(np.int64), d0.view(np.int64)), (q, width)
                 assert np.array_equal(p, p0), (q, width)
                 assert np.array_equal(eng.aon().view(np.int64), y0.view(np.int64)), (q, width)
+
+
+def test_lds_kernel_looks_at_a_link_once(engine_mod, oracle_lib):
+    """Nodes with more links than a record holds: an expansion relaxes each
+    of the node's eight links once."""
+    import oracle
+    print("case lds links once", flush=True)
+    from traffic_assignment_amd import synth
+    rng = np.random.default_rng(8)
+    N, Z, degree = 2000, 30, 8
+    init = np.repeat(np.arange(1, N + 1), degree)
+    term = rng.integers(1, N + 1, init.size)
+    term[::degree] = np.roll(np.arange(1, N + 1), -1)
+    order = np.lexsort((term, init))
+    E = init.size
+    net = synth.Network(num_zones=Z, num_nodes=N, first_thru_node=1, init=init[order], term=term[order],
+                        capacity=np.full(E, 100.0), length=np.ones(E), fftime=rng.uniform(0.5, 3.0, E),
+                        B=np.full(E, 0.15), power=np.full(E, 4.0), speed=np.zeros(E), toll=np.zeros(E),
+                        ltype=np.ones(E, np.int16))
+    origins = np.arange(1, Z + 1)
+    od, _ = oracle.sssp_all(net, net.fftime)
+    with engine_mod.TapEngine(net, random_demand(net, rng)) as eng:
+        eng.set_strategy("lds")
+        eng.aon()
+        a = eng.stats()
+        eng.aon()
+        b = eng.stats()
+        d, _ = eng.sssp(origins)
+    assert np.array_equal(d[1:].view(np.int64), od[1:].view(np.int64))
+    n = {k: b[k] - a[k] for k in ("origin_scanned", "origin_expansions")}
+    assert 0 < n["origin_scanned"] <= degree * n["origin_expansions"]
