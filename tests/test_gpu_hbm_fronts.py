@@ -107,3 +107,42 @@ def test_hbm_nodes_beyond_a_record(engine_mod, degree):
                 eng.set_origin_delta(width)
                 _both(eng, net.fftime, starts)
                 _both(eng, np.floor(net.fftime * 2.0), starts)           # level ties
+
+
+def test_hbm_batch_memory_and_parts(engine_mod):
+    """A batch beyond LDS: creation holds the mirrors of one variant (its
+    loadings usually run on the lanes kernel); loadings by the labels-in-HBM
+    kernel of more variants than 512 MiB of mirrors hold go by parts, and the
+    free-flow volumes of variants on both sides of a part's end are those of
+    the variant alone."""
+    import torch
+    from traffic_assignment_amd import synth
+    print("case hbm batch parts", flush=True)
+    N, Z, V = 60000, 4, 115
+    net, rng = random_graph(N, 1, Z, 3)                  # 4.8 MB of mirrors a variant: 111 in a part
+    st = np.arange(Z + 1) * (Z - 1)
+    dest = np.concatenate([[d for d in range(1, Z + 1) if d != o] for o in range(1, Z + 1)])
+    dem = synth.Demand(Z, st, dest, np.arange(1.0, dest.size + 1.0))
+    E = net.num_links
+    t0 = rng.uniform(0.5, 3.0, (V, E))
+
+    def used():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    before = used()
+    with engine_mod.TapEngine(net, dem, num_variants=V, fftime=t0) as eng:
+        # nine arrays of doubles and one of bytes per link and variant, sums of the line search
+        assert used() - before <= 1.05 * V * (73 * E + 65536) + (64 << 20)
+        eng.set_lanes(0)
+        eng.fw_init()
+        x = {v: eng.flows(v)[0] for v in (0, 57, 109, 110, 111, 112, 114)}
+        eng.fw_run(max_iters=2)                          # (captured, in parts)
+        x2 = {v: eng.flows(v)[0] for v in x}
+    for v in x:
+        with engine_mod.TapEngine(net, dem, num_variants=1, fftime=t0[v:v + 1]) as one:
+            one.fw_init()
+            assert np.array_equal(one.flows()[0], x[v]), v
+            one.fw_run(max_iters=2)
+            assert np.array_equal(one.flows()[0], x2[v]), v

@@ -522,11 +522,11 @@ struct OriginArgs {
   const double* sellw;               // [V][sell_n] sliced in-link costs
   const unsigned* sell_id;           // [sell_n] link id << 16 | tail
   const int* sell_ptr;               // [ceil(N/64) + 1] first entry of each slice
-  const struct HbmRec* hrec;         // [V][hrec_n] out-link records (labels-in-HBM kernel)
+  const struct HbmRec* hrec;         // [variants of the launch][hrec_n] out-link records (labels-in-HBM kernel)
   const struct HbmRecOf* hrec_of;    // [hrec_n]
   int hrec_n;
   const uint2* hsell_id;             // [hsell_n] tail, link id
-  const double* hsellw;              // [V][hsell_n]
+  const double* hsellw;              // [variants of the launch][hsell_n]
   const int* hsell_ptr;
   long long hsell_n;
   const int *place, *node;           // its numbering: node -> place, place -> node
@@ -2516,6 +2516,7 @@ struct tapgpu_ctx {
   double *rec = nullptr, *sellw = nullptr;
   int *recpos = nullptr, *sellpos = nullptr, *sell_ptr = nullptr;
   HbmRec* hrec = nullptr;             // the labels-in-HBM kernel's mirrors (alloc_hbm_mirrors)
+  int hvars = 0, hvars_max = INT_MAX; // variants they hold, and may hold
   HbmRecOf* hrec_of = nullptr;
   int hrec_n = 0;
   uint2* hsell_id = nullptr;
@@ -2712,6 +2713,12 @@ int balloc(tapgpu_ctx* ctx, T** p, size_t n) {
   ctx->block_at += bytes;
   ctx->block_left -= bytes;
   return TAPGPU_OK;
+}
+
+void dfree(tapgpu_ctx* ctx, void* p) {
+  if (!p) return;
+  ctx->allocs.erase(std::remove(ctx->allocs.begin(), ctx->allocs.end(), p), ctx->allocs.end());
+  (void)hipFree(p);
 }
 
 template <class T>
@@ -2950,18 +2957,23 @@ OriginArgs make_origin_args(tapgpu_ctx* c, const unsigned char* var_on) {
   return A;
 }
 
-// The cost arrays of A moved to variant v (the kernels' variant 0).
+// The cost arrays of A moved to variant v (the kernels' variant 0; the
+// labels-in-HBM kernel's mirrors are those of a launch's variants).
 void advance_variant(tapgpu_ctx* c, OriginArgs& A, int64_t v) {
   A.fww += (size_t)v * c->E;
   A.rvw += (size_t)v * c->E;
-  if (c->hrec) {
-    A.hrec += (size_t)v * c->hrec_n;
-    A.hsellw += (size_t)v * c->hsell_n;
-  }
   if (c->rec) {
     A.rec += (size_t)v * c->N * kRecDoubles;
     A.sellw += (size_t)v * c->sell_n;
   }
+}
+
+// Arguments of a loading of the variants from v on.
+OriginArgs variant_args(tapgpu_ctx* c, const unsigned char* var_on, int v) {
+  OriginArgs A = make_origin_args(c, var_on ? var_on + v : nullptr);
+  advance_variant(c, A, v);
+  A.y += (size_t)v * c->E;
+  return A;
 }
 
 // (before any capture too: a replay takes the mirrors as the passes keep them)
@@ -2998,8 +3010,8 @@ void launch_lds(tapgpu_ctx* c, dim3 grid, hipStream_t st, const OriginArgs& A, i
 constexpr int kChaseCandidates[] = {0, 2, 4, 8, 16, 32};
 constexpr int kTuneBlocks = 4096;              // workgroups of a tuning launch on a batch
 
-int ensure_hbm(tapgpu_ctx* c);
-void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn);
+int ensure_hbm(tapgpu_ctx* c, int Vn);
+void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn, hipStream_t st);
 
 // Per-origin round counts of the recording loading (zeroed: origins a
 // loading skips keep 0 and go last).
@@ -3020,18 +3032,11 @@ int launch_origin(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, fl
   if (!c->pre_cleared)
     HIPCHK(c, hipMemsetAsync(c->y + (size_t)v0 * c->E, 0, sizeof(double) * (size_t)Vn * c->E, c->stream));
   if (c->Z > 0) {
-    OriginArgs A = make_origin_args(c, var_on);
-    advance_variant(c, A, v0); A.y += (size_t)v0 * c->E;
-    if (var_on) A.var_on = var_on + v0;
     const int zh = (c->hbm_ok && c->split > 0) ? std::min(c->split, c->Z - 1) : 0;
     const int zl = c->Z - zh;
-    if (zh > 0) {
-      int rc = ensure_hbm(c);
-      if (rc) return rc;
-      A = make_origin_args(c, var_on);            // (with what ensure_hbm has made)
-      advance_variant(c, A, v0); A.y += (size_t)v0 * c->E;
-      if (var_on) A.var_on = var_on + v0;
-    }
+    if (zh > 0)
+      if (int rc = ensure_hbm(c, Vn)) return rc;
+    OriginArgs A = variant_args(c, var_on, v0);
     if (zh == 0) {
       if (c->origin_order_ready) {
         A.src_list = c->d_origin_order;
@@ -3046,18 +3051,18 @@ int launch_origin(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, fl
     }
     if (ms) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
     if (zh > 0) {
-      launch_hbm_mirrors(c, A, Vn);
       HIPCHK(c, hipEventRecord(c->ev_fork, c->stream));
       HIPCHK(c, hipStreamWaitEvent(c->stream2, c->ev_fork, 0));
-      OriginArgs B = A;
-      B.z0 = zl;
-      B.zn = zh;
-      B.src_list = nullptr;
-      B.work = nullptr;
-      const int items = zh * Vn;
-      hipLaunchKernelGGL(k_origin_hbm, dim3(std::min(c->hbm_grid, items)), dim3(kHbmBlock),
-                         c->hbm_lds, c->stream2, B, 1, items);
-      HIPCHK(c, hipGetLastError());
+      for (int v = 0; v < Vn; v += c->hvars) {
+        const int n = std::min(c->hvars, Vn - v), items = zh * n;
+        OriginArgs B = variant_args(c, var_on, v0 + v);
+        B.z0 = zl;
+        B.zn = zh;
+        launch_hbm_mirrors(c, B, n, c->stream2);
+        hipLaunchKernelGGL(k_origin_hbm, dim3(std::min(c->hbm_grid, items)), dim3(kHbmBlock),
+                           c->hbm_lds, c->stream2, B, 1, items);
+        HIPCHK(c, hipGetLastError());
+      }
       HIPCHK(c, hipEventRecord(c->ev_join, c->stream2));
     }
     launch_lds(c, dim3(zl, Vn), c->stream, A, 1);
@@ -3334,10 +3339,40 @@ void hbm_places(int N, int ft0, const std::vector<int>& off, const std::vector<i
   }
 }
 
-// The labels-in-HBM kernel's mirrors: made with the context where its labels
-// do not fit LDS, otherwise when the kernel is chosen or first runs.
-int alloc_hbm_mirrors(tapgpu_ctx* c) try {
-  if (c->hsellw) return TAPGPU_OK;
+// The labels-in-HBM kernel's mirrors, of Vn variants or of as many as
+// kHbmMirrorBytes hold: launches over more variants go by parts (58 variants
+// of regional are 232,000 items, for 512 workgroups).  Those of one variant
+// are made with the context where its labels do not fit LDS, since
+// tapgpu_sssp_noalloc allocates nothing, otherwise when the kernel is chosen
+// or first runs; a batch that only the lanes kernel loads holds no more (512
+// variants of regional: 5 GB).  They grow before an iteration is captured.
+constexpr size_t kHbmMirrorBytes = 512ull << 20;
+
+int alloc_hbm_mirrors(tapgpu_ctx* c, int Vn) try {
+  auto grow = [&]() -> int {
+    const size_t each = sizeof(HbmRec) * (size_t)c->hrec_n + sizeof(double) * (size_t)c->hsell_n;
+    const int most = std::min<int>(c->hvars_max, (int)std::max<size_t>(1, kHbmMirrorBytes / each));
+    for (int n = std::min(Vn, most); n > c->hvars; n /= 2) {
+      HbmRec* rec = nullptr;
+      double* w = nullptr;
+      int rc = dalloc(c, &rec, (size_t)n * c->hrec_n);
+      if (!rc && (rc = dalloc(c, &w, (size_t)n * c->hsell_n))) dfree(c, rec);
+      if (rc && (n == 1 || rc != TAPGPU_E_NOMEM)) return rc;
+      if (rc) {                                        // with fewer at a time, then and later
+        c->hvars_max = std::max(1, n / 2);
+        continue;
+      }
+      HIPCHK(c, hipStreamSynchronize(c->stream));
+      dfree(c, c->hrec);
+      dfree(c, c->hsellw);
+      c->hrec = rec;
+      c->hsellw = w;
+      c->hvars = n;
+      break;
+    }
+    return TAPGPU_OK;
+  };
+  if (c->hvars) return grow();
   const int N = c->N, W = (N + kWave - 1) / kWave;
   std::vector<int> off(N + 1), dst(c->E), roff(N + 1), rsrc(c->E);
   auto get = [&](std::vector<int>& h, const int* d) {
@@ -3384,28 +3419,27 @@ int alloc_hbm_mirrors(tapgpu_ctx* c) try {
   if (!c->hplace && (rc = dalloc(c, &c->hplace, h.size()))) return rc;
   if (!c->hrec_of && (rc = dalloc(c, &c->hrec_of, of.size()))) return rc;
   if ((rc = upload(c, c->hrec_of, of.data(), of.size()))) return rc;
-  if (!c->hrec && (rc = dalloc(c, &c->hrec, (size_t)c->V * c->hrec_n))) return rc;
   if (!c->hsell_id && (rc = dalloc(c, &c->hsell_id, (size_t)c->hsell_n))) return rc;
   if ((rc = upload(c, c->hplace, h.data(), h.size()))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  return dalloc(c, &c->hsellw, (size_t)c->V * c->hsell_n);
+  return grow();
 } catch (const std::bad_alloc&) {
   return c->fail(TAPGPU_E_NOMEM, "out of host memory for the node numbering");
 }
 
 // Before a launch of the labels-in-HBM kernel: the mirrors of Vn variants
-// (A is advanced to the first), on the context's stream.
-void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn) {
+// (A is advanced to the first, and hvars holds them).
+void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn, hipStream_t st) {
   const int nodes = std::max((c->N + kWave - 1) / kWave * kWave, c->hrec_n);
   hipLaunchKernelGGL(k_hbm_mirrors, dim3((nodes + kBlock - 1) / kBlock, std::min(Vn, 65535)), dim3(kBlock), 0,
-                     c->stream, A, Vn, const_cast<HbmRec*>(A.hrec), const_cast<uint2*>(A.hsell_id),
+                     st, A, Vn, const_cast<HbmRec*>(A.hrec), const_cast<uint2*>(A.hsell_id),
                      const_cast<double*>(A.hsellw));
 }
 
 // Per-workgroup scratch rows of the labels-in-HBM kernel (allocated on
 // first use: hbm_grid rows of N labels, predecessors and tails).
-int ensure_hbm(tapgpu_ctx* c) {
-  if (int rc = alloc_hbm_mirrors(c)) return rc;
+int ensure_hbm(tapgpu_ctx* c, int Vn) {
+  if (int rc = alloc_hbm_mirrors(c, Vn)) return rc;
   if (c->h_dist) return TAPGPU_OK;
   const size_t n = (size_t)c->hbm_grid * c->N;
   int rc;
@@ -3434,29 +3468,33 @@ int launch_hbm(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, int i
   if (!c->pre_cleared)
     HIPCHK(c, hipMemsetAsync(c->y + (size_t)v0 * c->E, 0, sizeof(double) * (size_t)Vn * c->E, c->stream));
   if (c->Z == 0) return TAPGPU_OK;
-  if (int rc = ensure_hbm(c)) return rc;        // (no allocation once made)
-  OriginArgs A = make_origin_args(c, var_on);
-  advance_variant(c, A, v0); A.y += (size_t)v0 * c->E;
-  if (var_on) A.var_on = var_on + v0;
-  const int items = std::min(c->Z * Vn, items_cap);
-  const int G = std::min(c->hbm_grid, items);
-  launch_hbm_mirrors(c, A, Vn);
-  if (c->origin_order_ready) {
-    A.order = c->d_origin_order;
-    A.vn = Vn;
-  } else if (!c->capturing && c->Z > 1) {
+  if (int rc = ensure_hbm(c, Vn)) return rc;    // (no allocation once made)
+  int* work = nullptr;
+  if (!c->origin_order_ready && !c->capturing && c->Z > 1) {
     if (!c->d_origin_work) {
       int rc = ensure_origin_work(c);
       if (rc) return rc;
     }
-    A.work = c->d_origin_work;
+    work = c->d_origin_work;
     c->origin_recorded = true;
   }
-  A.next = c->d_hbm_next;
-  hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, c->stream, c->d_hbm_next);
   if (ms) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
-  hipLaunchKernelGGL(k_origin_hbm, dim3(G), dim3(kHbmBlock), c->hbm_lds, c->stream, A, 1, items);
-  HIPCHK(c, hipGetLastError());
+  for (int v = 0; v < Vn && items_cap > 0; v += c->hvars) {
+    const int n = std::min(c->hvars, Vn - v), items = std::min(c->Z * n, items_cap);
+    items_cap -= items;
+    OriginArgs A = variant_args(c, var_on, v0 + v);
+    if (c->origin_order_ready) {
+      A.order = c->d_origin_order;
+      A.vn = n;
+    }
+    A.work = work;
+    A.next = c->d_hbm_next;
+    launch_hbm_mirrors(c, A, n, c->stream);
+    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, c->stream, c->d_hbm_next);
+    hipLaunchKernelGGL(k_origin_hbm, dim3(std::min(c->hbm_grid, items)), dim3(kHbmBlock), c->hbm_lds, c->stream,
+                       A, 1, items);
+    HIPCHK(c, hipGetLastError());
+  }
   if (ms) {
     HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
     HIPCHK(c, hipEventSynchronize(c->ev[1]));
@@ -3505,7 +3543,7 @@ int tune_delta(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
 
 int aon_hbm(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
   auto t0 = std::chrono::steady_clock::now();
-  int rc = ensure_hbm(c);
+  int rc = ensure_hbm(c, Vn);
   if (rc) return rc;
   if ((rc = origin_order_update(c))) return rc;
   if (!c->pre_cleared) HIPCHK(c, hipMemsetAsync(c->err_dev, 0, sizeof(int) * 3, c->stream));
@@ -3948,7 +3986,7 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
   if ((rc = upload(c, c->present, hpres.data(), VE))) return rc;
   if ((rc = upload(c, c->col_src, col_src.data(), c->P))) return rc;
   if ((rc = upload(c, c->grp_var, grp_var.data(), c->Galloc))) return rc;
-  if (!c->lds_ok && c->hbm_ok && (rc = alloc_hbm_mirrors(c))) return rc;   // (tapgpu_sssp_noalloc allocates nothing)
+  if (!c->lds_ok && c->hbm_ok && (rc = alloc_hbm_mirrors(c, 1))) return rc;   // (tapgpu_sssp_noalloc allocates nothing)
   if (c->lds_ok) {
     if ((rc = upload(c, c->sell_ptr, sell_ptr.data(), sell_ptr.size()))) return rc;
     hipLaunchKernelGGL(k_mirrors, dim3((W * kWave + kBlock - 1) / kBlock), dim3(kBlock), 0, c->stream,
@@ -4093,7 +4131,7 @@ int tapgpu_sssp(tapgpu_ctx* c, int64_t variant, const int64_t* start_nodes, int6
     // one workgroup per start node (labels in LDS), or the persistent
     // labels-in-HBM grid; chunks of up to 1024 starts
     const bool hbm = !use_lds(c);
-    if (hbm && (rc = ensure_hbm(c))) return rc;
+    if (hbm && (rc = ensure_hbm(c, 1))) return rc;
     const int64_t chunk = std::min<int64_t>(std::max<int64_t>(num_start, 1), 1024);
     SsspStage S;
     rc = stage_sssp(c, chunk, &S);
@@ -4106,7 +4144,7 @@ int tapgpu_sssp(tapgpu_ctx* c, int64_t variant, const int64_t* start_nodes, int6
       hipLaunchKernelGGL(k_sssp_begin, dim3(grid_for((long long)c->N * ns / kWave + 1)), dim3(kBlock), 0,
                          c->stream, S.pred, (long long)c->N * ns, S.err);
       if (hbm) {
-        if (s0 == 0) launch_hbm_mirrors(c, A, 1);
+        if (s0 == 0) launch_hbm_mirrors(c, A, 1, c->stream);
         hipLaunchKernelGGL(k_origin_hbm, dim3(std::min(ns, c->hbm_grid)), dim3(kHbmBlock), c->hbm_lds,
                            c->stream, A, 0, ns);
       } else
@@ -4282,7 +4320,7 @@ int tapgpu_sssp_noalloc(tapgpu_ctx* c, int64_t variant, const int64_t* d_start_n
   if (lds) {
     launch_lds(c, dim3((unsigned)num_start, 1), c->stream, A, 0);
   } else {
-    launch_hbm_mirrors(c, A, 1);
+    launch_hbm_mirrors(c, A, 1, c->stream);
     hipLaunchKernelGGL(k_origin_hbm, dim3((unsigned)std::min<int64_t>(num_start, rows)),
                        dim3(kHbmBlock), c->hbm_lds, c->stream, A, 0, (int)num_start);
   }
@@ -4442,7 +4480,7 @@ static int capture(tapgpu_ctx* c, hipGraphExec_t* exec, F&& issue) {
 static int iter_graph(tapgpu_ctx* c, const Links& K, int m) {
   const bool lds = use_lds(c);
   if (!lds) {
-    int rc = ensure_hbm(c);
+    int rc = ensure_hbm(c, c->V);
     if (rc) return rc;
   }
   long long dbits;
@@ -4837,7 +4875,7 @@ int tapgpu_set_strategy(tapgpu_ctx* c, int strategy) {
   c->strategy = strategy;
   // (tapgpu_sssp_noalloc allocates nothing, and takes this kernel then)
   if (!use_lds(c) && c->hbm_ok)
-    if (int rc = alloc_hbm_mirrors(c)) {
+    if (int rc = alloc_hbm_mirrors(c, 1)) {
       c->strategy = before;
       return rc;
     }
