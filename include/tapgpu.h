@@ -346,7 +346,8 @@ double tapgpu_get_lanes_delta(const tapgpu_ctx *ctx);
    launch and the synchronisation are paid once for several.  mode = 2..8:
    that many iterations per replay on those paths.  Networks of up to 192
    nodes, 1,024 links and 64 zones whose powers are all 4 run up to 256
-   iterations (and tapgpu_fw_init's loading) inside one kernel instead, with
+   iterations (and tapgpu_fw_init's loading) inside one kernel instead where
+   their nodes, zones, in-links and variants make it the faster form, with
    the LDS strategy and the default link passes, unless the lanes kernel was
    asked for (tapgpu_set_lanes).  mode = 0: the same launches issued one by
    one.  Profiling (tapgpu_set_profiling) issues them one by one too, so the

@@ -315,3 +315,79 @@ def test_lds_kernel_looks_at_a_link_once(engine_mod, oracle_lib):
     assert np.array_equal(d[1:].view(np.int64), od[1:].view(np.int64))
     n = {k: b[k] - a[k] for k in ("origin_scanned", "origin_expansions")}
     assert 0 < n["origin_scanned"] <= degree * n["origin_expansions"]
+
+
+def grid_network(rows, cols, Z, diagonals, power=4.0):
+    """A grid of through nodes whose first Z are zones, with both diagonals of
+    every square or none: up to 4 or 8 links into a node."""
+    from traffic_assignment_amd import synth
+    rng = np.random.default_rng(rows * cols + Z)
+    i = 1 + np.arange(rows * cols).reshape(rows, cols)
+    pairs = [(i[:, :-1], i[:, 1:]), (i[:-1], i[1:])]
+    if diagonals:
+        pairs += [(i[:-1, :-1], i[1:, 1:]), (i[:-1, 1:], i[1:, :-1])]
+    a = np.concatenate([p.ravel() for p, _ in pairs])
+    b = np.concatenate([q.ravel() for _, q in pairs])
+    init, term = np.concatenate([a, b]), np.concatenate([b, a])
+    order = np.lexsort((term, init))
+    E = init.size
+    pw = np.full(E, 4.0)
+    pw[0] = power
+    net = synth.Network(num_zones=Z, num_nodes=rows * cols, first_thru_node=1, init=init[order],
+                        term=term[order], capacity=rng.uniform(20.0, 200.0, E), length=np.ones(E),
+                        fftime=rng.uniform(0.5, 3.0, E), B=np.full(E, 0.15), power=pw, speed=np.zeros(E),
+                        toll=np.zeros(E), ltype=np.ones(E, np.int16))
+    return net, rng
+
+
+@pytest.mark.parametrize("rows,cols,Z,diagonals,V,power,one", [
+    (4, 6, 24, 0, 1, 4.0, True), (4, 8, 32, 1, 1, 4.0, True), (8, 8, 64, 0, 1, 4.0, True),
+    (8, 8, 16, 1, 1, 4.0, True), (9, 11, 16, 0, 1, 4.0, True), (13, 14, 16, 0, 1, 4.0, True),
+    (13, 14, 64, 0, 64, 4.0, True), (9, 11, 48, 1, 64, 4.0, True),
+    (13, 14, 64, 0, 1, 4.0, False), (9, 11, 16, 1, 1, 4.0, False), (8, 8, 48, 1, 1, 4.0, False),
+    (12, 12, 60, 1, 1, 4.0, False), (9, 11, 48, 1, 4, 4.0, False), (14, 14, 8, 0, 1, 4.0, False),
+    (4, 6, 24, 0, 1, 3.0, False), (4, 6, 24, 0, 3, 2.5, False)])
+def test_one_workgroup_kernel_where_it_pays(engine_mod, rows, cols, Z, diagonals, V, power, one):
+    """Which form the iterations take (replays of a graph are counted, the
+    one kernel's launches are not), and that both give the same."""
+    print(f"case one-workgroup choice {rows}x{cols} Z={Z} diag={diagonals} V={V} p={power}", flush=True)
+    net, rng = grid_network(rows, cols, Z, diagonals, power)
+    dem = random_demand(net, rng)
+    kw = {}
+    if V > 1:
+        kw = dict(num_variants=V, capacity=net.capacity * rng.uniform(0.8, 1.25, (V, net.num_links)))
+    out = []
+    for graphs in (1, 0):
+        with engine_mod.TapEngine(net, dem, **kw) as eng:
+            eng.set_graphs(graphs)
+            eng.fw_init()
+            eng.fw_run(max_iters=12)
+            n = eng.stats()["graph_launches"]
+            assert (n == 0) == (one or not graphs), n
+            out.append(([eng.flows(v) for v in range(V)], [eng.trace(v) for v in range(V)]))
+    _same(*out)
+
+
+@pytest.mark.parametrize("N,Z,ft,extra", [(31, 8, 9, 31), (33, 10, 11, 33), (64, 16, 1, 64), (65, 30, 31, 30),
+                                          (128, 17, 1, 60), (129, 40, 41, 50), (192, 32, 33, 60)])
+@pytest.mark.parametrize("kind", ["cont", "ints"])
+def test_one_workgroup_batches(engine_mod, N, Z, ft, extra, kind):
+    """64 variants, for which the one kernel is the faster form with more
+    nodes and in-links too: zones that are no through nodes, level ties, one
+    to three nodes a lane and several origins a wavefront."""
+    print(f"case one-workgroup batch N={N} Z={Z} ft={ft} {kind}", flush=True)
+    net, rng = small_network(5 * N, N, Z, ft, extra, kind)
+    dem = random_demand(net, rng)
+    V = 64
+    cap = net.capacity * rng.uniform(0.8, 1.25, (V, net.num_links))
+    out = []
+    for graphs in (1, 0):
+        with engine_mod.TapEngine(net, dem, num_variants=V, capacity=cap) as eng:
+            eng.set_graphs(graphs)
+            eng.fw_init()
+            x = [eng.flows(v) for v in range(V)]
+            eng.fw_run(max_iters=6)
+            if graphs:                                 # (every other form replays graphs)
+                assert eng.stats()["graph_launches"] == 0
+            out.append((x + [eng.flows(v) for v in range(V)], [eng.trace(v) for v in range(V)]))
+    _same(*out)

@@ -2632,7 +2632,7 @@ struct tapgpu_ctx {
   int lanes_min = 0;                  // active variants needed to use it (0: never)
   bool lanes_auto = true;             // lanes_min is the default
   int cus = 0;                        // compute units of the device
-  bool tiny_ok = false;               // the one-workgroup kernel holds this network
+  bool tiny_ok = false;               // the one-workgroup kernel holds this network, and is the faster one
   bool lanes_ok = false;              // its LDS (bitmaps + queues) fits
   int lanes_qcap = 0;                 // LDS frontier queue entries per round
   int lanes_qcap_max = 0;             // entries its LDS allocation holds
@@ -3819,10 +3819,6 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
       c->qcap = c->qcap_max;
       c->lds_bytes = origin_lds_bytes(c->N, c->qcap_max);
     }
-    bool pow4 = true;
-    for (int64_t j = 0; j < (pw_v ? V * E : E); ++j) pow4 = pow4 && (pw_v ? pw_v : net->power)[j] == 4.0;
-    c->tiny_ok = c->lds_ok && pow4 && tiny_fits(c->N, c->E, c->Z) &&
-                 tiny_lds_bytes(c->N, c->E) + 128 <= (size_t)lds_max;
     // (the networks it takes: 24 bytes of LDS for 64 nodes)
     c->hbm_ok = 24 * (((size_t)N + 63) / 64) + 256 <= (size_t)lds_max;
     if (c->hbm_ok) {
@@ -3841,6 +3837,17 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
     int ncu = 0, per_cu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) ncu = 1;
     c->cus = ncu;
+    if (c->lds_ok && tiny_fits(c->N, c->E, c->Z) && tiny_lds_bytes(c->N, c->E) + 128 <= (size_t)lds_max) {
+      int in = 0, zone_in = 0;                    // most in-links of a through node (that count) and of a zone
+      for (int v = 0; v < c->N; ++v) {
+        int n = 0;
+        for (int k = rv_off[v]; k < rv_off[v + 1]; ++k) n += v < c->ft0 || (rv_src[k] >= c->ft0 && rv_src[k] != v);
+        (v < c->ft0 ? zone_in : in) = std::max(v < c->ft0 ? zone_in : in, n);
+      }
+      bool pow4 = true;
+      for (int64_t j = 0; j < (pw_v ? V * E : E); ++j) pow4 = pow4 && (pw_v ? pw_v : net->power)[j] == 4.0;
+      c->tiny_ok = pow4 && tiny_pays(c->N, c->Z, in, zone_in, c->V, ncu);
+    }
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_origin_hbm, kHbmBlock, c->hbm_lds) !=
         hipSuccess || per_cu < 1)
       per_cu = 1;
