@@ -750,8 +750,9 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
     if (__builtin_expect(h & kRecMore, 0)) {          // more out-links than lanes
       if (h & kRecCsr) {                              // ... than the record holds
         // (the first kGroup links of the CSR are among those just relaxed)
-        const int ee = A.fw_off[u + 1];
-        for (int e = A.fw_off[u] + kGroup + (int)g; e < ee; e += kGroup) {
+        const int ee = A.fw_off[u + 1] - kGroup;
+        for (int e0 = A.fw_off[u] + (int)g; e0 < ee; e0 += kGroup) {
+          const int e = e0 + kGroup;
           const int v = A.fw_dst[e];
           if (v < ft0) continue;
           ++n_scan;
