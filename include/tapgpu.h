@@ -359,7 +359,9 @@ int tapgpu_get_graphs(tapgpu_ctx *ctx, int *mode);
    the reference).  0 (the default): networks of up to 512 links run all of
    an iteration's link work in one launch, one workgroup per variant; larger
    ones in two, the search over many workgroups (the last one to finish
-   decides, and sums any further line-search window by itself) and the step.
+   decides, and sums a further line-search window by itself on networks of up
+   to 16,384 links; on larger ones a host loop has each done by many) and the
+   step.
    1 / 2: always the first / the second form.  window: step sizes 2^-j a
    window decides on (1..16; 0: 16, the default) -- smaller windows exercise
    the later-window paths on ordinary steps.  The step chosen never depends

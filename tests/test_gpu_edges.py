@@ -391,3 +391,45 @@ def test_one_workgroup_batches(engine_mod, N, Z, ft, extra, kind):
                 assert eng.stats()["graph_launches"] == 0
             out.append((x + [eng.flows(v) for v in range(V)], [eng.trace(v) for v in range(V)]))
     _same(*out)
+
+
+@pytest.mark.parametrize("form", ["plain", "one by one", "batch", "lanes", "hbm"])
+def test_further_windows_over_many_workgroups(engine_mod, oracle_lib, form):
+    """A twentieth of the links with a millionth of their capacity: some steps
+    are far below the first window's 2^-15.  On a network of 28,084 links each
+    further window is a pass over many workgroups, counted with the others;
+    steps and volumes are the oracle's, whichever form the iterations take,
+    and a batch's other variant is not held up."""
+    import oracle
+    print(f"case further windows {form}", flush=True)
+    base, rng = grid_network(60, 60, 12, 1)
+    dem = random_demand(base, rng)
+    net = base.copy()
+    narrow = np.random.default_rng(5).random(net.num_links) < 0.05
+    net.capacity = np.where(narrow, 1e-6, 1.0) * net.capacity
+    iters = 60
+    ref = []
+    oracle.lib().ora_set_pow_mode(1)
+    try:
+        for n in (net, base):
+            ref.append(oracle.fw_solve(n, dem, max_iters=iters))
+    finally:
+        oracle.lib().ora_set_pow_mode(0)
+    deep = int((ref[0]["trace"]["lambda_"] < 2.0 ** -15).sum())
+    assert deep >= 5 and (ref[1]["trace"]["lambda_"] >= 2.0 ** -15).all()
+    kw = {}
+    if form in ("batch", "lanes"):
+        kw = dict(num_variants=2, capacity=np.stack([net.capacity, base.capacity]))
+    with engine_mod.TapEngine(net, dem, **kw) as eng:
+        if form == "one by one":
+            eng.set_graphs(0)
+        if form == "lanes":
+            eng.set_lanes(1)
+        if form == "hbm":
+            eng.set_strategy("hbm")
+        eng.fw_init()
+        eng.fw_run(max_iters=iters)
+        assert eng.stats()["link_passes"] >= iters + deep
+        for v in range(eng.V):
+            assert np.array_equal(eng.trace(v)["lambda_"], ref[v]["trace"]["lambda_"])
+            assert np.array_equal(eng.flows(v)[0], ref[v]["x"])

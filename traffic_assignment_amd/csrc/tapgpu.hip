@@ -2370,12 +2370,16 @@ __device__ bool merge_blocks(tap_acc* sums, tap_acc* sh, tap_acc* part, unsigned
 
 // The line search of an iteration in one launch: `blocks` blocks a variant
 // sum the first window, and the last one to finish merges their sums and
-// decides; a step below the first window (2^-15: rare) makes it sum further
-// windows over all links by itself.  A variant that is off, and every
-// variant after a loading that reported an error (a level tie in the lanes
-// kernel, redone by the host), takes no step: its state stays as it was.
-// With one block a variant (small networks) the block also takes the step,
-// so an iteration's link work is one launch; else k_link_step follows.
+// decides.  A step below the first window (2^-15: rare) needs further ones:
+// on networks of up to kSoloLinks links that block sums them by itself; on
+// larger ones each takes a launch with `more`, which the host issues when it
+// sees need_more.  Until then the variant is off, so that the iterations
+// left in a replay pass it by and its loading stays.
+// A variant that is off, and every variant after a loading that reported an
+// error (a level tie in the lanes kernel, redone by the host), takes no step:
+// its state stays as it was.  With one block a variant (small networks) the
+// block sums every window and takes the step, so an iteration's link work is
+// one launch; else k_link_step follows.
 //
 // A link costs 16 cost evaluations (~1,000 instructions) and a block's
 // reduction ~450, so a thread takes one link while that leaves the chip
@@ -2388,6 +2392,12 @@ __device__ bool merge_blocks(tap_acc* sums, tap_acc* sh, tap_acc* part, unsigned
 constexpr int kLinkPer = 8;
 constexpr long long kLinkFill = 1 << 20;   // links a launch has per link of a thread
 constexpr int kSmallLinks = 512;     // links up to which one block a variant is faster
+// Links up to which one block sums a further window as fast as the host has it
+// done by many: ~2 us for each link of a thread, against ~100 us.  Measured, ms
+// for solves with such steps, one block and the host: 200 iterations with 64 of
+// them on 3,800 links 13.3 and 15.6, with 70 on 28,000 60.4 and 41.4, with 49 on
+// 57,000 117 and 78.
+constexpr int kSoloLinks = 16384;
 
 int link_blocks(long long E, long long V, bool alone) {
   const long long per = std::min<long long>(kLinkPer, 1 + E * V / kLinkFill + E / 65536);
@@ -2396,10 +2406,10 @@ int link_blocks(long long E, long long V, bool alone) {
 
 __global__ __launch_bounds__(kBlock) void k_link_search(Links K, VarState* st, unsigned char* var_on,
                                                         tap_acc* part, unsigned* done, const int* err,
-                                                        const FwParams* prm, int alone) {
+                                                        const FwParams* prm, int alone, int solo, int more) {
   constexpr int kWaves = kBlock / kWave;
   const int var = blockIdx.y, tid = threadIdx.x;
-  if (!var_on[var] || err[0] != 0) {
+  if (more ? !st[var].need_more : (!var_on[var] || err[0] != 0)) {
     if (blockIdx.x == 0 && tid == 0) st[var].stepping = 0;
     return;
   }
@@ -2417,12 +2427,12 @@ __global__ __launch_bounds__(kBlock) void k_link_search(Links K, VarState* st, u
       if (K.present[off + k]) link_sums(acc, K, off + k, lam0, first);
     block_reduce_acc<kWaves>(acc, sh, sums);
   };
-  window(0, true, blockIdx.x * kBlock + tid, nb * kBlock);
+  window(more ? st[var].jnext : 0, !more, blockIdx.x * kBlock + tid, nb * kBlock);
   if (nb > 1 && !merge_blocks(sums, sh, part + (size_t)var * nb * kQ, &done[var])) return;
   VarState s{};                                              // (kept by wavefront 0)
   FwParams p{};
   if (tid < kWave) { s = st[var]; p = *prm; }
-  for (int only_g = 0;; only_g = 1) {
+  for (int only_g = more;; only_g = 1) {
     if (tid < kWave) {
       decide_window(s, sums, only_g, p, var);
       if (tid == 0) {
@@ -2432,15 +2442,15 @@ __global__ __launch_bounds__(kBlock) void k_link_search(Links K, VarState* st, u
       }
     }
     __syncthreads();
-    if (!s_more) break;
+    if (!s_more || !solo) break;
     window(s_jnext, false, tid, kBlock);
   }
   if (alone)
     for (int k = tid; k < K.E; k += kBlock) step_link(K, var, k, s_lambda);
   if (tid == 0) {
-    s.stepping = !alone;
+    s.stepping = !alone && !s.need_more;
     st[var] = s;
-    var_on[var] = (unsigned char)s.active;
+    var_on[var] = (unsigned char)(s.active && !s.need_more);
   }
 }
 
@@ -4427,12 +4437,14 @@ static int upload_params(tapgpu_ctx* c, int max_iters, double target) {
 
 // The link passes of an iteration: the line search (with the flags) and the
 // step, and the copy of the iteration block (error flag, counters, states,
-// flags) to pinned host memory.
-static int issue_link_passes(tapgpu_ctx* c, const Links& K, bool readback = true) {
+// flags) to pinned host memory.  With `more` the next window of the variants
+// whose step is below the last one.
+static int issue_link_passes(tapgpu_ctx* c, const Links& K, bool readback = true, int more = 0) {
   const bool alone = c->link_mode == 1 || (c->link_mode == 0 && c->E <= kSmallLinks);
   const int nb = link_blocks(c->E, c->V, alone);
   hipLaunchKernelGGL(k_link_search, dim3(nb, c->V), dim3(kBlock), 0, c->stream, K, c->st, c->var_on,
-                     c->part, c->done, c->err_dev, c->prm, alone ? 1 : 0);
+                     c->part, c->done, c->err_dev, c->prm, alone ? 1 : 0,
+                     alone || c->E <= kSoloLinks ? 1 : 0, more);
   if (!alone)
     hipLaunchKernelGGL(k_link_step, dim3(nb, c->V), dim3(kBlock), 0, c->stream, K, c->st);
   HIPCHK(c, hipGetLastError());
@@ -4579,6 +4591,7 @@ int tapgpu_fw_run(tapgpu_ctx* c, int max_iters, double target_relgap, tapgpu_res
   // variants already past the stop rule do not run (the loop test comes first)
   HIPCHK(c, hipMemcpy(hs.data(), c->st, sizeof(VarState) * c->V, hipMemcpyDeviceToHost));
   for (int v = 0; v < c->V; ++v) {
+    hs[v].need_more = 0;                // (a run that ended in an error may have left it)
     hs[v].active = (max_iters <= 0 || hs[v].iter < max_iters) &&
                    (target_relgap <= 0 || hs[v].relgap > target_relgap);
     hon[v] = (unsigned char)hs[v].active;
@@ -4700,6 +4713,14 @@ int tapgpu_fw_run(tapgpu_ctx* c, int max_iters, double target_relgap, tapgpu_res
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if ((rc = absorb_pending(c))) return rc;
     c->stats.link_passes += 1;
+    auto undecided = [&]() {
+      return std::any_of(c->pin_st, c->pin_st + c->V, [](const VarState& s) { return s.need_more != 0; });
+    };
+    while (undecided()) {
+      if ((rc = issue_link_passes(c, lanes_now ? make_links(c, false) : K, true, 1))) return rc;
+      HIPCHK(c, hipStreamSynchronize(c->stream));
+      c->stats.link_passes += 1;
+    }
     std::copy(c->pin_st, c->pin_st + c->V, hs.begin());
     std::copy(c->pin_on, c->pin_on + c->V, hon.begin());
     const double it_ms =
