@@ -522,7 +522,7 @@ struct OriginArgs {
   const double* sellw;               // [V][sell_n] sliced in-link costs
   const unsigned* sell_id;           // [sell_n] link id << 16 | tail
   const int* sell_ptr;               // [ceil(N/64) + 1] first entry of each slice
-  const struct HbmRec* hrec;         // [variants of the launch][hrec_n] out-link records (labels-in-HBM kernel)
+  const void* hrec;                  // [variants of the launch][hrec_n] out-link records (labels-in-HBM kernel)
   const struct HbmRecOf* hrec_of;    // [hrec_n]
   int hrec_n;
   const uint2* hsell_id;             // [hsell_n] tail, link id
@@ -1120,8 +1120,7 @@ __global__ void k_zero_i32(int* p) { *p = 0; }
 // predecessors' second bitmap takes the place of these.
 constexpr int kHbmQueueMin = 64;                // entries, whatever size is asked for
 constexpr size_t kHbmQueueBytes = 48;           // per entry of the queue size
-constexpr int kHbmGroup = 2;                    // lanes per expanded node
-constexpr int kHbmCand = (5 + kHbmGroup - 1) / kHbmGroup;   // links per lane, at most
+constexpr int kHbmCand = 3;                     // links per lane of an expanded node
 constexpr int kHbmRedo = 64;                    // places kept for entries to be followed up again
 constexpr int kHbmFew = 32;                     // entries brought near at once, below which the far queue is weeded
 constexpr int kHbmSlots = 1024;                 // of the table that settles which lane lowers a label
@@ -1139,30 +1138,38 @@ size_t origin_hbm_lds_bytes(int N, int hqcap) {
 // come in lines too: a search takes them as entries of their own, a round
 // later.  Read from the CSR instead, two links at a time and past the table
 // that settles which label is stored, such nodes held up their wavefronts:
-// grids of 22,500 nodes with 6, 8 and 12 through links each, 200 origins, 3
-// iterations 11.5, 11.3 and 13.2 ms, and 8.5, 8.1 and 9.5 so; 90,000 nodes
-// with 8, 300 origins 66 and 22; regional, where one node in a thousand has
-// more than 5, 39.2 and 36.7 ms a loading.  (Following the records within the
-// round, the workgroup waiting for those that have more: 8.3, 7.6, 10.5, 30
-// and 39.5.)
+// a grid of 22,500 nodes with 12 through links each, 200 origins, 3
+// iterations 13.2 ms, and 9.5 so; a star of 20,000 nodes, 100 origins, one
+// loading 44 and 11; regional, where one node in a thousand has more than 5,
+// 39.2 and 36.7 ms a loading.  (Following the records within the round, the
+// workgroup waiting for those that have more: 10.5, - and 39.5.)
 // The kernel has a numbering of its own: zones keep their numbers, through
 // nodes get places such that each 128-byte line of labels (16 nodes) holds
 // neighbours of each other (hbm_places).  A search's front is a ring; with
 // nodes numbered along rows of a city every node of it brings a line of its
 // own, which 64 workgroups an XCD cannot keep in 4 MB of L2.  Ties are
 // broken by node numbers, not places, so the trees do not depend on it.
-constexpr int kHrecLinks = 5;
+// Records of 5 links (a line) are read by 2 lanes.  Where most nodes have
+// more than 5 links and no more than 10, records hold 10 and are read by 4,
+// so that a node is expanded in one round.  Measured ms with records of 10
+// and of 5 links: grids of 22,500 nodes with 4, 6, 8 and 12 links each, 200
+// origins, 3 iterations 4.9 and 4.9, 7.0 and 8.5, 6.1 and 8.1, 10.4 and 9.6;
+// 48,400 nodes with 6, 12 origins, 10 iterations 30 and 37; regional (4 links)
+// 125 and 109 for two iterations.
+constexpr int hrec_links(int group) { return group == 2 ? 5 : 10; }
+constexpr size_t hrec_bytes(int group) { return 32 * (size_t)group; }
+template <int kGroup>
 struct __align__(64) HbmRec {
-  double w[kHrecLinks];
-  int head[kHrecLinks];
+  double w[hrec_links(kGroup)];
+  int head[hrec_links(kGroup)];
   int more;
+  static_assert(hrec_links(kGroup) <= kHbmCand * kGroup, "a lane takes kHbmCand links");
 };
-static_assert(sizeof(HbmRec) == 64 && kHrecLinks <= kHbmCand * kHbmGroup, "an out-link record is one 64-byte line");
+static_assert(sizeof(HbmRec<2>) == hrec_bytes(2) && sizeof(HbmRec<4>) == hrec_bytes(4), "whole lines");
 // HbmRec::more: the record that follows, whether the one after that follows
 // too (a node's further records are a row that is read as a heap: record k
 // leads to 2k + 1 and 2k + 2), and whether the row goes on
 constexpr int kHrecNext = 0x0FFFFFFF, kHrecRow = 1 << 29, kHrecTwo = 1 << 30;
-static_assert(kHbmGroup == 2, "each lane of a group follows one of the two");
 struct HbmRecOf {
   int first, end;                    // its links: those of [first, end) to through nodes
   int more;                          // HbmRec::more
@@ -1170,8 +1177,10 @@ struct HbmRecOf {
 };
 
 // a thread per (variant, record), and per padding lane of the last slice
-__global__ __launch_bounds__(kBlock) void k_hbm_mirrors(OriginArgs A, int Vn, HbmRec* hrec,
+template <int kGroup>
+__global__ __launch_bounds__(kBlock) void k_hbm_mirrors(OriginArgs A, int Vn, HbmRec<kGroup>* hrec,
                                                         uint2* sell_id, double* sellw_all) {
+  constexpr int kLinks = hrec_links(kGroup);
   const int i = blockIdx.x * kBlock + threadIdx.x;       // record; below N the place of its node
   const int N = A.N, sl = i / kWave;
   const bool slice = sl < (N + kWave - 1) / kWave;
@@ -1185,15 +1194,15 @@ __global__ __launch_bounds__(kBlock) void k_hbm_mirrors(OriginArgs A, int Vn, Hb
     int at = begin;
     if (i < A.hrec_n) {
       const HbmRecOf of = A.hrec_of[i];
-      HbmRec R;
+      HbmRec<kGroup> R;
       int n = 0;
 #pragma unroll
-      for (int g = 0; g < kHrecLinks; ++g) { R.w[g] = INFINITY; R.head[g] = min(i, N - 1); }
+      for (int g = 0; g < kLinks; ++g) { R.w[g] = INFINITY; R.head[g] = min(i, N - 1); }
       for (int k = of.first; k < of.end; ++k) {
         const int d = A.fw_dst[k];
         if (d < A.ft0 || d == A.tail[k]) continue;
 #pragma unroll
-        for (int g = 0; g < kHrecLinks; ++g)
+        for (int g = 0; g < kLinks; ++g)
           if (g == n) { R.w[g] = fw[k]; R.head[g] = A.place[d]; }
         ++n;
       }
@@ -1224,8 +1233,10 @@ __device__ __forceinline__ int ldg_i32(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+template <int kGroup>
 __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void k_origin_hbm(OriginArgs A, int load, int items) {
   extern __shared__ unsigned long long sm[];
+  constexpr int kLinks = hrec_links(kGroup), kRecBytes = (int)hrec_bytes(kGroup);
   constexpr int kWaves = kHbmBlock / kWave;
   const int N = A.N, ft0 = A.ft0, qcap = A.hqcap;
   const int W = (N + 63) >> 6;
@@ -1282,7 +1293,7 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
     const int src = A.place[origin];          // (nodes below are places, unless they come from the CSR)
     const double* __restrict__ fw = A.fww + (size_t)var * A.E;
     const double* __restrict__ rw = A.rvw + (size_t)var * A.E;
-    const char* recb = (const char*)(A.hrec + (size_t)var * A.hrec_n);
+    const char* recb = (const char*)A.hrec + (size_t)var * A.hrec_n * kRecBytes;
     const double* __restrict__ sellw = A.hsellw + (size_t)var * A.hsell_n;
     const long long clk0 = wall_clock64();
     // ---- label-correcting rounds in buckets.  Round r expands the near
@@ -1323,7 +1334,7 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
     //      links at a million times their cost: 2,360 moves an origin and
     //      160 ms a loading, 39 weeded, as without such links).
     //      A round is a chain of trips to the XCD's L2 and beyond, so what
-    //      counts is their number and the lines they touch: kHbmGroup lanes
+    //      counts is their number and the lines they touch: kGroup lanes
     //      share an expanded node, whose links are one line that is read
     //      beside its label; the labels of the heads are next.  Links to
     //      zones are left out (their labels are pulled at the end), and
@@ -1338,8 +1349,8 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
     unsigned long long T = 0;
     int r = 1, fb = 0, lim = qcap;             // lim: places of the near queue for lowered nodes
     bool wide = false;
-    constexpr int kPass = kHbmBlock / kHbmGroup;     // nodes taken at once
-    const int g = lane & (kHbmGroup - 1), grp = lane / kHbmGroup;
+    constexpr int kPass = kHbmBlock / kGroup;     // nodes taken at once
+    const int g = lane & (kGroup - 1), grp = lane / kGroup;
     // this lane's place among the lanes with `want`, counted on *n
     auto place = [&](bool want, int* n) {
       const unsigned long long bal = __ballot(want);
@@ -1442,23 +1453,23 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
       for (int s = tid; s < kHbmSlots; s += kHbmBlock) { tab_node[s] = 0u; tab_lab[s] = ~0ull; }
       for (int j0 = 0; j0 < qn; j0 += kPass) {
         // ---- the lanes of a group take an entry (all lanes come here) ----
-        const int j = j0 + wave * (kWave / kHbmGroup) + grp;
+        const int j = j0 + wave * (kWave / kGroup) + grp;
         const bool on = j < qn;
         const int at = from + (j < n1 ? j : qcap - 1 - (j - n1));
         const int u = on ? (int)near_node[at] : src;
         const unsigned long long lab = on ? near_lab[at] : kMax;
-        const unsigned ro = (unsigned)u * 64u;
+        const unsigned ro = (unsigned)u * kRecBytes;
         // (an entry from N on is a further record of a node that was expanded)
         // (no load is masked: a merge with a default waits for each of them)
         double w[kHbmCand];
         int v[kHbmCand];
         const unsigned long long seen = ldg_u64(&dist[min(u, N - 1)]), have = u < N ? seen : lab;
-        const int more = *(const int*)(recb + (ro + 12u * kHrecLinks));
+        const int more = *(const int*)(recb + (ro + 12u * kLinks));
 #pragma unroll
         for (int i = 0; i < kHbmCand; ++i) {
-          const unsigned k = min((unsigned)(g + i * kHbmGroup), (unsigned)(kHrecLinks - 1));
+          const unsigned k = min((unsigned)(g + i * kGroup), (unsigned)(kLinks - 1));
           w[i] = *(const double*)(recb + (ro + k * 8u));
-          v[i] = *(const int*)(recb + (ro + 8u * kHrecLinks + k * 4u));
+          v[i] = *(const int*)(recb + (ro + 8u * kLinks + k * 4u));
         }
         if (j0 == 0) __syncthreads();                  // (the table is clear; the loads are on their way)
         const bool lost = on && g == 0 && have > lab;
@@ -1474,7 +1485,7 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         bool first = on && g == 0 && have == lab;
         const unsigned long long bit = 1ull << (u & 63);
         if (first && u < N) first = !(atomicOr(&bmA[u >> 6], bit) & bit);
-        const bool go = (__ballot(first) >> (lane & ~(kHbmGroup - 1))) & 1ull;
+        const bool go = (__ballot(first) >> (lane & ~(kGroup - 1))) & 1ull;
         n_exp += first && u < N;
         unsigned long long cb[kHbmCand], hv[kHbmCand];
         bool low[kHbmCand];
@@ -1486,7 +1497,7 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         }
 #pragma unroll
         for (int i = 0; i < kHbmCand; ++i) {
-          const bool in = go && cb[i] < kMax && g + i * kHbmGroup < kHrecLinks;
+          const bool in = go && cb[i] < kMax && g + i * kGroup < kLinks;
           n_scan += in;
           low[i] = in && cb[i] < hv[i];
           slot[i] = -1;
@@ -1497,7 +1508,7 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         for (int i = 0; i < kHbmCand; ++i)
           if (slot[i] >= 0) low[i] = tab_lab[slot[i]] == cb[i];   // else a smaller one is stored
         relax(v, cb, low, room);
-        const bool rec = go && (g ? more & kHrecTwo : more & kHrecNext);
+        const bool rec = go && (g == 0 ? more & kHrecNext : g == 1 && (more & kHrecTwo));
         if (__ballot(rec)) {                           // the records that follow
           int k = place(rec, &s_near[r % 3]);
           const bool rest = rec && k >= room;
@@ -1706,15 +1717,19 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
         taken += __popcll(m);
         n_exp += go;
         for (int q = go ? u : src;;) {                   // its records
-          const HbmRec* rec = (const HbmRec*)recb + q;
-          int x[kHrecLinks];
-          unsigned long long c[kHrecLinks], have[kHrecLinks];
+          const HbmRec<kGroup>* rec = (const HbmRec<kGroup>*)recb + q;
+          constexpr int K = 5;                           // links at once
           const int more = rec->more;
+#pragma unroll 1
+          for (int k = 0; k < kLinks; k += K) {
+            int x[K];
+            unsigned long long c[K], have[K];
 #pragma unroll
-          for (int i = 0; i < kHrecLinks; ++i) { x[i] = rec->head[i]; c[i] = as_b(as_d(lab) + rec->w[i]); }
+            for (int i = 0; i < K; ++i) { x[i] = rec->head[k + i]; c[i] = as_b(as_d(lab) + rec->w[k + i]); }
 #pragma unroll
-          for (int i = 0; i < kHrecLinks; ++i) have[i] = ldg_u64(&dist[x[i]]);
-          lower(x, c, have, go);
+            for (int i = 0; i < K; ++i) have[i] = ldg_u64(&dist[x[i]]);
+            lower(x, c, have, go);
+          }
           go = go && more & kHrecRow;
           if (!__ballot(go)) break;
           if (go) q = q < N ? more & kHrecNext : q + 1;
@@ -2526,7 +2541,8 @@ struct tapgpu_ctx {
   // the LDS kernel's mirrors of the graph and the costs
   double *rec = nullptr, *sellw = nullptr;
   int *recpos = nullptr, *sellpos = nullptr, *sell_ptr = nullptr;
-  HbmRec* hrec = nullptr;             // the labels-in-HBM kernel's mirrors (alloc_hbm_mirrors)
+  unsigned char* hrec = nullptr;      // the labels-in-HBM kernel's mirrors (alloc_hbm_mirrors)
+  int hgroup = 2;                     // lanes per expanded node (with the records' size)
   int hvars = 0, hvars_max = INT_MAX; // variants they hold, and may hold
   HbmRecOf* hrec_of = nullptr;
   int hrec_n = 0;
@@ -3022,7 +3038,8 @@ constexpr int kChaseCandidates[] = {0, 2, 4, 8, 16, 32};
 constexpr int kTuneBlocks = 4096;              // workgroups of a tuning launch on a batch
 
 int ensure_hbm(tapgpu_ctx* c, int Vn);
-void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn, hipStream_t st);
+void launch_hbm_kernel(tapgpu_ctx* c, const OriginArgs& A, int Vn, int load, int items, int blocks, hipStream_t st,
+                       bool mirrors = true);
 
 // Per-origin round counts of the recording loading (zeroed: origins a
 // loading skips keep 0 and go last).
@@ -3069,9 +3086,7 @@ int launch_origin(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, fl
         OriginArgs B = variant_args(c, var_on, v0 + v);
         B.z0 = zl;
         B.zn = zh;
-        launch_hbm_mirrors(c, B, n, c->stream2);
-        hipLaunchKernelGGL(k_origin_hbm, dim3(std::min(c->hbm_grid, items)), dim3(kHbmBlock),
-                           c->hbm_lds, c->stream2, B, 1, items);
+        launch_hbm_kernel(c, B, n, 1, items, c->hbm_grid, c->stream2);
         HIPCHK(c, hipGetLastError());
       }
       HIPCHK(c, hipEventRecord(c->ev_join, c->stream2));
@@ -3361,12 +3376,12 @@ constexpr size_t kHbmMirrorBytes = 512ull << 20;
 
 int alloc_hbm_mirrors(tapgpu_ctx* c, int Vn) try {
   auto grow = [&]() -> int {
-    const size_t each = sizeof(HbmRec) * (size_t)c->hrec_n + sizeof(double) * (size_t)c->hsell_n;
+    const size_t recs = hrec_bytes(c->hgroup) * (size_t)c->hrec_n, each = recs + sizeof(double) * (size_t)c->hsell_n;
     const int most = std::min<int>(c->hvars_max, (int)std::max<size_t>(1, kHbmMirrorBytes / each));
     for (int n = std::min(Vn, most); n > c->hvars; n /= 2) {
-      HbmRec* rec = nullptr;
+      unsigned char* rec = nullptr;
       double* w = nullptr;
-      int rc = dalloc(c, &rec, (size_t)n * c->hrec_n);
+      int rc = dalloc(c, &rec, n * recs);
       if (!rc && (rc = dalloc(c, &w, (size_t)n * c->hsell_n))) dfree(c, rec);
       if (rc && (n == 1 || rc != TAPGPU_E_NOMEM)) return rc;
       if (rc) {                                        // with fewer at a time, then and later
@@ -3409,12 +3424,20 @@ int alloc_hbm_mirrors(tapgpu_ctx* c, int Vn) try {
   // a node's records: the first at its place, further ones in a row behind
   // all places
   std::vector<HbmRecOf> of(N);
+  auto counts = [&](int v, int k) { return dst[k] >= c->ft0 && dst[k] != v; };
+  int large = 0;
+  for (int v = 0; v < N; ++v) {
+    int n = 0;
+    for (int k = off[v]; k < off[v + 1]; ++k) n += counts(v, k);
+    large += n > hrec_links(2) && n <= hrec_links(4);
+  }
+  c->hgroup = large > N / 2 ? 4 : 2;
   for (int i = 0; i < N; ++i) {
     const int v = h[(size_t)N + i], base = (int)of.size() - 1;
     int at = i, n = 0;
     of[i] = {off[v], off[v + 1], 0, i};
     for (int k = off[v]; k < off[v + 1]; ++k) {
-      if (dst[k] < c->ft0 || dst[k] == v || n++ < kHrecLinks) continue;
+      if (!counts(v, k) || n++ < hrec_links(c->hgroup)) continue;
       n = 1;
       of[at].end = k;
       at = (int)of.size();
@@ -3442,9 +3465,25 @@ int alloc_hbm_mirrors(tapgpu_ctx* c, int Vn) try {
 // (A is advanced to the first, and hvars holds them).
 void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn, hipStream_t st) {
   const int nodes = std::max((c->N + kWave - 1) / kWave * kWave, c->hrec_n);
-  hipLaunchKernelGGL(k_hbm_mirrors, dim3((nodes + kBlock - 1) / kBlock, std::min(Vn, 65535)), dim3(kBlock), 0,
-                     st, A, Vn, const_cast<HbmRec*>(A.hrec), const_cast<uint2*>(A.hsell_id),
-                     const_cast<double*>(A.hsellw));
+  const dim3 grid((nodes + kBlock - 1) / kBlock, std::min(Vn, 65535));
+  uint2* id = const_cast<uint2*>(A.hsell_id);
+  double* w = const_cast<double*>(A.hsellw);
+  if (c->hgroup == 4)
+    hipLaunchKernelGGL(k_hbm_mirrors<4>, grid, dim3(kBlock), 0, st, A, Vn, (HbmRec<4>*)c->hrec, id, w);
+  else
+    hipLaunchKernelGGL(k_hbm_mirrors<2>, grid, dim3(kBlock), 0, st, A, Vn, (HbmRec<2>*)c->hrec, id, w);
+}
+
+// The mirrors of Vn variants, then the kernel over `items` of theirs by at
+// most `blocks` workgroups.
+void launch_hbm_kernel(tapgpu_ctx* c, const OriginArgs& A, int Vn, int load, int items, int blocks, hipStream_t st,
+                       bool mirrors) {
+  if (mirrors) launch_hbm_mirrors(c, A, Vn, st);
+  const dim3 grid(std::min(blocks, items));
+  if (c->hgroup == 4)
+    hipLaunchKernelGGL(k_origin_hbm<4>, grid, dim3(kHbmBlock), c->hbm_lds, st, A, load, items);
+  else
+    hipLaunchKernelGGL(k_origin_hbm<2>, grid, dim3(kHbmBlock), c->hbm_lds, st, A, load, items);
 }
 
 // Per-workgroup scratch rows of the labels-in-HBM kernel (allocated on
@@ -3500,10 +3539,8 @@ int launch_hbm(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, int i
     }
     A.work = work;
     A.next = c->d_hbm_next;
-    launch_hbm_mirrors(c, A, n, c->stream);
     hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, c->stream, c->d_hbm_next);
-    hipLaunchKernelGGL(k_origin_hbm, dim3(std::min(c->hbm_grid, items)), dim3(kHbmBlock), c->hbm_lds, c->stream,
-                       A, 1, items);
+    launch_hbm_kernel(c, A, n, 1, items, c->hbm_grid, c->stream);
     HIPCHK(c, hipGetLastError());
   }
   if (ms) {
@@ -3859,7 +3896,7 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
       for (int64_t j = 0; j < (pw_v ? V * E : E); ++j) pow4 = pow4 && (pw_v ? pw_v : net->power)[j] == 4.0;
       c->tiny_ok = pow4 && tiny_pays(c->N, c->Z, in, zone_in, c->V, ncu);
     }
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_origin_hbm, kHbmBlock, c->hbm_lds) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_origin_hbm<2>, kHbmBlock, c->hbm_lds) !=
         hipSuccess || per_cu < 1)
       per_cu = 1;
     c->hbm_grid = std::max(1, ncu * per_cu);
@@ -4161,11 +4198,9 @@ int tapgpu_sssp(tapgpu_ctx* c, int64_t variant, const int64_t* start_nodes, int6
       A.src_list = S.src; A.err = S.err; A.out_dist = S.dist; A.out_pred = S.pred; A.ld = ns;
       hipLaunchKernelGGL(k_sssp_begin, dim3(grid_for((long long)c->N * ns / kWave + 1)), dim3(kBlock), 0,
                          c->stream, S.pred, (long long)c->N * ns, S.err);
-      if (hbm) {
-        if (s0 == 0) launch_hbm_mirrors(c, A, 1, c->stream);
-        hipLaunchKernelGGL(k_origin_hbm, dim3(std::min(ns, c->hbm_grid)), dim3(kHbmBlock), c->hbm_lds,
-                           c->stream, A, 0, ns);
-      } else
+      if (hbm)
+        launch_hbm_kernel(c, A, 1, 0, ns, c->hbm_grid, c->stream, s0 == 0);
+      else
         launch_lds(c, dim3(ns, 1), c->stream, A, 0);
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess)
@@ -4338,9 +4373,7 @@ int tapgpu_sssp_noalloc(tapgpu_ctx* c, int64_t variant, const int64_t* d_start_n
   if (lds) {
     launch_lds(c, dim3((unsigned)num_start, 1), c->stream, A, 0);
   } else {
-    launch_hbm_mirrors(c, A, 1, c->stream);
-    hipLaunchKernelGGL(k_origin_hbm, dim3((unsigned)std::min<int64_t>(num_start, rows)),
-                       dim3(kHbmBlock), c->hbm_lds, c->stream, A, 0, (int)num_start);
+    launch_hbm_kernel(c, A, 1, 0, (int)num_start, rows, c->stream);
   }
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipMemcpyAsync(c->h_int, c->err_dev, sizeof(int) * 3, hipMemcpyDeviceToHost, c->stream));
