@@ -281,9 +281,9 @@ int tapgpu_get_origin_chase(const tapgpu_ctx *ctx);
    the LDS path, where the next loading picks it with the workgroup size
    (the most, 1024 or 256: a shorter queue takes less LDS, so more
    workgroups share a CU); 0: bitmap scans only; larger values are clamped
-   to that most.  The labels-in-HBM kernel's queues have at least 64 entries;
-   a search whose front exceeds them goes on with bitmaps.  tapgpu_get_origin_queue returns the value of the kernel in
-   use.  Results do not depend on it. */
+   to that most.  The labels-in-HBM kernel goes on with bitmaps once a
+   search's front exceeds its queues.  tapgpu_get_origin_queue returns the
+   value of the kernel in use.  Results do not depend on it. */
 int tapgpu_set_origin_queue(tapgpu_ctx *ctx, int entries);
 int tapgpu_get_origin_queue(const tapgpu_ctx *ctx);
 

@@ -146,3 +146,25 @@ def test_hbm_batch_memory_and_parts(engine_mod):
             assert np.array_equal(one.flows()[0], x[v]), v
             one.fw_run(max_iters=2)
             assert np.array_equal(one.flows()[0], x2[v]), v
+
+
+def test_hbm_queue_size_is_the_one_asked_for(engine_mod):
+    """With no queue, or one entry, a search goes on with bitmaps at once:
+    few nodes wait in a queue for a later bucket.  The results are those of
+    full queues."""
+    print("case hbm queue sizes", flush=True)
+    net, dem = network("metro", 0.3)
+    out = []
+    with engine_mod.TapEngine(net, dem) as eng:
+        eng.set_strategy("hbm")
+        eng.set_origin_delta(1.0)
+        waited = []
+        for q in (-1, 0, 1, 2, 16, 65):
+            eng.set_origin_queue(q)
+            a = eng.stats()["origin_deferred"]
+            out.append(eng.aon())
+            waited.append(eng.stats()["origin_deferred"] - a)
+            assert eng.origin_queue == q or q < 0
+    assert 10 * max(waited[1], waited[2]) < waited[0]
+    for y in out[1:]:
+        assert np.array_equal(y, out[0])

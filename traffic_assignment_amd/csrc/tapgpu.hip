@@ -1118,7 +1118,7 @@ __global__ void k_zero_i32(int* p) { *p = 0; }
 // LDS of the labels-in-HBM kernel: a bitmap 8W | the table, two near queues
 // and a far queue of twice their size, of (label 8 B, node 4 B) entries; the
 // predecessors' second bitmap takes the place of these.
-constexpr int kHbmQueueMin = 64;                // entries, whatever size is asked for
+constexpr int kHbmQueueMin = 64;                // entries there is room for at least (fewer can be asked for)
 constexpr size_t kHbmQueueBytes = 48;           // per entry of the queue size
 constexpr int kHbmCand = 3;                     // links per lane of an expanded node
 constexpr int kHbmRedo = 64;                    // places kept for entries to be followed up again
@@ -2975,7 +2975,7 @@ OriginArgs make_origin_args(tapgpu_ctx* c, const unsigned char* var_on) {
   A.var_on = var_on; A.y = c->y; A.err = c->err_dev; A.counters = c->counters;
   A.chase = c->chase >= 0 ? c->chase : kDefaultChase;
   A.qcap = c->qcap;
-  A.hqcap = std::max(c->hqcap, kHbmQueueMin);
+  A.hqcap = std::max(c->hqcap, 1);            // (with 1 a search goes on with bitmaps from its first nodes)
   A.h_dist = c->h_dist; A.h_pred = c->h_pred; A.h_ptail = c->h_ptail;
   // (negative: a width to start from; before tuning, or without buckets)
   A.delta = c->delta_mult > 0 ? c->delta_mult * c->mean_t0 : c->mean_t0 > 0 ? -4.0 * c->mean_t0 : -1.0;
