@@ -221,9 +221,10 @@ typedef struct {
   int64_t origin_launches, origin_blocks;
   int64_t origin_expansions;   /* node expansions (label-correcting)        */
   int64_t origin_scanned;      /* out-links relaxed                         */
-  int64_t origin_updates;      /* labels lowered (labels-in-HBM and lanes   */
-                               /* kernels: atomic mins issued, one per      */
-                               /* candidate below the label read)           */
+  int64_t origin_updates;      /* labels lowered (labels-in-HBM kernel:     */
+                               /* labels stored; lanes kernel: atomic mins  */
+                               /* issued; one per candidate below the label */
+                               /* read)                                     */
   int64_t origin_relax_rounds;  /* relaxation rounds, summed over origins    */
   int64_t origin_load_rounds;   /* longest loading walk, summed over origins */
   int64_t origin_loaded;        /* tree links given flow                     */
@@ -250,7 +251,9 @@ typedef struct {
 } tapgpu_stats;
 
 /* Counters and wall times of the last tapgpu_fw_run (or of the calls since
-   the last fw_run for sssp/aon). */
+   the last fw_run for sssp/aon).  Iterations inside the one kernel of small
+   networks (tapgpu_set_graphs) count workgroups, relaxation rounds and walk
+   steps, and their time is link_ms. */
 int tapgpu_get_stats(tapgpu_ctx *ctx, tapgpu_stats *stats);
 
 /* on != 0: time every sweep / level launch with HIP events (small overhead). */

@@ -472,3 +472,24 @@ def test_one_workgroup_failed_loading_changes_nothing(engine_mod):
     for a, b in zip(*states):
         assert np.array_equal(a[0], b[0])
         assert np.array_equal(a[1], b[1], equal_nan=True)
+
+
+def test_one_workgroup_statistics(engine_mod):
+    """What the one kernel counts is what the launches count under that name;
+    what it does not count is 0."""
+    print("case one-workgroup statistics", flush=True)
+    net, rng = grid_network(6, 7, 20, 0)
+    dem = random_demand(net, rng)
+    st = []
+    for graphs in (1, 0):
+        with engine_mod.TapEngine(net, dem) as eng:
+            eng.set_graphs(graphs)
+            eng.fw_init()
+            eng.fw_run(max_iters=9)
+            st.append(eng.stats())
+    one, launches = st
+    for k in ("origin_blocks", "origin_walk_steps", "link_passes"):
+        assert one[k] == launches[k] > 0, k
+    assert one["origin_relax_rounds"] > 0
+    for k in ("origin_loaded", "origin_expansions", "origin_scanned", "origin_updates"):
+        assert one[k] == 0 < launches[k], k
