@@ -493,3 +493,33 @@ def test_one_workgroup_statistics(engine_mod):
     assert one["origin_relax_rounds"] > 0
     for k in ("origin_loaded", "origin_expansions", "origin_scanned", "origin_updates"):
         assert one[k] == 0 < launches[k], k
+
+
+@pytest.mark.parametrize("form,power", [("tiny", 4.0), ("lds", 2.0), ("lanes", 2.0), ("passes", 2.0)])
+def test_more_variants_than_a_grid_dimension(engine_mod, form, power):
+    """66,000 variants, above the 65,535 of a launch in the grid's second
+    dimension: those on both sides of the cut are what a context of their own
+    gives, whichever kernels load them and take their steps."""
+    print(f"case 66,000 variants {form}", flush=True)
+    net, rng = grid_network(3, 3, 3, 0, power)
+    dem = random_demand(net, rng)
+    V = 66000
+    cap = net.capacity * rng.uniform(0.8, 1.25, (V, net.num_links))
+
+    def solve(**kw):
+        with engine_mod.TapEngine(net, dem, **kw) as eng:
+            if form != "tiny":
+                eng.set_graphs(0)
+            if form == "passes":
+                eng.set_link_passes(2)
+            if kw.get("num_variants", 1) > 1 and form != "tiny":
+                eng.set_lanes(1 if form == "lanes" else 0)
+            eng.fw_init()
+            eng.fw_run(max_iters=3)
+            at = watched if "num_variants" in kw else [0]
+            return [eng.flows(v) for v in at], [eng.trace(v) for v in at], [eng.totals(v) for v in at]
+    watched = [0, 65534, 65535, V - 1]
+    many = solve(num_variants=V, capacity=cap)
+    alone = [solve(capacity=cap[v:v + 1]) for v in watched]
+    _same(many, [[one[k][0] for one in alone] for k in range(3)])
+    np.testing.assert_allclose(many[2], [one[2][0] for one in alone], rtol=1e-14, atol=0.0)

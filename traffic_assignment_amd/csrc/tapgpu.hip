@@ -58,6 +58,7 @@ namespace {
 constexpr int kWave = 64;
 constexpr int kBlock = 256;                 // 4 wavefronts
 constexpr int kWavesPerBlock = kBlock / kWave;
+constexpr int kGridVariants = 65535;        // variants of a launch in the grid's second dimension
 constexpr int kJ = 16;                      // step sizes 2^-j evaluated per link pass
 constexpr int kQ = 3 + kJ;                  // g0, objective, vht, g(2^-j)...
 constexpr int kMaxHalvings = 1001;          // lambda = 2^-1 ... 2^-1001
@@ -2421,9 +2422,9 @@ int link_blocks(long long E, long long V, bool alone) {
 
 __global__ __launch_bounds__(kBlock) void k_link_search(Links K, VarState* st, unsigned char* var_on,
                                                         tap_acc* part, unsigned* done, const int* err,
-                                                        const FwParams* prm, int alone, int solo, int more) {
+                                                        const FwParams* prm, int v0, int alone, int solo, int more) {
   constexpr int kWaves = kBlock / kWave;
-  const int var = blockIdx.y, tid = threadIdx.x;
+  const int var = v0 + blockIdx.y, tid = threadIdx.x;
   if (more ? !st[var].need_more : (!var_on[var] || err[0] != 0)) {
     if (blockIdx.x == 0 && tid == 0) st[var].stepping = 0;
     return;
@@ -2469,8 +2470,8 @@ __global__ __launch_bounds__(kBlock) void k_link_search(Links K, VarState* st, u
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_link_step(Links K, const VarState* st) {
-  const int var = blockIdx.y;
+__global__ __launch_bounds__(kBlock) void k_link_step(Links K, const VarState* st, int v0) {
+  const int var = v0 + blockIdx.y;
   if (!st[var].stepping) return;
   const double lambda = st[var].lambda;
   for (int k = blockIdx.x * kBlock + threadIdx.x; k < K.E; k += gridDim.x * kBlock) step_link(K, var, k, lambda);
@@ -2479,8 +2480,9 @@ __global__ __launch_bounds__(kBlock) void k_link_step(Links K, const VarState* s
 // Per variant at the current volumes: out[2v] = VHT = sum x * c, out[2v+1]
 // = the Beckmann objective (sum of the link cost integrals), compensated
 // sums in a fixed order.
-__global__ __launch_bounds__(kBlock) void k_totals(Links K, tap_acc* part, unsigned* done, double* out) {
-  const int var = blockIdx.y, nb = gridDim.x;
+__global__ __launch_bounds__(kBlock) void k_totals(Links K, tap_acc* part, unsigned* done, double* out,
+                                                   int v0) {
+  const int var = v0 + blockIdx.y, nb = gridDim.x;
   tap_acc acc[kQ];
 #pragma unroll
   for (int q = 0; q < kQ; ++q) acc[q] = tap_acc{0.0, 0.0};
@@ -3091,7 +3093,12 @@ int launch_origin(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on, fl
       }
       HIPCHK(c, hipEventRecord(c->ev_join, c->stream2));
     }
-    launch_lds(c, dim3(zl, Vn), c->stream, A, 1);
+    for (int v = 0; v < Vn; v += kGridVariants) {
+      OriginArgs B = variant_args(c, var_on, v0 + v);
+      B.src_list = A.src_list;
+      B.work = v == 0 ? A.work : nullptr;
+      launch_lds(c, dim3(zl, std::min(Vn - v, kGridVariants)), c->stream, B, 1);
+    }
     HIPCHK(c, hipGetLastError());
     if (zh > 0) HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
     if (ms) HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
@@ -3465,7 +3472,7 @@ int alloc_hbm_mirrors(tapgpu_ctx* c, int Vn) try {
 // (A is advanced to the first, and hvars holds them).
 void launch_hbm_mirrors(tapgpu_ctx* c, const OriginArgs& A, int Vn, hipStream_t st) {
   const int nodes = std::max((c->N + kWave - 1) / kWave * kWave, c->hrec_n);
-  const dim3 grid((nodes + kBlock - 1) / kBlock, std::min(Vn, 65535));
+  const dim3 grid((nodes + kBlock - 1) / kBlock, std::min(Vn, kGridVariants));
   uint2* id = const_cast<uint2*>(A.hsell_id);
   double* w = const_cast<double*>(A.hsellw);
   if (c->hgroup == 4)
@@ -4475,11 +4482,13 @@ static int upload_params(tapgpu_ctx* c, int max_iters, double target) {
 static int issue_link_passes(tapgpu_ctx* c, const Links& K, bool readback = true, int more = 0) {
   const bool alone = c->link_mode == 1 || (c->link_mode == 0 && c->E <= kSmallLinks);
   const int nb = link_blocks(c->E, c->V, alone);
-  hipLaunchKernelGGL(k_link_search, dim3(nb, c->V), dim3(kBlock), 0, c->stream, K, c->st, c->var_on,
-                     c->part, c->done, c->err_dev, c->prm, alone ? 1 : 0,
-                     alone || c->E <= kSoloLinks ? 1 : 0, more);
-  if (!alone)
-    hipLaunchKernelGGL(k_link_step, dim3(nb, c->V), dim3(kBlock), 0, c->stream, K, c->st);
+  for (int v = 0; v < c->V; v += kGridVariants)
+    hipLaunchKernelGGL(k_link_search, dim3(nb, std::min(c->V - v, kGridVariants)), dim3(kBlock), 0,
+                       c->stream, K, c->st, c->var_on, c->part, c->done, c->err_dev, c->prm, v,
+                       alone ? 1 : 0, alone || c->E <= kSoloLinks ? 1 : 0, more);
+  for (int v = 0; v < c->V && !alone; v += kGridVariants)
+    hipLaunchKernelGGL(k_link_step, dim3(nb, std::min(c->V - v, kGridVariants)), dim3(kBlock), 0,
+                       c->stream, K, c->st, v);
   HIPCHK(c, hipGetLastError());
   if (readback)
     HIPCHK(c, hipMemcpyAsync(c->pin_block, c->iter_dev, c->iter_bytes, hipMemcpyDeviceToHost,
@@ -4488,8 +4497,10 @@ static int issue_link_passes(tapgpu_ctx* c, const Links& K, bool readback = true
 }
 
 static void launch_totals(tapgpu_ctx* c) {
-  hipLaunchKernelGGL(k_totals, dim3(link_blocks(c->E, c->V, false), c->V), dim3(kBlock), 0, c->stream,
-                     make_links(c), c->part, c->done, c->vht);
+  const int nb = link_blocks(c->E, c->V, false);
+  for (int v = 0; v < c->V; v += kGridVariants)
+    hipLaunchKernelGGL(k_totals, dim3(nb, std::min(c->V - v, kGridVariants)), dim3(kBlock), 0, c->stream,
+                       make_links(c), c->part, c->done, c->vht, v);
 }
 
 // Records what `issue` puts on the context's stream into an executable
