@@ -235,10 +235,12 @@ typedef struct {
   double origin_tune_ms;        /* fastest launch of the schedule tuning     */
   int64_t origin_chase;         /* chained expansions per thread and round   */
   double origin_delta;          /* bucket width of the labels-in-HBM kernel, */
-                                /*   in mean free-flow link times (0: none)  */
+                                /*   in mean free-flow link times (0: by the */
+                               /*   number of nodes in a bucket)            */
   int64_t origin_split;         /* origins per variant co-run by the HBM     */
                                 /*   kernel beside the LDS kernel            */
-  int64_t origin_deferred;      /* queued nodes kept for a later bucket      */
+  int64_t origin_deferred;      /* nodes kept for a later bucket, once for   */
+                               /*   each time they are listed there         */
   int64_t origin_block;         /* LDS path: threads per workgroup           */
   int64_t origin_queue;         /* frontier queue entries of the kernel used */
   /* lanes kernel (batched loading, one variant per wavefront lane) */
@@ -268,7 +270,7 @@ int tapgpu_set_profiling(tapgpu_ctx *ctx, int on);
 int tapgpu_set_strategy(tapgpu_ctx *ctx, int strategy);
 
 /* Worklist schedule of the one-origin-per-workgroup path (strategy 2),
-   rounds that scan the frontier bitmap (see tapgpu_set_origin_queue): how
+   rounds that scan for the frontier (see tapgpu_set_origin_queue): how
    many labels a thread lowers and then expands itself, in a chain, within
    one round (0: every lowered node waits for the next round).  -1 (the
    default): tuned on the next loading by timing each candidate
@@ -279,11 +281,11 @@ int tapgpu_get_origin_chase(const tapgpu_ctx *ctx);
 /* Frontier queues of the one-origin-per-workgroup paths (strategies 2 and
    3) and of the lanes kernel: a round whose frontier (the nodes lowered or
    kept in the round before) has at most this many nodes takes them from an
-   LDS list; a larger frontier is found by scanning its bitmap.  -1 (the
+   LDS list; a larger frontier is found by scanning flags.  -1 (the
    default): the most each kernel's spare LDS holds (up to 4096), except on
    the LDS path, where the next loading picks it with the workgroup size
    (the most, 1024 or 256: a shorter queue takes less LDS, so more
-   workgroups share a CU); 0: bitmap scans only; larger values are clamped
+   workgroups share a CU); 0: scans only; larger values are clamped
    to that most.  The labels-in-HBM kernel goes on with bitmaps once a
    search's front exceeds its queues.  tapgpu_get_origin_queue returns the
    value of the kernel in use.  Results do not depend on it. */

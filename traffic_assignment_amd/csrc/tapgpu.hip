@@ -3,9 +3,14 @@
 //
 // Replaces the reference's per-iteration work (trunk/tap/tap_frankwolfe_*.c,
 // trunk/tap/pape_*.cu, trunk/tap/volume_update_*.cu) with HBM-resident state
-// and four kernel families, all FP64 and none of them MFMA-shaped:
+// and these kernel families, all FP64 and none of them MFMA-shaped:
 //
-//  * all-origin shortest paths: node-major labels dist[v][col] with one
+//  * shortest paths and loading, one origin per workgroup: the path of almost
+//    every call, with labels in LDS (k_origin_lds) where they fit and in HBM
+//    (k_origin_hbm) where not; a batch's variants in the lanes of a wavefront
+//    where that is faster (taplanes.inc); whole iterations of the smallest
+//    networks in one workgroup (taptiny.inc).
+//  * all-origin shortest paths (any size): node-major labels dist[v][col] with one
 //    origin per wavefront lane (64 origins per "group"); pull relaxations
 //    over an explicit worklist of (node, group) items; a node's out-neighbours
 //    are queued for the next sweep when any lane improved, deduplicated by a
@@ -13,7 +18,7 @@
 //    Labels are the least fixed point of fl(dist[u] + w) over paths whose
 //    inner nodes are not zones (trunk/tap/sssp_pape.c:355), so they are
 //    bit-identical to d'Esopo-Pape's for any relaxation order.
-//  * all-or-nothing loading: bottom-up accumulation on the predecessor trees
+//  * their all-or-nothing loading: bottom-up accumulation on the predecessor trees
 //    (children counted in a dense pass, then ready nodes push their subtree
 //    demand to the parent level by level); per-group partial link volumes are
 //    summed in a fixed order, so volumes are deterministic (and exact for
@@ -21,9 +26,9 @@
 //  * link passes: one fused pass evaluates g(0) = sum c*d, the Beckmann
 //    objective, VHT and g(2^-j) for a window of j (the only step sizes the
 //    reference's bisection ever tests, trunk/tap/tap_functions.c:469-507)
-//    with compensated block sums; a decision kernel per variant picks lambda
-//    and updates gap / relative gap; an update pass does x += lambda*d and
-//    BPR.
+//    with compensated block sums, and the last of a variant's blocks picks
+//    lambda and updates gap / relative gap; an update pass does
+//    x += lambda*d and BPR.
 //  * everything is per "variant": a batch of TAPs over one union topology
 //    (uneven link sets via a presence mask) runs in the same launches.
 //
@@ -434,8 +439,8 @@ __global__ __launch_bounds__(kBlock) void k_aon_reduce(int E, int Gv, int v0, in
 // 160 KB LDS, so a 1024-thread workgroup runs the whole origin: rounds of
 // label-correcting relaxation (64-bit LDS atomicMin on the label bits --
 // non-negative doubles order like their bit patterns; the nodes lowered in a
-// round form the next round's frontier, deduplicated by a bitmap and listed
-// in an LDS queue so that each frontier node gets a thread of its own), then
+// round form the next round's frontier, marked by a bit of the label itself
+// and listed in an LDS queue, kGroup lanes expanding each), then
 // predecessor selection, then loading: each destination walks its tree path
 // adding its demand to LDS node flows (FP64 LDS atomics), and every tree
 // link with flow adds it to the HBM link volumes (FP64 atomics).  One launch
@@ -455,9 +460,9 @@ __global__ __launch_bounds__(kBlock) void k_aon_reduce(int E, int Gv, int v0, in
 // path is unique this is the reference's predecessor.
 
 // Workgroup sizes of the LDS kernel; a size serves networks of up to
-// kLdsPerThread nodes per thread (the per-thread register arrays of the
-// predecessor phase).  1024 by default; the schedule tuner may pick a
-// smaller one where it fits.
+// kLdsPerThread nodes per thread: a wavefront of the predecessor phase takes
+// that many slices of 64 nodes at most, whose bounds it keeps one a lane.
+// 1024 by default; the schedule tuner may pick a smaller one where it fits.
 constexpr int kLdsBlock = 1024;
 constexpr int kLdsBlocks[] = {1024, 512, 256};
 constexpr int kDefaultChase = 4;               // before tuning / shortest-path-only calls
@@ -539,7 +544,7 @@ struct OriginArgs {
   int chase;                         // expansions a thread chains per round
   int qcap;                          // LDS frontier queue entries per round (0: bitmap scan only)
   int hqcap;                         // labels-in-HBM kernel: entries of a queue
-  double delta;                      // labels-in-HBM kernel: bucket width (<= 0: none)
+  double delta;                      // labels-in-HBM kernel: bucket width (< 0: the first of one that adapts)
   int z0, zn;                        // labels-in-HBM kernel: origins [z0, z0 + zn) of each variant
   double* y;                         // [V * E], zeroed by the caller
   int* err;                          // [3]
@@ -649,7 +654,6 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
   unsigned short* pred = (unsigned short*)(bmC + W);               // [N]
   unsigned short* ptail = pred + Al;                               // [N]
   unsigned short* queue0 = ptail + Al;                             // 2 x [qcap + 2]
-  unsigned short* queue1 = queue0 + A.qcap + 2;
   __shared__ int s_qn[3];
   __shared__ unsigned long long s_cnt[8];
 
@@ -3167,8 +3171,9 @@ int tune_chase(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
 // Workgroup size and queue size of the LDS kernel: every allowed size
 // (kLdsPerThread nodes per thread at most) with, unless the queue size was
 // set, the full queue and two shorter ones (less LDS per workgroup, so more
-// workgroups per CU), each timed on one full launch; the fastest pair is
-// kept.  Results do not depend on them.
+// workgroups per CU), each timed on one launch over the variants given (of a
+// batch, enough of them to fill the chip); the fastest pair is kept.  Results
+// do not depend on them.
 int tune_lds_shape(tapgpu_ctx* c, int v0, int Vn, const unsigned char* var_on) {
   if (!c->ev[0])
     for (auto& e : c->ev) HIPCHK(c, hipEventCreate(&e));

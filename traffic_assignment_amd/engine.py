@@ -340,7 +340,7 @@ class TapEngine:
 
     def set_origin_chase(self, chase):
         """Chained expansions per thread and round on the one-origin-per-
-        workgroup path, in rounds that scan the frontier bitmap (-1: tune on
+        workgroup path, in rounds that scan for the frontier (-1: tune on
         the next loading)."""
         self._check(lib().tapgpu_set_origin_chase(self._h, int(chase)))
 
@@ -350,7 +350,8 @@ class TapEngine:
 
     def set_origin_queue(self, entries):
         """Largest frontier the one-origin-per-workgroup paths take from
-        their LDS queues (-1: as many as their LDS holds, 0: bitmap scans
+        and the lanes kernel take from their LDS queues (-1: as many as
+        their LDS holds, on the LDS path picked by the next loading; 0: scans
         only)."""
         self._check(lib().tapgpu_set_origin_queue(self._h, int(entries)))
 
@@ -378,7 +379,8 @@ class TapEngine:
 
     def set_origin_delta(self, mult):
         """Bucket width of the labels-in-HBM path in mean free-flow link
-        times (0: none, -1: tune on the next loading)."""
+        times (0: by the number of nodes in a bucket, -1: tune on the next
+        loading)."""
         self._check(lib().tapgpu_set_origin_delta(self._h, float(mult)))
 
     @property
