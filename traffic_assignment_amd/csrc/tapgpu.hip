@@ -1345,8 +1345,8 @@ __global__ __launch_bounds__(kHbmBlock, kHbmPerCu * kHbmBlock / kWave / 4) void 
     //      zones are left out (their labels are pulled at the end), and
     //      keeping a node for a later bucket costs nothing in the rounds
     //      between.  Measured on regional (4,000 origins, 94,000 nodes, 500
-    //      rounds an origin): 3.1 ms an origin and workgroup for the labels,
-    //      0.9 for the predecessors, 0.5 for the loading, 38 ms a loading;
+    //      rounds an origin): 2.9 ms an origin and workgroup for the labels,
+    //      0.9 for the predecessors, 0.5 for the loading, 37 ms a loading;
     //      with one lane a node, CSR reads, an L2 atomic a lowered label and
     //      queued nodes looked at in every round 6.0, 1.2 and 0.8, 66 ms. ----
     const bool adapt = A.delta < 0.0;
