@@ -523,3 +523,53 @@ def test_more_variants_than_a_grid_dimension(engine_mod, form, power):
     alone = [solve(capacity=cap[v:v + 1]) for v in watched]
     _same(many, [[one[k][0] for one in alone] for k in range(3)])
     np.testing.assert_allclose(many[2], [one[2][0] for one in alone], rtol=1e-14, atol=0.0)
+
+
+@pytest.mark.parametrize("kind", ["cont", "ints", "zeros"])
+def test_lds_kernel_nodes_of_many_in_links(engine_mod, kind):
+    """Nodes with 15 to 900 in-links (a slice holds 16, a wavefront looks at
+    64 at a time), some of them parallel: the tree link is the tight one with
+    the smallest tail label, then tail, then link, and the labels-in-HBM
+    kernel chooses the same, equal labels included."""
+    from traffic_assignment_amd import synth
+    print(f"case LDS kernel, nodes of many in-links, {kind}", flush=True)
+    rng = np.random.default_rng(5)
+    N, Z, ft = 1200, 20, 11                            # (zones 11..20 are through nodes)
+    ring, zones = np.arange(ft, N + 1), np.arange(1, ft)
+    at = rng.choice(ring, zones.size, replace=False)
+    init = [ring, np.roll(ring, -1), zones, at]
+    term = [np.roll(ring, -1), ring, at, zones]
+    for v, n in zip(rng.choice(np.arange(ft, N + 1), 9, replace=False), (15, 16, 17, 63, 64, 65, 128, 300, 900)):
+        t = rng.integers(1, N + 1, n)
+        t[t == v] = ft if v == N else v + 1
+        init += [t, np.full(n, v)]
+        term += [np.full(n, v), t]
+    init, term = np.concatenate(init), np.concatenate(term)
+    order = np.lexsort((term, init))
+    E = init.size
+    cost = {"cont": rng.uniform(0.5, 3.0, E), "ints": rng.integers(1, 4, E).astype(float),
+            "zeros": rng.integers(0, 2, E).astype(float)}[kind]
+    net = synth.Network(num_zones=Z, num_nodes=N, first_thru_node=ft, init=init[order], term=term[order],
+                        capacity=np.full(E, 100.0), length=np.ones(E), fftime=cost, B=np.full(E, 0.15),
+                        power=np.full(E, 4.0), speed=np.zeros(E), toll=np.zeros(E), ltype=np.ones(E, np.int16))
+    dem = random_demand(net, rng)
+    starts = np.arange(1, 60)
+    got = {}
+    for strategy in ("lds", "hbm"):
+        with engine_mod.TapEngine(net, dem) as eng:
+            eng.set_strategy(strategy)
+            eng.set_costs(cost)
+            d, p = eng.sssp(starts)
+            got[strategy] = (d, p, eng.aon())
+    for a, b in zip(got["lds"], got["hbm"]):
+        np.testing.assert_array_equal(a, b)
+    d, p, _ = got["lds"]
+    tail, head = net.init, net.term
+    for j, s in enumerate(starts):
+        dist, pred = d[1:, j], p[1:, j]
+        du, dv = dist[tail - 1], dist[head - 1]
+        tight = (du + cost == dv) & (du < dv) & ((tail >= ft) | (tail == s)) & (tail != head)
+        k = np.flatnonzero(tight)
+        k = k[np.lexsort((k, tail[k], du[k], head[k]))]
+        first = np.r_[True, head[k][1:] != head[k][:-1]] if k.size else np.zeros(0, bool)
+        np.testing.assert_array_equal(pred[head[k[first]] - 1], k[first])

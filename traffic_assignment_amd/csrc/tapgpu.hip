@@ -491,8 +491,8 @@ constexpr unsigned kNoPred = 0xFFFF;
 //    the cost.  Only links between through nodes: those of zones are looked
 //    at by themselves.  An entry without a link has the node itself as its
 //    tail and an infinite cost.
-//    At most kSellWidth rows a slice; a node with more in-links is redone
-//    from the CSR.
+//    At most kSellWidth rows a slice; a node with more in-links is looked at
+//    after the slices, from the CSR.
 constexpr int kRecDoubles = 8, kRecLinks = 6;
 constexpr unsigned kRecNode = 0x3FFF, kRecMore = 0x4000, kRecCsr = 0x8000;
 static_assert(kRecLinks * 10 <= 64 && kRecLinks <= 2 * kGroup, "an out-link record is 64 bytes");
@@ -847,7 +847,7 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
   //      the slices: its label 0 is the smallest there is, and its id too,
   //      so such a link wins where it is tight.  Then the zones, whose
   //      labels are the minimum over their in-links.  Bound by instruction
-  //      issue (about 15 a row; 156 slices of 4 rows on metro): 13.7 us per
+  //      issue (about 15 a row; 156 slices of 4 rows on metro): 14.5 us per
   //      workgroup, 25.6 with a thread reading its node's in-links from the
   //      CSR. ----
   __shared__ int s_level_ties;
@@ -905,11 +905,15 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
       return (__builtin_amdgcn_readlane(last, k) - __builtin_amdgcn_readlane(first, k)) / kWave;
     };
     auto fetch = [&](int k, Rows& R) {
-      const unsigned at = (unsigned)(__builtin_amdgcn_readlane(first, k) + lane);
+      // (no load is left out: one under a branch waits for those before it)
       const int rows = rows_of(k);
+      const unsigned at = (unsigned)((rows ? __builtin_amdgcn_readlane(first, k) : 0) + lane);
 #pragma unroll
-      for (int i = 0; i < kSellFetch; ++i)
-        if (i < rows) { R.id[i] = A.sell_id[at + i * kWave]; R.w[i] = sellw[at + i * kWave]; }
+      for (int i = 0; i < kSellFetch; ++i) {
+        const unsigned a = at + (unsigned)(max(min(i, rows - 1), 0) * kWave);
+        R.id[i] = A.sell_id[a];
+        R.w[i] = sellw[a];
+      }
     };
     auto select = [&](int k, const Rows& R) {
       const int sl = sl0 + k * kWaves, v = sl * kWave + lane, rows = rows_of(k);
@@ -930,10 +934,6 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
       if (rows > kSellFetch) {
         const unsigned at = (unsigned)(__builtin_amdgcn_readlane(first, k) + lane);
         for (int i = kSellFetch; i < rows; ++i) offer(A.sell_id[at + i * kWave], sellw[at + i * kWave]);
-        if (rows == kSellWidth && v < N && v >= ft0)
-          for (int e = A.rv_off[v]; e < A.rv_off[v + 1]; ++e)
-            if (A.rv_src[e] >= ft0 && A.rv_src[e] != v)
-              offer((unsigned)A.rv_src[e] | (unsigned)A.rv_eid[e] << 16, rw[e]);
       }
       const bool chosen = (bmC[min(sl, W - 1)] >> lane) & 1ull;
       if (v < N && v >= ft0) {
@@ -952,6 +952,33 @@ __global__ __launch_bounds__(BLOCK) void k_origin_lds(OriginArgs A, int load) {
       select(k, Ra);
       if (k + 2 < n) fetch(k + 2, Ra);
       if (k + 1 < n) select(k + 1, Rb);
+    }
+    // Nodes with more in-links than a slice has rows are looked at again, each
+    // by the whole wavefront (100 origins on a star of 10,000 links: 4.3 ms a
+    // loading, 6.1 with a lane reading them all in the loop above).
+    for (unsigned long long ks = __ballot(last - first >= kSellWidth * kWave); ks; ks &= ks - 1) {
+      const int sl = sl0 + (__ffsll((long long)ks) - 1) * kWaves, v = sl * kWave + lane;
+      const bool more = v < N && v >= ft0 && v != src && key[v] != kMax << 1 &&
+                        !((bmC[sl] >> lane) & 1ull) && A.rv_off[v + 1] - A.rv_off[v] > kSellWidth;
+      for (unsigned long long m = __ballot(more); m; m &= m - 1) {
+        const int l = __ffsll((long long)m) - 1, x = sl * kWave + l;
+        const unsigned long long dx = key[x];
+        unsigned long long du = dx, id = ~0ull;        // the lane's choice: label, then tail, then link
+        for (int e = A.rv_off[x] + lane; e < A.rv_off[x + 1]; e += kWave) {
+          const int u = A.rv_src[e];
+          const unsigned long long d = key[u], i = (unsigned long long)u << 32 | (unsigned)A.rv_eid[e];
+          if (u < ft0 || d >= dx || as_b(as_d(d >> 1) + rw[e]) != dx >> 1) continue;
+          if (d < du || (d == du && i < id)) { du = d; id = i; }
+        }
+        for (int o = kWave / 2; o > 0; o >>= 1) {
+          const unsigned long long d = __shfl_xor(du, o), i = __shfl_xor(id, o);
+          if (d < du || (d == du && i < id)) { du = d; id = i; }
+        }
+        if (lane == l && id != ~0ull) {
+          atomicAnd(&bmB[x >> 6], ~(1ull << (x & 63)));  // (the first rows may have had none)
+          choose(x, (unsigned)(id >> 32) | (unsigned)id << 16, dx);
+        }
+      }
     }
   }
   if (ft0 > 0) {
@@ -4030,7 +4057,7 @@ int build(tapgpu_ctx* c, const tapgpu_network* net, const tapgpu_demand* dem, in
       rows = std::max(rows, std::min(kSellWidth, n));
     }
     for (int i = 0; i < W; ++i) sell_ptr[i + 1] = sell_ptr[i] + sell_ptr[i + 1] * kWave;
-    c->sell_n = sell_ptr[W];
+    c->sell_n = std::max(sell_ptr[W], kWave);          // (a slice without rows reads the first one's)
     ALLOC(rec, (size_t)V * (N * kRecDoubles + c->sell_n));
     ALLOC(recpos, 2 * (size_t)E + W + 1 + c->sell_n);
     c->sellw = c->rec + (size_t)V * N * kRecDoubles;
